@@ -211,7 +211,7 @@ int validate_graph(Graph &g, bool check_symmetry, int64_t *bad_rows)
     const int32_t nv = g.st.nv;
     const int64_t nnz = g.st.nnz;
     hipStream_t s = g.stream;
-    TC_TRY(g.accum.ensure(16 * sizeof(unsigned long long)));
+    TC_TRY(g.accum.ensure(32 * sizeof(unsigned long long)));
     unsigned long long *res = g.accum.as<unsigned long long>();
     hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, s, res, 16);
     TC_HIP(hipGetLastError());
@@ -497,7 +497,7 @@ int graph_compare(Graph &a, Graph &b, int64_t *size_mismatch, int64_t *entry_mis
     }
     hipStream_t s = a.stream;
     TC_HIP(hipStreamSynchronize(b.stream));
-    TC_TRY(a.accum.ensure(16 * sizeof(unsigned long long)));
+    TC_TRY(a.accum.ensure(32 * sizeof(unsigned long long)));
     unsigned long long *res = a.accum.as<unsigned long long>();
     hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, s, res, 3);
     if (a.st.nv > 0)
@@ -527,7 +527,8 @@ void graph_destroy(Graph *g)
                       &g->coff, &g->crow, &g->work, &g->jobs, &g->tmp, &g->tmp2, &g->tmp3, &g->tmp4,
                       &g->accum, &g->bsrc, &g->bdst, &g->bflag, &g->bkeys, &g->bkeys2,
                       &g->bvals2, &g->boffb, &g->bdel, &g->flagpool, &g->vmark, &g->order,
-                      &g->rnk, &g->tasks, &g->pcnt, &g->hjobs, &g->outr};
+                      &g->rnk, &g->tasks, &g->pcnt, &g->hjobs, &g->outr, &g->dmat, &g->ditems,
+                      &g->dgraphs, &g->dgid};
     for (DevBuf *b : bufs) b->release();
     for (DevBuf &b : g->sb) b.release();
     for (DevBuf &b : g->ov) b.release();

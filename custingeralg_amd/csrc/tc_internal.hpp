@@ -151,6 +151,11 @@ struct Graph {
     // grow_add (the update allocator's policy); 0: the next power of two
     int32_t grow_mul_x16 = 0;
     int32_t grow_add = 0;
+    // bit-matrix counts (tc_dense.hip): matrix, items of long rows; batched
+    // graphs: their matrices' places, the graph of every vertex and the words
+    // of all matrices (0: some graph is too large)
+    DevBuf dmat, ditems, dgraphs, dgid;
+    int64_t dense_words = 0;
     DevBuf lbuf[5];  // delta: items, their prefix, per-edge counts, merge segments, their prefix
     bool degree_stale = false;
     // batched counting: graph boundaries and per-graph output (device)
@@ -212,6 +217,15 @@ int prepare_views(Graph &g, bool oriented, int32_t hub_degree = 0, int fallback 
 int build_direct_vinfo(Graph &g);
 // Validation of sortedness/range, self-loop count, optional symmetry check.
 int validate_graph(Graph &g, bool check_symmetry, int64_t *bad_rows);
+
+// Bit-matrix count of graphs of few vertices (tc_dense.hip): whether it takes
+// this count, its kernels on g.stream (acc: the 32
+// counters of the count, zeroed here; bad: bit 0 an entry without its reverse,
+// bit 1 an entry outside its graph), and the plan of a batched handle.
+bool dense_eligible(const Graph &g, const tc_schedule &sched);
+int dense_count(Graph &g, uint32_t *out, unsigned long long *acc, int32_t *bad, bool oriented,
+                bool skip_lower, hipEvent_t built);
+int dense_plan_batched(Graph &g);
 
 int static_count(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sched,
                  tc_stats *stats, bool skip_lower = false);

@@ -111,7 +111,7 @@ int lb_edge_prefix(Graph &g, const int32_t *verts, int64_t len, int64_t *pre)
 
 int lb_degree_bins(Graph &g, const int32_t *verts, int64_t len, int64_t counts[3])
 {
-    TC_TRY(g.accum.ensure(16 * sizeof(unsigned long long)));
+    TC_TRY(g.accum.ensure(32 * sizeof(unsigned long long)));
     unsigned long long *acc = g.accum.as<unsigned long long>();
     hipLaunchKernelGGL(k_zero_ull, dim3(1), dim3(64), 0, g.stream, acc, (int64_t)3);
     if (len > 0)
@@ -132,7 +132,8 @@ int batched_graph_create(int32_t G, const int64_t *voff, const int64_t *off, con
     TC_TRY(graph_borrow_csr(nv_total, nnz, off, adj, s, &g));
     g->batch_voff = voff;
     g->batch_ngraphs = G;
-    const int st = validate_graph(*g, true, nullptr);
+    int st = validate_graph(*g, true, nullptr);
+    if (st == TC_OK) st = dense_plan_batched(*g);
     if (st != TC_OK) {
         graph_destroy(g);
         return st;

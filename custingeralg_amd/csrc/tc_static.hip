@@ -3038,6 +3038,7 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     // tasks
     TC_TRY(g.accum.ensure(32 * sizeof(unsigned long long)));
     unsigned long long *acc = g.accum.as<unsigned long long>();
+    const bool dense = nnz > 0 && dense_eligible(g, sched);
     uint32_t *outp = out;
     if (!outp) {
         TC_TRY(g.tmp4.ensure((size_t)std::max<int32_t>(nv, 1) * sizeof(uint32_t)));
@@ -3045,10 +3046,12 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     }
 
     TC_HIP(rec(g.ev[0]));
-    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, s, acc, (int64_t)32);
-    hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(nv, 256, 65536)), dim3(256), 0, s, outp,
-                       (int64_t)nv, 0u);
-    TC_HIP(hipGetLastError());
+    if (!dense) {
+        hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, s, acc, (int64_t)32);
+        hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(nv, 256, 65536)), dim3(256), 0, s, outp,
+                           (int64_t)nv, 0u);
+        TC_HIP(hipGetLastError());
+    }
 
     if (nv == 0 || nnz == 0) {
         TC_HIP(hipEventRecord(g.ev[1], s));
@@ -3057,6 +3060,52 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
         st.method_used = method;
         if (stats) *stats = st;
         return TC_OK;
+    }
+
+    if (dense) {
+        // few vertices: bit rows (every tc_stats counter of tasks and jobs
+        // stays 0; ms_prepare is the matrix, ms_count the intersections)
+        int32_t *bad = reinterpret_cast<int32_t *>(acc + 27);
+        TC_TRY(dense_count(g, outp, acc, bad, oriented, skip_lower, g.capturing ? nullptr : g.ev[2]));
+        g.plan.method = method;
+        g.plan.bad = bad;
+        for (int64_t &j : g.plan.jt) j = 0;
+        if (g.capturing) return TC_OK;
+        TC_HIP(hipEventRecord(g.ev[7], s));
+        TC_HIP(hipMemcpyAsync(g.hcounts, acc, 28 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+        TC_HIP(hipStreamSynchronize(s));
+        const int32_t hbad = (int32_t)(uint32_t)g.hcounts[27];
+        if (oriented && (hbad & 1)) {  // rows declared symmetric that are not
+            g.symmetric = 0;
+            if (sched.method == TC_METHOD_ORIENTED) {
+                set_last_error(TC_ERR_INVALID, "oriented layout: the rows are not symmetric");
+                return TC_ERR_INVALID;
+            }
+            oriented = false;  // the bit rows count any rows
+            method = g.plan.method = TC_METHOD_DIRECT;
+        }
+        if (!(hbad & 2)) {
+            if (global) *global = g.hcounts[0];
+            if (stats) {
+                st.method_used = method;
+                fill_counters(st, g.hcounts, g.plan.jt, oriented);
+                float ms = 0;
+                (void)hipEventElapsedTime(&ms, g.ev[0], g.ev[7]);
+                st.ms_total = ms;
+                (void)hipEventElapsedTime(&ms, g.ev[0], g.ev[2]);
+                st.ms_prepare = ms;
+                (void)hipEventElapsedTime(&ms, g.ev[2], g.ev[7]);
+                st.ms_count = ms;
+                *stats = st;
+            }
+            return TC_OK;
+        }
+        // a batched entry outside its graph: the general kernels, from the start
+        g.dense_words = 0;
+        if (g.batch_per_graph)
+            hipLaunchKernelGGL(k_fill_u64, dim3(grid_for(g.batch_ngraphs, 256, 4096)), dim3(256), 0, s,
+                               g.batch_per_graph, (int64_t)g.batch_ngraphs);
+        return count_pass(g, out, global, sched, stats, skip_lower);
     }
 
     // compact offsets, chunk rows and the (degree-partitioned) vertex views;
