@@ -528,7 +528,7 @@ void graph_destroy(Graph *g)
                       &g->accum, &g->bsrc, &g->bdst, &g->bflag, &g->bkeys, &g->bkeys2,
                       &g->bvals2, &g->boffb, &g->bdel, &g->flagpool, &g->vmark, &g->order,
                       &g->rnk, &g->tasks, &g->pcnt, &g->hjobs, &g->outr, &g->dmat, &g->ditems,
-                      &g->dgraphs, &g->dgid};
+                      &g->dgraphs, &g->dgid, &g->cmat};
     for (DevBuf *b : bufs) b->release();
     for (DevBuf &b : g->sb) b.release();
     for (DevBuf &b : g->ov) b.release();

@@ -155,6 +155,10 @@ struct Graph {
     // graphs: their matrices' places, the graph of every vertex and the words
     // of all matrices (0: some graph is too large)
     DevBuf dmat, ditems, dgraphs, dgid;
+    // oriented count: the core's bit rows (tc_core.hip) and its size in the
+    // current layout (0: none)
+    DevBuf cmat;
+    int32_t core_k = 0;
     int64_t dense_words = 0;
     DevBuf lbuf[5];  // delta: items, their prefix, per-edge counts, merge segments, their prefix
     bool degree_stale = false;
@@ -211,8 +215,10 @@ struct Graph {
 // Builds coff, crow and vinfo (and padj for the oriented layout) for the store;
 // hub_degree > 0 overrides the degree from which owners build their task
 // lists from their own rows; fallback = 1 takes the paths used when the
-// default's staging does not fit (per-entry appends, mask by degree).
-int prepare_views(Graph &g, bool oriented, int32_t hub_degree = 0, int fallback = 0);
+// default's staging does not fit (per-entry appends, mask by degree).  core_k
+// > 0: the owners of the core_k highest ranks get no tasks (tc_core.hip counts
+// their triangles); g.core_k says whether the layout was built so.
+int prepare_views(Graph &g, bool oriented, int32_t hub_degree = 0, int fallback = 0, int32_t core_k = 0);
 // Fills vinfo with the store's rows as given (direct layout, dm=0).
 int build_direct_vinfo(Graph &g);
 // Validation of sortedness/range, self-loop count, optional symmetry check.
@@ -226,6 +232,12 @@ bool dense_eligible(const Graph &g, const tc_schedule &sched);
 int dense_count(Graph &g, uint32_t *out, unsigned long long *acc, int32_t *bad, bool oriented,
                 bool skip_lower, hipEvent_t built);
 int dense_plan_batched(Graph &g);
+
+// The core of the rank order on a bit matrix (tc_core.hip): how many ranks it
+// takes (0: none), and its share of an oriented count, added to g.outr and
+// acc[0]; *bad is set where the rows turn out not to be symmetric.
+int32_t core_size(const Graph &g, const tc_schedule &sched);
+int core_count(Graph &g, unsigned long long *acc, int32_t *bad);
 
 int static_count(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sched,
                  tc_stats *stats, bool skip_lower = false);

@@ -957,10 +957,11 @@ __global__ void k_orient_transpose_hubs(
 // ascend per graph only; the search then lands on some rank, and owners above
 // it take the row-built task lists, which are correct for any owner.)  One
 // thread.
-__global__ void k_hub_lo(const VInfo *__restrict__ vi, int32_t nv, int32_t min_deg,
+// fixed_lo >= 0 is that rank instead (the core's first).
+__global__ void k_hub_lo(const VInfo *__restrict__ vi, int32_t nv, int32_t min_deg, int32_t fixed_lo,
                          unsigned long long *__restrict__ sc)
 {
-    int32_t lo = 0, hi = nv;
+    int32_t lo = fixed_lo >= 0 ? fixed_lo : 0, hi = fixed_lo >= 0 ? fixed_lo : nv;
     while (lo < hi) {
         const int32_t mid = (lo + hi) >> 1;
         if (vi[mid].len < min_deg) lo = mid + 1; else hi = mid;
@@ -1443,6 +1444,7 @@ struct PlanParams {
     int32_t bin_max[2];  // |owner| <= bin_max[0] -> bin 0, <= bin_max[1] -> bin 1, else 2
     int32_t job_items;   // target estimated items per job (per wavefront)
     int32_t flush_items; // minimum items per owner slot in a job
+    int32_t owner_end;   // owners from here up get no jobs (the core's)
 };
 
 __device__ inline int32_t est_items(int32_t L, int32_t pl)
@@ -1465,10 +1467,11 @@ template <bool ORIENTED>
 __global__ void k_owner_work(const int64_t *__restrict__ coff, const int32_t *__restrict__ crow,
                              const VInfo *__restrict__ vi,
                              const int32_t *__restrict__ adj, const TaskRec *__restrict__ tasks,
-                             int32_t nv, int64_t nnz, PlanParams P,
+                             int32_t nv, PlanParams P,
                              unsigned long long *__restrict__ work,
                              unsigned long long *__restrict__ bstats)
 {
+    const int64_t nnz = coff[P.owner_end];  // (owners from owner_end up have no jobs)
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t nchunks = ceil_div(nnz, kWave);
     const int64_t wstride = (int64_t)gridDim.x * (blockDim.x / kWave);
@@ -1561,7 +1564,7 @@ __global__ void k_plan_jobs(const VInfo *__restrict__ vi, const unsigned long lo
         int32_t T = ORIENTED ? x.dm : x.len;
         int32_t nj[3] = {0, 0, 0};
         unsigned long long w = work[v];
-        if (L > 0 && T > 0 && w > 0 && (ORIENTED || x.len >= 2)) {
+        if (L > 0 && T > 0 && w > 0 && v < P.owner_end && (ORIENTED || x.len >= 2)) {
             int bin = owner_bin(L, P);
             int64_t tiles = ceil_div(L, P.lmax[bin]);
             int64_t per_tile = (int64_t)(w / (unsigned long long)tiles) + 1;
@@ -2684,7 +2687,7 @@ int build_direct_vinfo(Graph &g)
     return TC_OK;
 }
 
-int prepare_views(Graph &g, bool oriented, int32_t hub_degree, int fallback)
+int prepare_views(Graph &g, bool oriented, int32_t hub_degree, int fallback, int32_t core_k)
 {
     const int32_t nv = g.st.nv;
     const int64_t nnz = g.st.nnz;
@@ -2693,6 +2696,7 @@ int prepare_views(Graph &g, bool oriented, int32_t hub_degree, int fallback)
     const int wblocks = grid_for(nchunks, 4, 1 << 16);  // 4 waves of 256 threads
     const int vblocks = grid_for(nv, 256, 65536);
     g.oriented_views = false;
+    g.core_k = 0;
     if (!oriented) {
         // compact offsets of the store rows, chunk rows, views of the rows as stored
         TC_TRY(g.coff.ensure((size_t)(nv + 1) * sizeof(int64_t)));
@@ -2908,11 +2912,18 @@ int prepare_views(Graph &g, bool oriented, int32_t hub_degree, int fallback)
         if (!part)  // out of memory for the staging: free it again
             for (int q = 13; q < 18; ++q) g.ov[q].release();
     }
+    // the core's owners get no tasks (the split leaves out entries from rank
+    // sc[1] up, as with hubs).  A core pays where hubs gather the wedges: with
+    // it, R-MAT graphs of 20k to 1M vertices took 0.93 (ef 4, 20k) to 0.58
+    // (ef 32, 262k) of the time, uniform ones 1.02 to 1.10 times as long, their
+    // largest degree below five times the mean
+    if (part && (double)hmax * nv >= 16.0 * (double)nnz) g.core_k = core_k;
     // hubs: owners whose task lists are built from their rows (the appends
     // would serialise on their cursors; the partitioned transpose has no
     // per-owner atomics and needs no hubs unless the schedule asks)
     hipLaunchKernelGGL(k_hub_lo, dim3(1), dim3(1), 0, s, vi, nv,
-                       hub_degree > 0 ? hub_degree : part ? INT32_MAX : kHubDegree, sc);
+                       hub_degree > 0 ? hub_degree : part ? INT32_MAX : kHubDegree,
+                       g.core_k > 0 ? nv - g.core_k : -1, sc);
     TC_HIP(hipGetLastError());
     if (part) {
         int64_t *fpos = g.ov[13].as<int64_t>();
@@ -2939,7 +2950,8 @@ int prepare_views(Graph &g, bool oriented, int32_t hub_degree, int fallback)
                            own2, bad);
         hipLaunchKernelGGL(k_tp_local, dim3((unsigned)std::min<int64_t>(fmax, 1 << 16)),
                            dim3(kTpThreads), 0, s, toff, fb, ctl, tasks, own2, bad);
-        hipLaunchKernelGGL(k_orient_transpose_hubs, dim3(cus * 16), dim3(256), 0, s, pcoff, toff,
+        if (g.core_k == 0)
+            hipLaunchKernelGGL(k_orient_transpose_hubs, dim3(cus * 16), dim3(256), 0, s, pcoff, toff,
                            order, rnk, ocoff, g.st.boff.as<int64_t>(), g.st.pool.as<int32_t>(), mask,
                            cscan, padj, nv, sc, g.tasks.as<TaskRec>(), bad);
         hipLaunchKernelGGL(k_tp_check, dim3(grid_for(fmax, 256, 4096)), dim3(256), 0, s, toff, fb, ctl,
@@ -3111,7 +3123,7 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     // compact offsets, chunk rows and the (degree-partitioned) vertex views;
     // rows declared symmetric that turn out not to be go the direct way
     if (oriented) {
-        const int pv = prepare_views(g, true, sched.hub_degree, sched.build);
+        const int pv = prepare_views(g, true, sched.hub_degree, sched.build, core_size(g, sched));
         if (pv == TC_ERR_INVALID && sched.method == TC_METHOD_AUTO && !g.symmetric) {
             oriented = false;
             method = TC_METHOD_DIRECT;
@@ -3145,15 +3157,16 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     P.bin_max[1] = std::min(std::max(sched.mid_max, P.bin_max[0]), kL1);
     P.job_items = std::max(sched.job_items, 256);
     P.flush_items = sched.flush_items > 0 ? sched.flush_items : 1024;
+    P.owner_end = nv - (oriented ? g.core_k : 0);
     TC_TRY(g.work.ensure((size_t)nv * sizeof(unsigned long long)));
     unsigned long long *work = g.work.as<unsigned long long>();
     hipLaunchKernelGGL(k_fill_u64, dim3(grid_for(nv, 256, 65536)), dim3(256), 0, s, work, (int64_t)nv);
     if (oriented)
         hipLaunchKernelGGL(k_owner_work<true>, dim3(wblocks), dim3(256), 0, s, coff, crow, vi, adj,
-                           tasks, nv, nent, P, work, stats ? acc + 4 : nullptr);
+                           tasks, nv, P, work, stats ? acc + 4 : nullptr);
     else
         hipLaunchKernelGGL(k_owner_work<false>, dim3(wblocks), dim3(256), 0, s, coff, crow, vi, adj,
-                           nullptr, nv, nent, P, work, stats ? acc + 4 : nullptr);
+                           nullptr, nv, P, work, stats ? acc + 4 : nullptr);
     TC_HIP(hipGetLastError());
     TC_TRY(g.tmp3.ensure((size_t)3 * nv * sizeof(int32_t) + (size_t)3 * (nv + 1) * sizeof(int64_t) + 16));
     int32_t *njobs = g.tmp3.as<int32_t>();
@@ -3245,6 +3258,7 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
         TC_TRY(launch_bin(b, oriented, jl[b], jt[b], A, s, g.capturing ? nullptr : &g.ev[8]));
     }
     TC_HIP(rec(g.ev[6]));  // end of the bin kernels
+    if (oriented && g.core_k > 0) TC_TRY(core_count(g, acc, reinterpret_cast<int32_t *>(acc + 27)));
     if (oriented && nplus > 0) {
         hipLaunchKernelGGL(k_plus_row_sum, dim3(grid_for(ceil_div(nplus, kWave), 4, 1 << 16)),
                            dim3(256), 0, s, g.ov[6].as<int64_t>(), g.ov[10].as<int32_t>(),
@@ -3261,8 +3275,16 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     TC_HIP(hipEventRecord(g.ev[7], s));
     TC_HIP(hipEventSynchronize(g.ev[7]));
 
-    unsigned long long hacc[26];
+    unsigned long long hacc[28];
     TC_HIP(hipMemcpy(hacc, acc, sizeof(hacc), hipMemcpyDeviceToHost));
+    if (oriented && g.core_k > 0 && hacc[27]) {  // rows declared symmetric that are not
+        g.symmetric = 0;
+        if (sched.method == TC_METHOD_ORIENTED) {
+            set_last_error(TC_ERR_INVALID, "oriented layout: the rows are not symmetric");
+            return TC_ERR_INVALID;
+        }
+        return count_pass(g, out, global, sched, stats, skip_lower);  // the direct way
+    }
     if (global) *global = hacc[0];
     if (stats) {
         fill_counters(st, hacc, jt, oriented);
@@ -3321,12 +3343,12 @@ int count_replay(Graph &g, uint64_t *global, tc_stats *stats)
     TC_HIP(hipGraphLaunch(g.cexec, s));
     TC_HIP(hipEventRecord(g.ev[7], s));
     TC_HIP(hipEventSynchronize(g.ev[7]));
-    unsigned long long hacc[26];
+    unsigned long long hacc[28];
     int32_t bad = 0;
     TC_HIP(hipMemcpy(hacc, g.accum.p, sizeof(hacc), hipMemcpyDeviceToHost));
     if (g.plan.method == TC_METHOD_ORIENTED && g.plan.bad)
         TC_HIP(hipMemcpy(&bad, g.plan.bad, sizeof(bad), hipMemcpyDeviceToHost));
-    if (bad) {  // cannot happen for an unchanged store that counted before
+    if (bad || (g.plan.method == TC_METHOD_ORIENTED && hacc[27])) {  // cannot happen for an unchanged store that counted before
         g.symmetric = 0;
         g.touch();
         set_last_error(TC_ERR_INVALID, "oriented layout: the rows are not symmetric");

@@ -1,0 +1,87 @@
+"""The oriented count's core (the highest ranks on a bit matrix) against the
+oracle: sizes at its smallest graph, core rows of every length around the
+group and wave limits, and rows declared symmetric that are not."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import custingeralg_amd as T
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _planted(n, hubs, seed, dense=0.05):
+    """hubs vertices of a random graph among themselves, every other vertex
+    joined to 0, 1, 2, ... 40 of them in turn, and a sparse background."""
+    rng = np.random.default_rng(seed)
+    ids = rng.permutation(n).astype(np.int32)
+    m = int(dense * hubs * hubs / 2)
+    hu, hv = rng.integers(0, hubs, m), rng.integers(0, hubs, m)
+    k = np.arange(n - hubs) % 41
+    lu = np.repeat(np.arange(hubs, n), k)
+    lv = (rng.pareto(0.6, len(lu)) * hubs / 40).astype(np.int64) % hubs
+    bu, bv = rng.integers(0, n, n), rng.integers(0, n, n)
+    u, v = np.concatenate([hu, lu, bu]), np.concatenate([hv, lv, bv])
+    return O.canon_csr(n, ids[u], ids[v])
+
+
+def _check(off, adj, **kw):
+    ref = O.custinger_count(off, adj)
+    g = T.cuStinger(off, adj)
+    for method in (T.METHOD_AUTO, T.METHOD_ORIENTED):
+        pv, glob, st = T.static_count(g, T.default_schedule(method=method, **kw))
+        assert st["method_used"] == T.METHOD_ORIENTED
+        assert np.array_equal(pv, ref)
+        assert glob == int(ref.astype(np.uint64).sum())
+    g.close()
+
+
+@pytest.mark.parametrize("n", [16385, 16999, 40003])
+@pytest.mark.parametrize("hubs", [300, 5000])
+def test_planted(n, hubs):
+    _check(*_planted(n, hubs, n))
+
+
+@pytest.mark.parametrize("scale,ef", [(15, 3), (17, 24)])
+def test_rmat(scale, ef):
+    _check(*O.rmat_graph(scale, ef, 11))
+    _check(*O.rmat_graph(scale, ef, 12), policy=T.POLICY_LEARNED)
+
+
+def test_recorded_counts():
+    off, adj = _planted(20000, 600, 5)
+    ref = O.custinger_count(off, adj)
+    g = T.cuStinger(off, adj)
+    out = T.DeviceArray(g.nv, np.uint32)
+    sched = T.default_schedule(capture=1)
+    for k in range(4):
+        _, glob, st = T.static_count(g, sched, out=out)
+        assert np.array_equal(out.to_host(), ref) and glob == int(ref.astype(np.uint64).sum())
+        assert st["graph_replay"] == (k > 0)
+    out.free()
+    g.close()
+
+
+def test_declared_symmetric_with_balanced_faults():
+    """One entry into a core vertex moved to another core vertex: every total
+    still fits, the per-vertex counts of entries do not."""
+    off, adj = _planted(20000, 600, 7)
+    deg = np.diff(off)
+    h1, h2 = (int(x) for x in np.argsort(deg)[-2:])
+    for a in range(len(deg)):  # a leaf that points to h1 and not to h2
+        row = adj[off[a]:off[a + 1]]
+        if 2 < len(row) < 40 and h1 in row and h2 not in row:
+            break
+    new = np.sort(np.where(row == h1, h2, row))
+    adj2 = adj.copy()
+    adj2[off[a]:off[a + 1]] = new
+    ref = O.custinger_count(off, adj2)
+    g = T.cuStinger(off, adj2, assume_symmetric=True)
+    with pytest.raises(T.TCError):
+        T.static_count(g, T.default_schedule(method=T.METHOD_ORIENTED))
+    pv, glob, st = T.static_count(g)
+    g.close()
+    assert st["method_used"] == T.METHOD_DIRECT
+    assert np.array_equal(pv, ref) and glob == int(ref.astype(np.uint64).sum())
