@@ -52,7 +52,7 @@ struct DenseArgs {
     unsigned long long *nitems;  // [kParts], kCtrStride apart, zero on entry
     int2 *items;                 // [kParts][icap] (row, first entry)
     int64_t icap;
-    int32_t *bad;                  // bit 0: an entry has no reverse, bit 1: one leaves its graph
+    int32_t *bad;                // set where an entry has no reverse
     int32_t skip_lower;
     int32_t check_sym;
 };
@@ -73,11 +73,6 @@ __device__ inline void wave_lds_sync()
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-__device__ inline bool in_graph(const DenseGraph &D, int32_t v)
-{
-    return D.n > 0 && (uint32_t)(v - D.v0) < (uint32_t)D.n;
 }
 
 // The rows of a wave: round-robin over a single graph (a hub's neighbours in id
@@ -118,28 +113,18 @@ __global__ __launch_bounds__(kRowWaves * kWave) void k_dense_rows(DenseArgs A)
     for (int64_t r = W.r; r < W.end; r += W.step) {
         const int32_t v = (int32_t)r;
         const DenseGraph D = graph_of_row(A, v);
-        if (!in_graph(D, v)) {  // boundaries that leave vertices out
-            if (lane == 0) atomicOr(A.bad, 2);
-            continue;
-        }
         const int32_t words = D.nch * kChunkWords, d = A.len[v];
         const int32_t *row = A.pool + A.boff[v];
         for (int i = lane; i < words; i += kWave) bits[i] = 0u;
         wave_lds_sync();
-        bool out_of = false;
         for (int32_t k0 = lane; k0 < d; k0 += 4 * kWave) {
             int32_t c[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) c[q] = row[min(k0 + q * kWave, d - 1)] - D.v0;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {  // (a repeat of the last entry sets its bit again)
-                if ((uint32_t)c[q] < (uint32_t)D.n)
-                    atomicOr(&bits[c[q] >> 5], 1u << (c[q] & 31));
-                else
-                    out_of = true;
-            }
+            for (int q = 0; q < 4; ++q)  // (a repeat of the last entry sets its bit again)
+                atomicOr(&bits[c[q] >> 5], 1u << (c[q] & 31));
         }
-        if (out_of) atomicOr(A.bad, 2);
         if (d > A.long_len) {
             unsigned long long base = 0;
             if (lane == 0) {
@@ -198,7 +183,7 @@ __device__ inline uint32_t dense_row(const DenseArgs &A, const DenseGraph &D, in
             }
 #pragma unroll
             for (int q = 0; q < U; ++q) {
-                in[q] = eb + q * 8 < e1 && u[q] != lv && u[q] < (uint32_t)D.n;
+                in[q] = eb + q * 8 < e1 && u[q] != lv;
                 u[q] = in[q] ? u[q] : lv;
 #pragma unroll
                 for (int c = 0; c < CH; ++c)
@@ -279,7 +264,6 @@ __global__ __launch_bounds__(256, 8) void k_dense_count(DenseArgs A)
         const int32_t v = (int32_t)r, d = A.len[v];
         if (d > A.long_len) continue;
         const DenseGraph D = graph_of_row(A, v);
-        if (!in_graph(D, v)) continue;
         const uint32_t h = (d >= 2 || A.check_sym) ? dense_part(A, D, v, 0, d, miss) : 0u;
         if (lane == 0) {
             // (a row of one entry counts nothing: the reference skips it)
@@ -375,13 +359,12 @@ int dense_plan_batched(Graph &g)
     unsigned long long h[2];
     TC_HIP(hipMemcpyAsync(h, res, sizeof(h), hipMemcpyDeviceToHost, s));
     TC_HIP(hipStreamSynchronize(s));
-    if (h[0] > (unsigned long long)kDenseMax || h[1] * 4 > (unsigned long long)kDenseBytes)
-        return TC_OK;
     TC_TRY(g.dgid.ensure((size_t)g.st.nv * sizeof(int32_t)));
     hipLaunchKernelGGL(k_dense_gid, dim3(grid_for(g.st.nv, 256, 4096)), dim3(256), 0, s, graphs, G,
                        g.st.nv, g.dgid.as<int32_t>());
     TC_HIP(hipGetLastError());
-    g.dense_words = (int64_t)h[1];
+    if (h[0] <= (unsigned long long)kDenseMax && h[1] * 4 <= (unsigned long long)kDenseBytes)
+        g.dense_words = (int64_t)h[1];
     return TC_OK;
 }
 

@@ -123,16 +123,17 @@ __device__ inline int32_t row_search_g(const int64_t *__restrict__ coff, int64_t
 }
 
 // Validation over compact entries: [0] unsorted/dup, [1] out of range,
-// [2] self loops, [3] missing reverse entries, [4] max degree.
+// [2] self loops, [3] missing reverse entries, [4] max degree, [5] entries
+// that leave their graph (gid: the graph of every vertex, or null).
 __global__ void k_validate(const int64_t *__restrict__ coff, const int64_t *__restrict__ boff,
                            const int32_t *__restrict__ len, const int32_t *__restrict__ pool,
-                           int32_t nv, int64_t nnz, int check_sym,
+                           int32_t nv, int64_t nnz, int check_sym, const int32_t *__restrict__ gid,
                            unsigned long long *__restrict__ res)
 {
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t nchunks = ceil_div(nnz, kWave);
     const int64_t wstride = (int64_t)gridDim.x * (blockDim.x / kWave);
-    unsigned long long bad = 0, oor = 0, loops = 0, miss = 0;
+    unsigned long long bad = 0, oor = 0, loops = 0, miss = 0, cross = 0;
     for (int64_t c = (int64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave; c < nchunks;
          c += wstride) {
         int64_t e = c * kWave + lane;
@@ -153,6 +154,7 @@ __global__ void k_validate(const int64_t *__restrict__ coff, const int64_t *__re
         }
         if (k > 0 && pool[addr - 1] >= b) ++bad;
         if (b == a) ++loops;
+        if (gid && gid[a] != gid[b]) ++cross;
         if (check_sym) {
             const int32_t *lst = pool + boff[b];
             int32_t lo = 0, hi = len[b];
@@ -168,12 +170,14 @@ __global__ void k_validate(const int64_t *__restrict__ coff, const int64_t *__re
         oor += __shfl_xor(oor, d);
         loops += __shfl_xor(loops, d);
         miss += __shfl_xor(miss, d);
+        cross += __shfl_xor(cross, d);
     }
     if (lane == 0) {
         if (bad) atomicAdd(&res[0], bad);
         if (oor) atomicAdd(&res[1], oor);
         if (loops) atomicAdd(&res[2], loops);
         if (miss) atomicAdd(&res[3], miss);
+        if (cross) atomicAdd(&res[5], cross);
     }
 }
 
@@ -223,7 +227,8 @@ int validate_graph(Graph &g, bool check_symmetry, int64_t *bad_rows)
             int64_t nchunks = ceil_div(nnz, kWave);
             hipLaunchKernelGGL(k_validate, dim3(grid_for(nchunks, 4, 1 << 16)), dim3(256), 0, s, coff,
                                g.st.boff.as<int64_t>(), g.st.len.as<int32_t>(),
-                               g.st.pool.as<int32_t>(), nv, nnz, check_symmetry ? 1 : 0, res);
+                               g.st.pool.as<int32_t>(), nv, nnz, check_symmetry ? 1 : 0,
+                               g.batch_voff ? g.dgid.as<int32_t>() : nullptr, res);
             TC_HIP(hipGetLastError());
         }
         hipLaunchKernelGGL(k_max_len, dim3(grid_for(nv, 256, 4096)), dim3(256), 0, s,
@@ -245,6 +250,11 @@ int validate_graph(Graph &g, bool check_symmetry, int64_t *bad_rows)
     g.self_loops = (int64_t)h[2];
     if (check_symmetry) g.symmetric = h[3] == 0 ? 1 : 0;
     g.max_degree = (int32_t)h[4];
+    // bit matrices hold a graph's own columns only
+    if (h[5]) {
+        g.dense_words = 0;
+        g.core_total = 0;
+    }
     return TC_OK;
 }
 
@@ -528,7 +538,7 @@ void graph_destroy(Graph *g)
                       &g->accum, &g->bsrc, &g->bdst, &g->bflag, &g->bkeys, &g->bkeys2,
                       &g->bvals2, &g->boffb, &g->bdel, &g->flagpool, &g->vmark, &g->order,
                       &g->rnk, &g->tasks, &g->pcnt, &g->hjobs, &g->outr, &g->dmat, &g->ditems,
-                      &g->dgraphs, &g->dgid, &g->cmat};
+                      &g->dgraphs, &g->dgid, &g->cmat, &g->cgraphs, &g->cblocks};
     for (DevBuf *b : bufs) b->release();
     for (DevBuf &b : g->sb) b.release();
     for (DevBuf &b : g->ov) b.release();

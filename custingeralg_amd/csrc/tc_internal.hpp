@@ -159,6 +159,10 @@ struct Graph {
     // current layout (0: none)
     DevBuf cmat;
     int32_t core_k = 0;
+    // batched graphs: their cores, the blocks that count them, and the totals
+    // (core_total 0: none)
+    DevBuf cgraphs, cblocks;
+    int32_t core_total = 0, core_blocks = 0;
     int64_t dense_words = 0;
     DevBuf lbuf[5];  // delta: items, their prefix, per-edge counts, merge segments, their prefix
     bool degree_stale = false;
@@ -226,8 +230,8 @@ int validate_graph(Graph &g, bool check_symmetry, int64_t *bad_rows);
 
 // Bit-matrix count of graphs of few vertices (tc_dense.hip): whether it takes
 // this count, its kernels on g.stream (acc: the 32
-// counters of the count, zeroed here; bad: bit 0 an entry without its reverse,
-// bit 1 an entry outside its graph), and the plan of a batched handle.
+// counters of the count, zeroed here; bad: set by an entry without its
+// reverse), and the plan of a batched handle.
 bool dense_eligible(const Graph &g, const tc_schedule &sched);
 int dense_count(Graph &g, uint32_t *out, unsigned long long *acc, int32_t *bad, bool oriented,
                 bool skip_lower, hipEvent_t built);
@@ -236,8 +240,13 @@ int dense_plan_batched(Graph &g);
 // The core of the rank order on a bit matrix (tc_core.hip): how many ranks it
 // takes (0: none), and its share of an oriented count, added to g.outr and
 // acc[0]; *bad is set where the rows turn out not to be symmetric.
+// gid: the graph of every rank (batched).  core_plan_batched lays out the
+// cores of a batched handle, core_order_batched moves them behind the other
+// ranks (vgid: the graph of every vertex).
 int32_t core_size(const Graph &g, const tc_schedule &sched);
-int core_count(Graph &g, unsigned long long *acc, int32_t *bad);
+int core_count(Graph &g, unsigned long long *acc, int32_t *bad, const int32_t *gid);
+int core_plan_batched(Graph &g);
+int core_order_batched(Graph &g, const int32_t *order, const int32_t *vgid, int32_t *order2, int32_t *rnk);
 
 int static_count(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sched,
                  tc_stats *stats, bool skip_lower = false);

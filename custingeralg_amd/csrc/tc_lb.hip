@@ -132,8 +132,10 @@ int batched_graph_create(int32_t G, const int64_t *voff, const int64_t *off, con
     TC_TRY(graph_borrow_csr(nv_total, nnz, off, adj, s, &g));
     g->batch_voff = voff;
     g->batch_ngraphs = G;
-    int st = validate_graph(*g, true, nullptr);
-    if (st == TC_OK) st = dense_plan_batched(*g);
+    int st = dense_plan_batched(*g);
+    if (st == TC_OK) st = core_plan_batched(*g);
+    if (st == TC_OK && !g->core_total) g->dense_words = 0;  // (odd boundaries)
+    if (st == TC_OK) st = validate_graph(*g, true, nullptr);
     if (st != TC_OK) {
         graph_destroy(g);
         return st;

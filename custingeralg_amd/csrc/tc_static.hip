@@ -2746,7 +2746,19 @@ int prepare_views(Graph &g, bool oriented, int32_t hub_degree, int fallback, int
         kbits += ceil_log2_i((int64_t)g.batch_ngraphs);
     }
     TC_TRY(radix_sort_u64(keys, order, nv, kbits, g.ov[4], g.ov[5], g.tmp, s));
-    hipLaunchKernelGGL(k_rank_inverse, dim3(vblocks), dim3(256), 0, s, order, nv, rnk);
+    // A core pays where hubs gather the wedges: with it, R-MAT graphs of 20k to
+    // 1M vertices took 0.93 (ef 4, 20k) to 0.58 (ef 32, 262k) of the time,
+    // uniform ones 1.02 to 1.10 times as long, their largest degree below five
+    // times the mean
+    if ((double)hmax * nv < 16.0 * (double)nnz) core_k = 0;
+    if (core_k > 0 && g.batch_voff) {
+        TC_TRY(g.ov[5].ensure((size_t)nv * sizeof(int32_t)));
+        TC_TRY(core_order_batched(g, order, g.dgid.as<int32_t>(), g.ov[5].as<int32_t>(), rnk));
+        std::swap(g.order, g.ov[5]);
+        order = g.order.as<int32_t>();
+    } else {
+        hipLaunchKernelGGL(k_rank_inverse, dim3(vblocks), dim3(256), 0, s, order, nv, rnk);
+    }
     TC_HIP(hipGetLastError());
 
 
@@ -2913,11 +2925,8 @@ int prepare_views(Graph &g, bool oriented, int32_t hub_degree, int fallback, int
             for (int q = 13; q < 18; ++q) g.ov[q].release();
     }
     // the core's owners get no tasks (the split leaves out entries from rank
-    // sc[1] up, as with hubs).  A core pays where hubs gather the wedges: with
-    // it, R-MAT graphs of 20k to 1M vertices took 0.93 (ef 4, 20k) to 0.58
-    // (ef 32, 262k) of the time, uniform ones 1.02 to 1.10 times as long, their
-    // largest degree below five times the mean
-    if (part && (double)hmax * nv >= 16.0 * (double)nnz) g.core_k = core_k;
+    // sc[1] up, as with hubs)
+    if (part) g.core_k = core_k;
     // hubs: owners whose task lists are built from their rows (the appends
     // would serialise on their cursors; the partitioned transpose has no
     // per-owner atomics and needs no hubs unless the schedule asks)
@@ -3087,7 +3096,7 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
         TC_HIP(hipMemcpyAsync(g.hcounts, acc, 28 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
         TC_HIP(hipStreamSynchronize(s));
         const int32_t hbad = (int32_t)(uint32_t)g.hcounts[27];
-        if (oriented && (hbad & 1)) {  // rows declared symmetric that are not
+        if (oriented && hbad) {  // rows declared symmetric that are not
             g.symmetric = 0;
             if (sched.method == TC_METHOD_ORIENTED) {
                 set_last_error(TC_ERR_INVALID, "oriented layout: the rows are not symmetric");
@@ -3096,28 +3105,20 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
             oriented = false;  // the bit rows count any rows
             method = g.plan.method = TC_METHOD_DIRECT;
         }
-        if (!(hbad & 2)) {
-            if (global) *global = g.hcounts[0];
-            if (stats) {
-                st.method_used = method;
-                fill_counters(st, g.hcounts, g.plan.jt, oriented);
-                float ms = 0;
-                (void)hipEventElapsedTime(&ms, g.ev[0], g.ev[7]);
-                st.ms_total = ms;
-                (void)hipEventElapsedTime(&ms, g.ev[0], g.ev[2]);
-                st.ms_prepare = ms;
-                (void)hipEventElapsedTime(&ms, g.ev[2], g.ev[7]);
-                st.ms_count = ms;
-                *stats = st;
-            }
-            return TC_OK;
+        if (global) *global = g.hcounts[0];
+        if (stats) {
+            st.method_used = method;
+            fill_counters(st, g.hcounts, g.plan.jt, oriented);
+            float ms = 0;
+            (void)hipEventElapsedTime(&ms, g.ev[0], g.ev[7]);
+            st.ms_total = ms;
+            (void)hipEventElapsedTime(&ms, g.ev[0], g.ev[2]);
+            st.ms_prepare = ms;
+            (void)hipEventElapsedTime(&ms, g.ev[2], g.ev[7]);
+            st.ms_count = ms;
+            *stats = st;
         }
-        // a batched entry outside its graph: the general kernels, from the start
-        g.dense_words = 0;
-        if (g.batch_per_graph)
-            hipLaunchKernelGGL(k_fill_u64, dim3(grid_for(g.batch_ngraphs, 256, 4096)), dim3(256), 0, s,
-                               g.batch_per_graph, (int64_t)g.batch_ngraphs);
-        return count_pass(g, out, global, sched, stats, skip_lower);
+        return TC_OK;
     }
 
     // compact offsets, chunk rows and the (degree-partitioned) vertex views;
@@ -3221,7 +3222,7 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     A.skip_lower = skip_lower ? 1 : 0;
     A.per_graph = g.batch_per_graph;
     A.gid = nullptr;
-    if (g.batch_per_graph) {
+    if (g.batch_per_graph || (g.batch_voff && oriented && g.core_k > 0)) {
         // graph of every owner, found once here instead of once per job
         TC_TRY(g.ov[11].ensure((size_t)std::max(nv, 1) * sizeof(int32_t)));
         hipLaunchKernelGGL(k_graph_of, dim3(grid_for(nv, 256, 65536)), dim3(256), 0, s, g.batch_voff,
@@ -3258,7 +3259,7 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
         TC_TRY(launch_bin(b, oriented, jl[b], jt[b], A, s, g.capturing ? nullptr : &g.ev[8]));
     }
     TC_HIP(rec(g.ev[6]));  // end of the bin kernels
-    if (oriented && g.core_k > 0) TC_TRY(core_count(g, acc, reinterpret_cast<int32_t *>(acc + 27)));
+    if (oriented && g.core_k > 0) TC_TRY(core_count(g, acc, reinterpret_cast<int32_t *>(acc + 27), A.gid));
     if (oriented && nplus > 0) {
         hipLaunchKernelGGL(k_plus_row_sum, dim3(grid_for(ceil_div(nplus, kWave), 4, 1 << 16)),
                            dim3(256), 0, s, g.ov[6].as<int64_t>(), g.ov[10].as<int32_t>(),

@@ -85,3 +85,30 @@ def test_declared_symmetric_with_balanced_faults():
     g.close()
     assert st["method_used"] == T.METHOD_DIRECT
     assert np.array_equal(pv, ref) and glob == int(ref.astype(np.uint64).sum())
+
+
+@pytest.mark.parametrize("sizes", [[20000, 1, 3, 5000], [4096, 17000, 2, 4097, 2048, 2049] * 3])
+def test_batched_cores(sizes):
+    """Graphs with their cores behind all other ranks, some all core."""
+    voff = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int64)
+    us, vs = [], []
+    for i, n in enumerate(sizes):
+        if n < 16:
+            continue
+        off, adj = _planted(n, n // 8, i, 0.1)
+        us.append(np.repeat(np.arange(n), np.diff(off)) + voff[i])
+        vs.append(adj + voff[i])
+    nv = int(voff[-1])
+    off, adj = O.canon_csr(nv, np.concatenate(us).astype(np.int32),
+                           np.concatenate(vs).astype(np.int32))
+    ref = O.custinger_count(off, adj)
+    want = np.add.reduceat(ref.astype(np.uint64), voff[:-1])
+    dv, do, da = (T.DeviceArray.from_host(x) for x in (voff, off, adj))
+    bg = T.BatchedGraph(dv, do, da)
+    pg, pv = T.DeviceArray(len(sizes), np.uint64), T.DeviceArray(nv, np.uint32)
+    for sched in (None, T.default_schedule(policy=T.POLICY_HASH), T.default_schedule(capture=1),
+                  T.default_schedule(capture=1), T.default_schedule(capture=1)):
+        bg.count(pg, pv, sched)
+        assert np.array_equal(pv.to_host(), ref)
+        assert np.array_equal(pg.to_host(), want)
+    bg.close()
