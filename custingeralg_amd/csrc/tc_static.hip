@@ -1436,6 +1436,100 @@ __global__ void k_direct_vinfo(const int64_t *__restrict__ boff, const int32_t *
     }
 }
 
+// ------------------------------------------- direct counts by the larger row --
+//
+// |N(v) cap N(u)| of an entry (v, u) costs the list that is streamed: the
+// owner of the pair's job is the endpoint with the longer row, whose list sits
+// in LDS, and the shorter one is streamed (645M instead of 2.9G entries on a
+// directed R-MAT graph of 2^18 vertices, ef 16).  An owner's tasks are the
+// entries of its own row that point to shorter rows and the entries of shorter
+// rows that point to it; the hits of a task go to the entry's source.
+
+struct DirectEntry {
+    int32_t owner, list, src;
+    bool ok;
+};
+
+// Counter of owner x among 2^b > x counters: neighbouring ids (R-MAT's hubs are
+// ids with few set bits) get different cache lines, whose atomics would queue
+// (one pass over 4M entries 443 -> 177 us).
+__device__ inline uint32_t direct_slot(int32_t x, uint32_t mask) { return ((uint32_t)x * 0x9E3779B1u) & mask; }
+
+// Entry e = 64c + lane of the compact rows: reference filters (cct.cu:247-249),
+// and which endpoint's job it is.
+__device__ inline DirectEntry direct_entry(const int64_t *__restrict__ coff, const int64_t *__restrict__ boff,
+                                           const int32_t *__restrict__ len, const int32_t *__restrict__ pool,
+                                           int32_t v, int64_t e, int64_t nnz, int skip_lower)
+{
+    DirectEntry d = {v, v, v, false};
+    if (e < nnz) {
+        const int32_t u = pool[boff[v] + (e - coff[v])];
+        const int32_t lv = len[v], lu = len[u];
+        d.ok = u != v && lv >= 2 && lu >= 2 && (!skip_lower || u > v);
+        d.owner = lu <= lv ? v : u;
+        d.list = lu <= lv ? u : v;
+    }
+    return d;
+}
+
+// WRITE = false: cnt[x] = tasks of owner x (zero on entry).  WRITE = true: the
+// tasks themselves, cnt being the cursors (zero on entry).  A row's own tasks
+// in a chunk take one atomic; the others one each.
+template <bool WRITE>
+__global__ void k_direct_tasks(const int64_t *__restrict__ coff, const int32_t *__restrict__ crow,
+                               const int64_t *__restrict__ boff, const int32_t *__restrict__ len,
+                               const int32_t *__restrict__ pool, int32_t nv, int64_t nnz, int skip_lower,
+                               int32_t *__restrict__ cnt, uint32_t mask, const int64_t *__restrict__ toff,
+                               TaskRec *__restrict__ tasks, int32_t *__restrict__ cred)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    const int64_t nchunks = ceil_div(nnz, kWave);
+    const int64_t wstride = (int64_t)gridDim.x * (blockDim.x / kWave);
+    const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
+    for (int64_t c = (int64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave; c < nchunks;
+         c += wstride) {
+        const int32_t v = wave_row_of(coff, crow, nv, c, nnz);
+        const DirectEntry d = direct_entry(coff, boff, len, pool, v, c * kWave + lane, nnz, skip_lower);
+        const bool own = d.ok && d.owner == v, other = d.ok && d.owner != v;
+        // the lanes of this lane's row (rows are runs of lanes)
+        const int32_t before = __shfl_up(v, 1, kWave);
+        const uint64_t starts = __ballot(lane == 0 || before != v);
+        const int s0 = 63 - __clzll((long long)(starts & (lt | (1ull << lane))));
+        const uint64_t after = starts & ~(lt | (1ull << lane));
+        const int s1 = after ? __ffsll((unsigned long long)after) - 1 : kWave;
+        const uint64_t seg = (s1 == kWave ? ~0ull : (1ull << s1) - 1) & ~((1ull << s0) - 1);
+        const uint64_t mine = __ballot(own) & seg;
+        int32_t slot = 0;
+        if (lane == s0 && mine) slot = atomicAdd(&cnt[direct_slot(v, mask)], __popcll(mine));
+        slot = __shfl(slot, s0, kWave) + __popcll(mine & lt);
+        if (other) slot = atomicAdd(&cnt[direct_slot(d.owner, mask)], 1);
+        if (WRITE && d.ok) {
+            const int64_t p = toff[d.owner] + slot;
+            tasks[p] = TaskRec::make(boff[d.list], len[d.list]);
+            cred[p] = v;
+        }
+    }
+}
+
+// Views for the planner and the count kernels (dm tasks, a row of len - dm),
+// and the counts in order for their scan.
+__global__ void k_direct_task_vinfo(const int64_t *__restrict__ boff, const int32_t *__restrict__ len,
+                                    int32_t *__restrict__ cnt, uint32_t mask, int32_t nv, VInfo *__restrict__ vi,
+                                    int32_t *__restrict__ tcnt)
+{
+    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nv;
+         v += (int64_t)gridDim.x * blockDim.x) {
+        VInfo x;
+        x.rb = boff[v];
+        const uint32_t q = direct_slot((int32_t)v, mask);
+        x.dm = cnt[q];
+        x.len = len[v] + x.dm;
+        vi[v] = x;
+        tcnt[v] = x.dm;
+        cnt[q] = 0;  // the cursors of the write pass
+    }
+}
+
 // ------------------------------------------------------------- planning --
 
 struct PlanParams {
@@ -1445,7 +1539,13 @@ struct PlanParams {
     int32_t job_items;   // target estimated items per job (per wavefront)
     int32_t flush_items; // minimum items per owner slot in a job
     int32_t owner_end;   // owners from here up get no jobs (the core's)
+    int32_t id_tiles;    // > 0: owners of bin 2 are tiled by id range, into this many
 };
+
+__device__ inline int32_t owner_tiles(int32_t L, int bin, const PlanParams &P)
+{
+    return bin == 2 && P.id_tiles > 0 ? P.id_tiles : (int32_t)ceil_div(L, P.lmax[bin]);
+}
 
 __device__ inline int32_t est_items(int32_t L, int32_t pl)
 {
@@ -1566,7 +1666,7 @@ __global__ void k_plan_jobs(const VInfo *__restrict__ vi, const unsigned long lo
         unsigned long long w = work[v];
         if (L > 0 && T > 0 && w > 0 && v < P.owner_end && (ORIENTED || x.len >= 2)) {
             int bin = owner_bin(L, P);
-            int64_t tiles = ceil_div(L, P.lmax[bin]);
+            int64_t tiles = owner_tiles(L, bin, P);
             int64_t per_tile = (int64_t)(w / (unsigned long long)tiles) + 1;
             // a job amortises building its LDS table over at least 16 items per slot
             // Each job ends by flushing up to one global atomic per owner slot,
@@ -1604,7 +1704,7 @@ __global__ void k_emit_jobs(const VInfo *__restrict__ vi, const int32_t *__restr
             if (!nj) continue;
             Job *out = bin == 0 ? jobs0 : (bin == 1 ? jobs1 : jobs2);
             int64_t base = jscan[(int64_t)bin * (nv + 1) + v];
-            int32_t tiles = (int32_t)ceil_div(L, P.lmax[bin]);
+            int32_t tiles = owner_tiles(L, bin, P);
             int32_t split = nj / tiles;
             int64_t q = 0;
             for (int32_t t = 0; t < tiles; ++t)
@@ -1684,10 +1784,13 @@ __global__ void k_graph_of(const int64_t *__restrict__ voff, int32_t G,
 
 // ---------------------------------------------------------- count kernel --
 
+enum { kDirect = 0, kOriented = 1, kByTasks = 2 };
+
 struct CountArgs {
     const int32_t *adj;
     const VInfo *vi;
     const TaskRec *tasks;  // oriented: task vertex and suffix of each task
+    const int32_t *cred;   // direct by tasks: the vertex each task's hits go to
     const int64_t *toff;   // oriented: first task of each owner
     const int32_t *order;  // oriented: vertex of each rank
     uint32_t *pcnt;        // oriented: per N+ entry, the hits of its task
@@ -1724,6 +1827,7 @@ struct CountArgs {
     // launch's next job, [1] the length of the list hjobs of the jobs it left
     // to the hash-table launch, [2] that launch's next entry of the list
     unsigned long long *job_ctr;
+    int32_t nv;
     int64_t *hjobs;  // room for every job of the largest bin (or null)
 };
 
@@ -1922,7 +2026,7 @@ __device__ inline void tile_filter(const int32_t *__restrict__ adj, int64_t &pb,
 // batched graphs, this beats 4 to 6 waves (fewer jobs in flight to hide
 // their dependent loads) and, in the mid bin, 8 (64 VGPRs, far more spills:
 // 45 -> 65 ms batched).
-template <int LMAX, int NW, bool ORIENTED>
+template <int LMAX, int NW, int MODE>
 #ifndef TC_MID_WAVES
 #define TC_MID_WAVES 7
 #endif
@@ -1947,6 +2051,9 @@ template <int LMAX, int NW, bool ORIENTED>
 __global__ __launch_bounds__(NW * kWave, LMAX <= 64 ? TC_SMALL_WAVES : LMAX <= 512 ? TC_MID_WAVES : 1) void k_count(const Job *__restrict__ jobs, int64_t njobs,
                                                       CountArgs A)
 {
+    // MODE: kDirect (tasks are the owner's row entries), kOriented, kByTasks
+    // (direct counts by the larger row, see k_direct_tasks)
+    constexpr bool ORIENTED = MODE == kOriented, TASKS = MODE != kDirect;
     // The owner tile lives in a bucketed two-choice hash table (BucketTableT),
     // load <= 1/2, so a lookup reads one bucket, a second only where the
     // first is full, and loops only when both are.  C counts hits per slot
@@ -1981,8 +2088,8 @@ __global__ __launch_bounds__(NW * kWave, LMAX <= 64 ? TC_SMALL_WAVES : LMAX <= 5
         const Job J = jobs[jb];
         const VInfo vo = A.vi[J.owner];
         const int64_t obase = vo.rb;
-        const int64_t tbase = ORIENTED ? A.toff[J.owner] : vo.rb;
-        const int32_t Lfull = ORIENTED ? vo.len - vo.dm : vo.len;
+        const int64_t tbase = TASKS ? A.toff[J.owner] : vo.rb;
+        const int32_t Lfull = TASKS ? vo.len - vo.dm : vo.len;
         const int32_t s0 = J.tile * LMAX;
         const int32_t L = min(LMAX, Lfull - s0);
         const bool tiled = LMAX >= 4096 && Lfull > LMAX;  // smaller bins hold whole lists
@@ -2089,7 +2196,7 @@ __global__ __launch_bounds__(NW * kWave, LMAX <= 64 ? TC_SMALL_WAVES : LMAX <= 5
             int32_t tv = 0, sl = 0;
             int64_t sb = 0;
             if (valid) {
-                if (ORIENTED) {
+                if (TASKS) {
                     const TaskRec tk = A.tasks[tbase + t];
                     sl = tk.len();
                     sb = tk.base();
@@ -2098,11 +2205,11 @@ __global__ __launch_bounds__(NW * kWave, LMAX <= 64 ? TC_SMALL_WAVES : LMAX <= 5
                 }
             }
             VInfo vt = {0, 0, 0};
-            if (!ORIENTED && valid) vt = A.vi[tv];
+            if (!TASKS && valid) vt = A.vi[tv];
             // oriented: the task list is the suffix of N+(tv) after the owner
-            int32_t pl = ORIENTED ? sl : vt.len;
-            int64_t pb = ORIENTED ? sb : vt.rb;
-            if (!ORIENTED && valid &&
+            int32_t pl = TASKS ? sl : vt.len;
+            int64_t pb = TASKS ? sb : vt.rb;
+            if (!TASKS && valid &&
                 (tv == J.owner || vt.len < 2 || vo.len < 2 || (A.skip_lower && tv < J.owner)))
                 valid = false;
             if (!valid) pl = 0;
@@ -2339,6 +2446,8 @@ __global__ __launch_bounds__(NW * kWave, LMAX <= 64 ? TC_SMALL_WAVES : LMAX <= 5
                         atomicAdd(&A.pcnt[sb - 1], c);
                     else
                         A.pcnt[sb - 1] = c;
+                } else if (TASKS) {
+                    atomicAdd(&A.out[A.cred[tbase + t]], c);
                 }
             }
             wave_sync();
@@ -2363,7 +2472,7 @@ __global__ __launch_bounds__(NW * kWave, LMAX <= 64 ? TC_SMALL_WAVES : LMAX <= 5
             }
         }
         const int32_t owner_v = ORIENTED ? A.order[J.owner] : J.owner;
-        if (threadIdx.x == 0 && hjob)
+        if ((ORIENTED || !TASKS) && threadIdx.x == 0 && hjob)
             atomicAdd(&A.out[owner_v], ORIENTED ? (uint32_t)(2 * hjob) : (uint32_t)hjob);
         hits_all += (threadIdx.x == 0) ? hjob : 0ull;
         if (A.per_graph && threadIdx.x == 0 && hjob)
@@ -2594,6 +2703,112 @@ __global__ __launch_bounds__(NW * kWave, BM ? 6 : 4) void k_count_long(const Job
     }
 }
 
+// Direct counts by tasks, owners of more than the small bin's entries: the
+// owner's row as plain bits over its id range (no slots are needed: nothing is
+// credited to the common neighbour), streamed lists as in k_count_long.  A
+// probe is one 4-byte LDS read.  A job takes the WORDS * 32 ids of its tile.
+__device__ inline int32_t row_lower(const int32_t *__restrict__ row, int32_t n, int64_t id)
+{
+    int32_t lo = 0, hi = n;
+    while (lo < hi) {
+        const int32_t mid = (lo + hi) >> 1;
+        if (row[mid] < id) lo = mid + 1; else hi = mid;
+    }
+    return lo;
+}
+
+template <int WORDS, int NT>
+__global__ __launch_bounds__(NT, NT == 512 ? 6 : 4) void k_direct_bits(const Job *__restrict__ jobs, int64_t njobs,
+                                                                     CountArgs A)
+{
+    constexpr int U = 8, NW = NT / kWave;
+    __shared__ uint32_t bits[WORDS + 1];  // (one word past the span: the zero guard word)
+    __shared__ int64_t s_job;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wid = threadIdx.x / kWave;
+    unsigned long long hits_all = 0, n_hash = 0;
+    for (;;) {
+        if (threadIdx.x == 0) s_job = (int64_t)atomicAdd(A.job_ctr, 1ull);
+        __syncthreads();
+        const int64_t jb = s_job;
+        __syncthreads();
+        if (jb >= njobs) break;  // (the same for the block)
+        const Job J = jobs[jb];
+        const VInfo vo = A.vi[J.owner];
+        const int64_t tbase = A.toff[J.owner];
+        int32_t L = vo.len - vo.dm;
+        const int32_t *Sg = A.adj + vo.rb;
+        const bool tiled = A.nv > WORDS * 32;
+        if (tiled) {  // the part of the row in the tile's ids
+            const int32_t lo = row_lower(Sg, L, (int64_t)J.tile * (WORDS * 32));
+            L = row_lower(Sg, L, (int64_t)(J.tile + 1) * (WORDS * 32)) - lo;
+            Sg += lo;
+            if (L == 0) continue;
+        }
+        const int32_t lo_v = Sg[0], hi_v = Sg[L - 1];
+        const int32_t nwords = (int32_t)(((uint32_t)(hi_v - lo_v) >> 5) + 1u);
+        const uint32_t guard = (uint32_t)nwords << 5;
+        for (int i = threadIdx.x; i <= nwords; i += NT) bits[i] = 0u;
+        __syncthreads();
+        // lanes past a list's end read id 0: its bit stays clear, and a list
+        // that starts with 0 has its hit added below
+        for (int i = threadIdx.x; i < L; i += NT) {
+            const int32_t w = Sg[i];
+            const uint32_t off = (uint32_t)(w - lo_v);
+            if (w != 0) atomicOr(&bits[off >> 5], 1u << (off & 31u));
+        }
+        __syncthreads();
+        unsigned long long hits_job = 0;
+        uint32_t hits_own = 0;
+        for (int32_t g0 = 0; J.t_begin + (g0 * kWave) * NW + wid < J.t_end; ++g0) {
+            const int32_t t = J.t_begin + (g0 * kWave + lane) * NW + wid;
+            int32_t pl = 0, cr = J.owner;
+            int64_t pb = 0;
+            uint32_t h0 = 0;
+            if (t < J.t_end) {
+                const TaskRec tk = A.tasks[tbase + t];
+                cr = A.cred[tbase + t];
+                pl = tk.len();
+                pb = tk.base();
+                if (tiled) tile_filter(A.adj, pb, pl, lo_v, hi_v);
+                if (lo_v == 0 && pl > 0) h0 = A.adj[pb] == 0;
+            }
+            n_hash += pl > 0;
+            const uint32_t h = h0 + stream_tasks<U, true>(A.adj, pl, pb, [&](const int32_t (&w)[U], uint32_t (&hc)[U]) {
+                uint32_t off[U], x[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    off[u] = min((uint32_t)(w[u] - lo_v), guard);  // w < lo wraps high
+                    x[u] = bits[off[u] >> 5];
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    hc[u] = (uint32_t)__popcll(__ballot(__builtin_amdgcn_ubfe(x[u], off[u], 1u) != 0u));
+            });
+            if (h) {
+                hits_job += h;
+                if (cr == J.owner)
+                    hits_own += h;
+                else
+                    atomicAdd(&A.out[cr], h);
+            }
+        }
+        const uint32_t own = wave_sum<uint32_t>(hits_own);
+        const unsigned long long hj = wave_sum<unsigned long long>(hits_job);
+        if (lane == 0) {
+            if (own) atomicAdd(&A.out[J.owner], own);
+            if (hj && A.per_graph) atomicAdd(&A.per_graph[A.gid[J.owner]], hj);
+            hits_all += hj;
+        }
+        __syncthreads();
+    }
+    if (lane == 0 && hits_all) atomicAdd(A.global, hits_all);
+    if (A.strat) {
+        const unsigned long long nh = wave_sum<unsigned long long>(n_hash);
+        if (lane == 0 && nh) atomicAdd(&A.strat[S_HASH], nh);
+    }
+}
+
 // ------------------------------------------------------------- driver --
 
 tc_schedule default_schedule()
@@ -2620,12 +2835,16 @@ constexpr int kHubDegree = 65536;  // with the appends
 #define TC_MID_NW 2
 #endif
 constexpr int kNW0 = 1, kNW1 = TC_MID_NW, kNW2 = 8;
+// ids of a bit row in LDS (k_direct_bits): 32 KB, four blocks of 8 waves a CU,
+// and 128 KB, one block of 16
+constexpr int kBitsIds0 = 1 << 18, kBitsIds1 = 1 << 20;
 
 // ev_long (bin 2, oriented): events recorded before and after the bitmap-tile
 // launch of k_count_long and after its hash-table-tile launch.
-int launch_bin(int bin, bool oriented, const Job *jobs, int64_t njobs, const CountArgs &A,
+int launch_bin(int bin, int mode, const Job *jobs, int64_t njobs, const CountArgs &A,
                hipStream_t s, hipEvent_t *ev_long)
 {
+    const bool oriented = mode == kOriented;
     if (njobs <= 0) return TC_OK;
     int dev = 0;
     TC_HIP(hipGetDevice(&dev));
@@ -2634,16 +2853,27 @@ int launch_bin(int bin, bool oriented, const Job *jobs, int64_t njobs, const Cou
     // persistent grid: enough resident blocks to fill every CU
     int per_cu = bin == 0 ? 4 * TC_SMALL_WAVES / kNW0 : (bin == 1 ? 4 * TC_MID_WAVES / kNW1 : 2);
     int64_t grid = std::min<int64_t>(njobs, (int64_t)cus * per_cu);
-    if (bin == 0) {
-        if (oriented)
-            hipLaunchKernelGGL((k_count<kL0, kNW0, true>), dim3((unsigned)grid), dim3(kNW0 * kWave), 0, s, jobs, njobs, A);
+    if (mode == kByTasks) {
+        if (bin == 0)
+            hipLaunchKernelGGL((k_count<kL0, kNW0, kByTasks>), dim3((unsigned)grid), dim3(kNW0 * kWave), 0, s, jobs, njobs, A);
+        else if (bin == 1)
+            hipLaunchKernelGGL((k_count<kL1, kNW1, kByTasks>), dim3((unsigned)grid), dim3(kNW1 * kWave), 0, s, jobs, njobs, A);
+        else if (A.nv <= kBitsIds0)
+            hipLaunchKernelGGL((k_direct_bits<kBitsIds0 / 32, 512>), dim3((unsigned)std::min<int64_t>(njobs, cus * 3)),
+                               dim3(512), 0, s, jobs, njobs, A);
         else
-            hipLaunchKernelGGL((k_count<kL0, kNW0, false>), dim3((unsigned)grid), dim3(kNW0 * kWave), 0, s, jobs, njobs, A);
+            hipLaunchKernelGGL((k_direct_bits<kBitsIds1 / 32, 1024>), dim3((unsigned)std::min<int64_t>(njobs, cus)),
+                               dim3(1024), 0, s, jobs, njobs, A);
+    } else if (bin == 0) {
+        if (oriented)
+            hipLaunchKernelGGL((k_count<kL0, kNW0, kOriented>), dim3((unsigned)grid), dim3(kNW0 * kWave), 0, s, jobs, njobs, A);
+        else
+            hipLaunchKernelGGL((k_count<kL0, kNW0, kDirect>), dim3((unsigned)grid), dim3(kNW0 * kWave), 0, s, jobs, njobs, A);
     } else if (bin == 1) {
         if (oriented)
-            hipLaunchKernelGGL((k_count<kL1, kNW1, true>), dim3((unsigned)grid), dim3(kNW1 * kWave), 0, s, jobs, njobs, A);
+            hipLaunchKernelGGL((k_count<kL1, kNW1, kOriented>), dim3((unsigned)grid), dim3(kNW1 * kWave), 0, s, jobs, njobs, A);
         else
-            hipLaunchKernelGGL((k_count<kL1, kNW1, false>), dim3((unsigned)grid), dim3(kNW1 * kWave), 0, s, jobs, njobs, A);
+            hipLaunchKernelGGL((k_count<kL1, kNW1, kDirect>), dim3((unsigned)grid), dim3(kNW1 * kWave), 0, s, jobs, njobs, A);
     } else {
         if (oriented) {
             // short tasks here, long hash tasks in k_count_long (bitmap and
@@ -2658,7 +2888,7 @@ int launch_bin(int bin, bool oriented, const Job *jobs, int64_t njobs, const Cou
             const bool forced = A.policy == TC_POLICY_MERGE || A.policy == TC_POLICY_BSEARCH ||
                                 A.policy == TC_POLICY_MERGEPATH;
             if (forced)
-                hipLaunchKernelGGL((k_count<kL2, kNW2, true>), dim3((unsigned)grid), dim3(kNW2 * kWave), 0, s, jobs, njobs, As);
+                hipLaunchKernelGGL((k_count<kL2, kNW2, kOriented>), dim3((unsigned)grid), dim3(kNW2 * kWave), 0, s, jobs, njobs, As);
             const int64_t gb = std::min<int64_t>(njobs, (int64_t)cus * 3);
             const int64_t gh = std::min<int64_t>(njobs, (int64_t)cus * 2);
             if (ev_long) TC_HIP(hipEventRecord(ev_long[0], s));
@@ -2669,7 +2899,7 @@ int launch_bin(int bin, bool oriented, const Job *jobs, int64_t njobs, const Cou
                 hipLaunchKernelGGL((k_count_long<kL2, kNW2, false>), dim3((unsigned)gh), dim3(kNW2 * kWave), 0, s, jobs, njobs, Al);
             if (ev_long) TC_HIP(hipEventRecord(ev_long[2], s));
         } else
-            hipLaunchKernelGGL((k_count<kL2, kNW2, false>), dim3((unsigned)grid), dim3(kNW2 * kWave), 0, s, jobs, njobs, A);
+            hipLaunchKernelGGL((k_count<kL2, kNW2, kDirect>), dim3((unsigned)grid), dim3(kNW2 * kWave), 0, s, jobs, njobs, A);
     }
     TC_HIP(hipGetLastError());
     return TC_OK;
@@ -3001,6 +3231,51 @@ extern const uint8_t *learned_table_device(int32_t *dim);
 
 namespace {
 
+// Whether a direct count goes by the larger row: default strategies (a forced
+// one names the kernels of the row entries), rows below 2^24 entries (task
+// records), and hubs, without which the shorter list is no shorter (the same
+// bound as the core's).
+bool direct_by_tasks(const Graph &g, const tc_schedule &sched)
+{
+    return (sched.policy == TC_POLICY_FIXED || sched.policy == TC_POLICY_LEARNED) && sched.ratio_x16 <= 0 &&
+           sched.mpath_min <= 0 && g.st.nv < (1 << 24) && g.validated &&
+           (double)g.max_degree * g.st.nv >= 16.0 * (double)g.st.nnz;
+}
+
+// The task lists of a direct count by the larger row (after the direct views):
+// offsets in ov[6], chunk rows in ov[10], records in tasks, credits in ov[16].
+int prepare_direct_tasks(Graph &g, bool skip_lower)
+{
+    const int32_t nv = g.st.nv;
+    const int64_t nnz = g.st.nnz, nchunks = ceil_div(nnz, kWave);
+    hipStream_t s = g.stream;
+    const int vblocks = grid_for(nv, 256, 65536), wblocks = grid_for(nchunks, 4, 1 << 16);
+    const uint32_t slots = 1u << std::max(1, ceil_log2_i((int64_t)nv)), mask = slots - 1;
+    TC_TRY(g.ov[2].ensure((size_t)slots * sizeof(int32_t)));
+    TC_TRY(g.ov[0].ensure((size_t)nv * sizeof(int32_t)));
+    TC_TRY(g.ov[6].ensure((size_t)(nv + 1) * sizeof(int64_t)));
+    TC_TRY(g.ov[10].ensure((size_t)(nchunks + 1) * sizeof(int32_t)));
+    TC_TRY(g.tasks.ensure((size_t)nnz * sizeof(TaskRec)));
+    TC_TRY(g.ov[16].ensure((size_t)nnz * sizeof(int32_t)));
+    int32_t *cnt = g.ov[2].as<int32_t>(), *tcnt = g.ov[0].as<int32_t>();
+    int64_t *toff = g.ov[6].as<int64_t>();
+    const int64_t *coff = g.coff.as<int64_t>(), *boff = g.st.boff.as<int64_t>();
+    const int32_t *crow = g.crow.as<int32_t>(), *len = g.st.len.as<int32_t>(), *pool = g.st.pool.as<int32_t>();
+    hipLaunchKernelGGL(k_fill_u32, dim3(vblocks), dim3(256), 0, s, reinterpret_cast<uint32_t *>(cnt),
+                       (int64_t)slots, 0u);
+    hipLaunchKernelGGL(k_direct_tasks<false>, dim3(wblocks), dim3(256), 0, s, coff, crow, boff, len, pool, nv, nnz,
+                       skip_lower ? 1 : 0, cnt, mask, nullptr, nullptr, nullptr);
+    TC_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_direct_task_vinfo, dim3(vblocks), dim3(256), 0, s, boff, len, cnt, mask, nv,
+                       g.vinfo.as<VInfo>(), tcnt);
+    TC_TRY(scan_counts_i32(tcnt, toff, nv, g.tmp, s));
+    hipLaunchKernelGGL(k_direct_tasks<true>, dim3(wblocks), dim3(256), 0, s, coff, crow, boff, len, pool, nv, nnz,
+                       skip_lower ? 1 : 0, cnt, mask, toff, g.tasks.as<TaskRec>(), g.ov[16].as<int32_t>());
+    hipLaunchKernelGGL(k_chunk_rows, dim3(vblocks), dim3(256), 0, s, toff, nv, g.ov[10].as<int32_t>());
+    TC_HIP(hipGetLastError());
+    return TC_OK;
+}
+
 // The per-bin counters of a count (accum words, see count_pass) into stats.
 void fill_counters(tc_stats &st, const unsigned long long *hacc, const int64_t *jt, bool oriented)
 {
@@ -3133,15 +3408,27 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
         }
     }
     if (!oriented) TC_TRY(prepare_views(g, false));
+    int mode = oriented ? kOriented : kDirect;
+    if (!oriented && direct_by_tasks(g, sched)) {
+        const int dt = prepare_direct_tasks(g, skip_lower);
+        if (dt == TC_OK) {
+            mode = kByTasks;
+        } else if (dt == TC_ERR_OOM) {  // no room for the lists: the row entries themselves
+            g.tasks.release();
+            g.ov[16].release();
+            TC_TRY(build_direct_vinfo(g));
+        } else {
+            return dt;
+        }
+    }
     st.method_used = method;
-    int64_t *coff = g.coff.as<int64_t>();
-    int32_t *crow = g.crow.as<int32_t>();
+    int64_t *coff = mode == kByTasks ? g.ov[6].as<int64_t>() : g.coff.as<int64_t>();
+    int32_t *crow = mode == kByTasks ? g.ov[10].as<int32_t>() : g.crow.as<int32_t>();
     VInfo *vi = g.vinfo.as<VInfo>();
     const int32_t *adj = oriented ? g.padj.as<int32_t>() : g.st.pool.as<int32_t>();
-    const TaskRec *tasks = oriented ? g.tasks.as<TaskRec>() : nullptr;
-    // planning walks the task array (oriented) or the store rows (direct)
-    const int64_t nent = oriented ? g.ntasks : nnz;
-    const int64_t nchunks = ceil_div(nent, kWave);
+    const TaskRec *tasks = mode != kDirect ? g.tasks.as<TaskRec>() : nullptr;
+    // planning walks the task array (oriented, by tasks) or the store rows (direct)
+    const int64_t nchunks = ceil_div(oriented ? g.ntasks : nnz, kWave);
     // 4 waves of 256 threads; 16 blocks per CU keep the chip busy and bound
     // the number of per-block statistics atomics
     const int wblocks = grid_for(nchunks, 4, 4096);
@@ -3159,10 +3446,25 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     P.job_items = std::max(sched.job_items, 256);
     P.flush_items = sched.flush_items > 0 ? sched.flush_items : 1024;
     P.owner_end = nv - (oriented ? g.core_k : 0);
+    // by tasks: bit rows hold any list whole, and a job of theirs ends without a
+    // flush.  Beyond kBitsIds1 ids a row is tiled by id range, which pays for
+    // the largest bin only (the mid bin's lists go through LDS tables).
+    P.id_tiles = 0;
+    const bool one_bits = mode == kByTasks && nv <= kBitsIds1;  // bins 1 and 2 in one launch
+    if (mode == kByTasks) {
+        P.id_tiles = (int32_t)ceil_div(nv, kBitsIds1);
+        P.lmax[2] = INT32_MAX;
+        P.nw[2] = 8;
+        P.flush_items = 16;
+        if (one_bits) {
+            P.lmax[1] = INT32_MAX;
+            P.nw[1] = 8;
+        }
+    }
     TC_TRY(g.work.ensure((size_t)nv * sizeof(unsigned long long)));
     unsigned long long *work = g.work.as<unsigned long long>();
     hipLaunchKernelGGL(k_fill_u64, dim3(grid_for(nv, 256, 65536)), dim3(256), 0, s, work, (int64_t)nv);
-    if (oriented)
+    if (mode != kDirect)
         hipLaunchKernelGGL(k_owner_work<true>, dim3(wblocks), dim3(256), 0, s, coff, crow, vi, adj,
                            tasks, nv, P, work, stats ? acc + 4 : nullptr);
     else
@@ -3172,7 +3474,7 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     TC_TRY(g.tmp3.ensure((size_t)3 * nv * sizeof(int32_t) + (size_t)3 * (nv + 1) * sizeof(int64_t) + 16));
     int32_t *njobs = g.tmp3.as<int32_t>();
     int64_t *jscan = reinterpret_cast<int64_t *>(njobs + 3 * (int64_t)nv + ((3 * (int64_t)nv) & 1));
-    if (oriented)
+    if (mode != kDirect)
         hipLaunchKernelGGL(k_plan_jobs<true>, dim3(grid_for(nv, 256, 4096)), dim3(256), 0, s, vi,
                            work, nv, P, njobs, stats ? acc + 13 : nullptr);
     else
@@ -3193,7 +3495,7 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     Job *j0 = g.jobs.as<Job>();
     Job *j1 = j0 + jt[0];
     Job *j2 = j1 + jt[1];
-    if (oriented)
+    if (mode != kDirect)
         hipLaunchKernelGGL(k_emit_jobs<true>, dim3(grid_for(nv, 256, 65536)), dim3(256), 0, s, vi,
                            njobs, jscan, nv, P, j0, j1, j2);
     else
@@ -3208,7 +3510,9 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     A.vi = vi;
     A.tasks = tasks;
     A.pcnt = nullptr;
-    A.toff = oriented ? coff : nullptr;
+    A.toff = mode != kDirect ? coff : nullptr;
+    A.cred = mode == kByTasks ? g.ov[16].as<int32_t>() : nullptr;
+    A.nv = nv;
     A.order = oriented ? g.order.as<int32_t>() : nullptr;
     A.out = outp;
     A.global = acc;
@@ -3256,7 +3560,10 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     const Job *jl[3] = {j0, j1, j2};
     for (int b = 0; b < 3; ++b) {
         TC_HIP(rec(g.ev[3 + b]));
-        TC_TRY(launch_bin(b, oriented, jl[b], jt[b], A, s, g.capturing ? nullptr : &g.ev[8]));
+        // bit rows of any list: the mid and largest bins' jobs in one launch
+        if (one_bits && b == 1) continue;
+        const int64_t nj = one_bits && b == 2 ? jt[1] + jt[2] : jt[b];
+        TC_TRY(launch_bin(b, mode, one_bits && b == 2 ? jl[1] : jl[b], nj, A, s, g.capturing ? nullptr : &g.ev[8]));
     }
     TC_HIP(rec(g.ev[6]));  // end of the bin kernels
     if (oriented && g.core_k > 0) TC_TRY(core_count(g, acc, reinterpret_cast<int32_t *>(acc + 27), A.gid));
