@@ -96,7 +96,13 @@ int tc_version(void) { return 10000; }
 int tc_device_alloc(void **ptr, uint64_t bytes)
 {
     TC_CHECK_ARG(ptr, "tc_device_alloc: null ptr");
-    if (hipMalloc(ptr, bytes ? bytes : 16) != hipSuccess) {
+    hipError_t e = hipMalloc(ptr, bytes ? bytes : 16);
+    if (e == hipErrorOutOfMemory) {  // the pool's blocks go first
+        (void)hipGetLastError();
+        tc::pool_flush();
+        e = hipMalloc(ptr, bytes ? bytes : 16);
+    }
+    if (e != hipSuccess) {
         (void)hipGetLastError();
         *ptr = nullptr;
         tc::set_last_error(TC_ERR_OOM, "hipMalloc failed");

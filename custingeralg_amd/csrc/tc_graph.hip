@@ -5,7 +5,9 @@
 #include "tc_internal.hpp"
 
 #include <algorithm>
+#include <map>
 #include <mutex>
+#include <vector>
 
 namespace tc {
 
@@ -17,33 +19,155 @@ void set_last_error(int code, const std::string &msg)
     g_last.msg = msg;
 }
 
+// ------------------------------------------------------- block pool --
+// A graph's handle owns some sixty device blocks, and a program that counts
+// graphs as they arrive paid for them on every handle: hipMalloc and hipFree
+// were 3 to 26 of the 5 to 28 ms that a new graph of 250k vertices took (the
+// cost of mapping differs from run to run).  Released blocks are kept here, by
+// size and device, and handed to the next handle.
+//   Bounded: kHoldBytes in all, no block above kHoldBlock; what exceeds it is
+//   freed, the largest first, and everything held is freed when an allocation
+//   fails.
+//   Safe across streams and threads: a block is given back only when its
+//   device is idle (DevBuf::release synchronises, as hipFree does), so no
+//   kernel of its last owner can still touch it; the lists are under a lock.
+namespace {
+
+constexpr size_t kHoldBytes = size_t(4) << 30;
+constexpr size_t kHoldBlock = size_t(1) << 30;
+
+struct HostKit {  // pinned words and events of a handle, by device
+    int dev;
+    unsigned long long *words;
+    hipEvent_t ev[16];
+};
+constexpr size_t kHoldKits = 32;
+
+struct BlockPool {
+    std::mutex mu;
+    std::multimap<std::pair<int, size_t>, void *> blocks;  // (device, bytes)
+    size_t held = 0;
+    std::vector<HostKit> kits;
+};
+
+// Never destroyed: at exit the runtime may be gone before a destructor runs.
+BlockPool &block_pool()
+{
+    static BlockPool *p = new BlockPool;
+    return *p;
+}
+
+// Sizes requests share: powers of two up to 1 MB, then eighths of one; blocks
+// that the pool would not keep stay exact.
+size_t block_size(size_t need)
+{
+    if (need > kHoldBlock) return need;
+    size_t p2 = 4096;
+    while (p2 < need) p2 <<= 1;
+    if (p2 <= (size_t(1) << 20)) return p2;
+    const size_t step = p2 / 16;
+    return (need + step - 1) / step * step;
+}
+
+void *pool_take(int dev, size_t bytes, size_t &got)
+{
+    BlockPool &P = block_pool();
+    std::lock_guard<std::mutex> lock(P.mu);
+    auto it = P.blocks.lower_bound({dev, bytes});
+    if (it == P.blocks.end() || it->first.first != dev || it->first.second > bytes + bytes / 4) return nullptr;
+    void *p = it->second;
+    got = it->first.second;
+    P.held -= got;
+    P.blocks.erase(it);
+    return p;
+}
+
+void pool_give(int dev, void *p, size_t bytes)
+{
+    std::vector<void *> out;
+    if (bytes > kHoldBlock) {
+        out.push_back(p);
+    } else {
+        BlockPool &P = block_pool();
+        std::lock_guard<std::mutex> lock(P.mu);
+        P.blocks.insert({{dev, bytes}, p});
+        P.held += bytes;
+        while (P.held > kHoldBytes) {
+            auto big = P.blocks.begin();
+            for (auto it = P.blocks.begin(); it != P.blocks.end(); ++it)
+                if (it->first.second > big->first.second) big = it;
+            P.held -= big->first.second;
+            out.push_back(big->second);
+            P.blocks.erase(big);
+        }
+    }
+    for (void *q : out) (void)hipFree(q);
+}
+
+}  // namespace
+
+void pool_flush()
+{
+    std::vector<void *> out;
+    {
+        BlockPool &P = block_pool();
+        std::lock_guard<std::mutex> lock(P.mu);
+        for (auto &b : P.blocks) out.push_back(b.second);
+        P.blocks.clear();
+        P.held = 0;
+    }
+    for (void *q : out) (void)hipFree(q);
+}
+
 int DevBuf::ensure(size_t need)
 {
     if (need == 0) need = 16;
     if (bytes >= need) return TC_OK;
     // a buffer that has to grow again gets 25% headroom: batch-sized scratch
-    // varies from call to call, and every regrowth stalls the device (free,
-    // then allocate); a first allocation is exact
+    // varies from call to call, and every regrowth stalls the device
     if (p) {
-        (void)hipFree(p);
-        p = nullptr;
-        bytes = 0;
+        release();
         need += need / 4;
     }
-    hipError_t e = hipMalloc(&p, need);
-    if (e != hipSuccess) {
-        p = nullptr;
-        (void)hipGetLastError();
-        set_last_error(TC_ERR_OOM, "hipMalloc of " + std::to_string(need) + " bytes failed");
-        return TC_ERR_OOM;
+    (void)hipGetDevice(&dev);
+    const size_t want = block_size(need);
+    size_t got = want;
+    p = pool_take(dev, want, got);
+    if (!p) {
+        hipError_t e = hipMalloc(&p, want);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            pool_flush();
+            e = hipMalloc(&p, want);
+        }
+        if (e != hipSuccess) {
+            p = nullptr;
+            (void)hipGetLastError();
+            set_last_error(TC_ERR_OOM, "hipMalloc of " + std::to_string(need) + " bytes failed");
+            return TC_ERR_OOM;
+        }
     }
-    bytes = need;
+    bytes = got;
     return TC_OK;
 }
 
-void DevBuf::release()
+void DevBuf::release(bool idle)
 {
-    if (p) (void)hipFree(p);
+    if (p) {
+        int now = dev;
+        (void)hipGetDevice(&now);
+        if (now != dev) {  // another device's block: freed, as this thread cannot wait for it
+            (void)hipFree(p);
+        } else {
+            // (a capturing thread cannot synchronise: the block is not reused)
+            if (idle || hipDeviceSynchronize() == hipSuccess) {
+                pool_give(dev, p, bytes);
+            } else {
+                (void)hipGetLastError();
+                (void)hipFree(p);
+            }
+        }
+    }
     p = nullptr;
     bytes = 0;
 }
@@ -51,12 +175,49 @@ void DevBuf::release()
 int Graph::ensure_events()
 {
     if (events_ready) return TC_OK;
+    int now = 0;
+    TC_HIP(hipGetDevice(&now));
+    if (!hcounts) {
+        BlockPool &P = block_pool();
+        std::lock_guard<std::mutex> lock(P.mu);
+        for (size_t k = 0; k < P.kits.size(); ++k)
+            if (P.kits[k].dev == now) {
+                hcounts = P.kits[k].words;
+                std::copy(P.kits[k].ev, P.kits[k].ev + 16, ev);
+                P.kits.erase(P.kits.begin() + (long)k);
+                kit_dev = now;
+                events_ready = true;
+                return TC_OK;
+            }
+    }
     if (!hcounts)
         TC_HIP(hipHostMalloc(reinterpret_cast<void **>(&hcounts), 32 * sizeof(unsigned long long),
                              hipHostMallocDefault));
     for (auto &e : ev) TC_HIP(hipEventCreate(&e));
+    kit_dev = now;
     events_ready = true;
     return TC_OK;
+}
+
+void Graph::drop_events()
+{
+    if (events_ready) {
+        BlockPool &P = block_pool();
+        std::lock_guard<std::mutex> lock(P.mu);
+        if (P.kits.size() < kHoldKits) {
+            HostKit k = {kit_dev, hcounts, {}};
+            std::copy(ev, ev + 16, k.ev);
+            P.kits.push_back(k);
+            hcounts = nullptr;
+            events_ready = false;
+            return;
+        }
+    }
+    if (events_ready)
+        for (auto &e : ev) (void)hipEventDestroy(e);
+    if (hcounts) (void)hipHostFree(hcounts);
+    hcounts = nullptr;
+    events_ready = false;
 }
 
 void Graph::drop_capture()
@@ -288,11 +449,7 @@ int graph_create_csr(int32_t nv, int64_t nnz, const int64_t *off, const int32_t 
     g->st.nv = nv;
     g->st.nnz = nnz;
     auto fail = [&](int code) {
-        g->st.boff.release();
-        g->st.len.release();
-        g->st.cap.release();
-        g->st.pool.release();
-        delete g;
+        graph_destroy(g);
         return code;
     };
     int st;
@@ -528,7 +685,7 @@ int graph_compare(Graph &a, Graph &b, int64_t *size_mismatch, int64_t *entry_mis
 void graph_destroy(Graph *g)
 {
     if (!g) return;
-    (void)hipDeviceSynchronize();
+    const bool idle = hipDeviceSynchronize() == hipSuccess;
     if (g->borrowed) {
         g->st.pool.p = nullptr;
         g->st.pool.bytes = 0;
@@ -539,13 +696,11 @@ void graph_destroy(Graph *g)
                       &g->bvals2, &g->boffb, &g->bdel, &g->flagpool, &g->vmark, &g->order,
                       &g->rnk, &g->tasks, &g->pcnt, &g->hjobs, &g->outr, &g->dmat, &g->ditems,
                       &g->dgraphs, &g->dgid, &g->cmat, &g->cgraphs, &g->cblocks};
-    for (DevBuf *b : bufs) b->release();
-    for (DevBuf &b : g->sb) b.release();
-    for (DevBuf &b : g->ov) b.release();
-    for (DevBuf &b : g->lbuf) b.release();
-    if (g->events_ready)
-        for (auto &e : g->ev) (void)hipEventDestroy(e);
-    if (g->hcounts) (void)hipHostFree(g->hcounts);
+    for (DevBuf *b : bufs) b->release(idle);
+    for (DevBuf &b : g->sb) b.release(idle);
+    for (DevBuf &b : g->ov) b.release(idle);
+    for (DevBuf &b : g->lbuf) b.release(idle);
+    g->drop_events();
     g->drop_capture();
     if (g->bexec) (void)hipGraphExecDestroy(g->bexec);
     if (g->bgraph) (void)hipGraphDestroy(g->bgraph);

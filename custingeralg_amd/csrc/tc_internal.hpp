@@ -42,13 +42,19 @@ void set_last_error(int code, const std::string &msg);
 
 // ------------------------------------------------------- device buffers --
 // Scratch allocations are owned by the graph handle and grown on demand.
+// Blocks come from and go back to a bounded pool (tc_graph.hip); release()
+// waits for the device unless the caller knows that it is idle.
 struct DevBuf {
     void *p = nullptr;
     size_t bytes = 0;
+    int dev = 0;
     int ensure(size_t need);
-    void release();
+    void release(bool idle = false);
     template <class T> T *as() const { return static_cast<T *>(p); }
 };
+
+// Frees every block that the pool holds.
+void pool_flush();
 
 // ------------------------------------------------------------- helpers --
 __host__ __device__ inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
@@ -174,7 +180,9 @@ struct Graph {
     bool borrowed = false;
     hipEvent_t ev[16] = {};
     bool events_ready = false;
+    int kit_dev = 0;
     int ensure_events();
+    void drop_events();
     // pinned host words the batch sequence's counts are copied to (32)
     unsigned long long *hcounts = nullptr;
     // store version: bumped by every update, so that plans and recorded

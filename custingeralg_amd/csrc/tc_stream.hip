@@ -1205,8 +1205,9 @@ int ensure_flags(Graph &g)
     if (g.flagpool.bytes < cap) {
         DevBuf nf;
         TC_TRY(nf.ensure(cap));
-        hipLaunchKernelGGL(k_zero_bytes, dim3(grid_for((int64_t)cap, 256, 65536)), dim3(256), 0,
-                           g.stream, nf.as<uint8_t>(), (int64_t)cap);
+        // (all of the block: it may be larger than asked for)
+        hipLaunchKernelGGL(k_zero_bytes, dim3(grid_for((int64_t)nf.bytes, 256, 65536)), dim3(256), 0,
+                           g.stream, nf.as<uint8_t>(), (int64_t)nf.bytes);
         if (g.flagpool.p && g.st.pool_used > 0)
             TC_HIP(hipMemcpyAsync(nf.p, g.flagpool.p, (size_t)g.st.pool_used, hipMemcpyDeviceToDevice,
                                   g.stream));
@@ -1228,13 +1229,13 @@ int ensure_pool(Graph &g, int64_t extra)
     int64_t ncap = std::max<int64_t>(2 * cap, g.st.pool_used + extra + 1024);
     DevBuf np, nf;
     TC_TRY(np.ensure((size_t)ncap * sizeof(int32_t)));
-    int st = nf.ensure((size_t)ncap);
+    int st = nf.ensure(np.bytes / sizeof(int32_t));
     if (st != TC_OK) {
         np.release();
         return st;
     }
-    hipLaunchKernelGGL(k_zero_bytes, dim3(grid_for(ncap, 256, 65536)), dim3(256), 0, g.stream,
-                       nf.as<uint8_t>(), ncap);
+    hipLaunchKernelGGL(k_zero_bytes, dim3(grid_for((int64_t)nf.bytes, 256, 65536)), dim3(256), 0, g.stream,
+                       nf.as<uint8_t>(), (int64_t)nf.bytes);
     if (g.st.pool_used > 0) {
         TC_HIP(hipMemcpyAsync(np.p, g.st.pool.p, (size_t)g.st.pool_used * sizeof(int32_t),
                               hipMemcpyDeviceToDevice, g.stream));
