@@ -411,6 +411,7 @@ int validate_graph(Graph &g, bool check_symmetry, int64_t *bad_rows)
     g.self_loops = (int64_t)h[2];
     if (check_symmetry) g.symmetric = h[3] == 0 ? 1 : 0;
     g.max_degree = (int32_t)h[4];
+    g.degree_stale = false;
     // bit matrices hold a graph's own columns only
     if (h[5]) {
         g.dense_words = 0;

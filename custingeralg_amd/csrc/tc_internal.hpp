@@ -245,6 +245,12 @@ int dense_count(Graph &g, uint32_t *out, unsigned long long *acc, int32_t *bad, 
                 bool skip_lower, hipEvent_t built);
 int dense_plan_batched(Graph &g);
 
+// Counts of graphs whose rows are all short (tc_rows.hip), as dense_eligible
+// and dense_count.
+bool rows_eligible(const Graph &g, const tc_schedule &sched);
+int rows_count(Graph &g, uint32_t *out, unsigned long long *acc, int32_t *bad, bool oriented, bool skip_lower,
+               hipEvent_t built);
+
 // The core of the rank order on a bit matrix (tc_core.hip): how many ranks it
 // takes (0: none), and its share of an oriented count, added to g.outr and
 // acc[0]; *bad is set where the rows turn out not to be symmetric.

@@ -3334,7 +3334,8 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     // tasks
     TC_TRY(g.accum.ensure(32 * sizeof(unsigned long long)));
     unsigned long long *acc = g.accum.as<unsigned long long>();
-    const bool dense = nnz > 0 && dense_eligible(g, sched);
+    const bool rows = nnz > 0 && rows_eligible(g, sched);
+    const bool dense = rows || (nnz > 0 && dense_eligible(g, sched));
     uint32_t *outp = out;
     if (!outp) {
         TC_TRY(g.tmp4.ensure((size_t)std::max<int32_t>(nv, 1) * sizeof(uint32_t)));
@@ -3359,10 +3360,11 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     }
 
     if (dense) {
-        // few vertices: bit rows (every tc_stats counter of tasks and jobs
-        // stays 0; ms_prepare is the matrix, ms_count the intersections)
+        // few vertices: bit rows; short rows: the rows as they are (every
+        // tc_stats counter of tasks and jobs stays 0; ms_prepare is the matrix,
+        // ms_count the intersections)
         int32_t *bad = reinterpret_cast<int32_t *>(acc + 27);
-        TC_TRY(dense_count(g, outp, acc, bad, oriented, skip_lower, g.capturing ? nullptr : g.ev[2]));
+        TC_TRY((rows ? rows_count : dense_count)(g, outp, acc, bad, oriented, skip_lower, g.capturing ? nullptr : g.ev[2]));
         g.plan.method = method;
         g.plan.bad = bad;
         for (int64_t &j : g.plan.jt) j = 0;
