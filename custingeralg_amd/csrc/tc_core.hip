@@ -65,8 +65,10 @@ __global__ __launch_bounds__(256) void k_core_rows(const VInfo *__restrict__ vi,
                                                    int32_t k, CoreGraph one,
                                                    const CoreGraph *__restrict__ graphs,
                                                    const int32_t *__restrict__ gid, uint32_t *__restrict__ mat,
-                                                   uint32_t *__restrict__ pcount)
+                                                   uint32_t *__restrict__ pcount,
+                                                   const unsigned long long *__restrict__ fault)
 {
+    if (*fault) return;  // (rows not symmetric: the plus array was not written)
     constexpr int words = Q * (kCoreCols / 32);
     __shared__ alignas(16) uint32_t lds[256 / kWave][words];
     const int lane = threadIdx.x & (kWave - 1);
@@ -136,6 +138,7 @@ struct CoreArgs {
     uint32_t *pcount;  // plus entries that point to each core vertex, zero on entry
     unsigned long long *global;
     unsigned long long *per_graph;  // may be null
+    const unsigned long long *fault;
 };
 
 template <int Q>
@@ -314,6 +317,7 @@ template <int Q>
 __global__ __launch_bounds__(kCoreThreads, Q <= 2 ? 7 : 6) void k_core_count(CoreArgs A)
 {
     __shared__ CoreShared<Q> S;
+    if (*A.fault) return;  // (set before this kernel: the same for all)
     const int t = threadIdx.x;
     CoreGraph D = A.one;
     int32_t part = blockIdx.x, parts = gridDim.x, graph = 0;
@@ -480,7 +484,7 @@ int core_launch(Graph &g, CoreArgs A, int32_t *bad, const int32_t *gid, int64_t 
     A.pcount = mat + words;
     const int32_t graphs = A.graphs ? g.batch_ngraphs : 1, nblk = A.graphs ? 8 : 512;
     hipLaunchKernelGGL(k_core_rows<Q>, dim3(grid_for(k, 4)), dim3(256), 0, s, A.vi, A.padj, A.core_lo, k, A.one,
-                       A.graphs, gid, mat, A.pcount);
+                       A.graphs, gid, mat, A.pcount, A.fault);
     hipLaunchKernelGGL(k_core_transpose<Q>, dim3((unsigned)(nblk * (int64_t)graphs)), dim3(256), 0, s, A.one,
                        A.graphs, nblk, mat);
     hipLaunchKernelGGL(k_core_count<Q>, dim3((unsigned)grid), dim3(kCoreThreads), 0, s, A);
@@ -501,6 +505,7 @@ int core_count(Graph &g, unsigned long long *acc, int32_t *bad, const int32_t *g
     A.core_lo = nv - k;
     A.outr = g.outr.as<uint32_t>();
     A.global = acc;
+    A.fault = acc + 27;
     if (g.batch_voff) {
         A.graphs = g.cgraphs.as<CoreGraph>();
         A.blocks = g.cblocks.as<CoreBlock>();

@@ -198,10 +198,7 @@ struct Graph {
         uint64_t key = 0;
         int method = 0;
         unsigned long long hmax = 0;        // maximum degree (rank-sort bits)
-        int64_t nplus = 0, ntasks = 0;      // plus-array and task-array entries
         std::vector<std::pair<int64_t, int64_t>> huge;  // N+ rows sorted in global memory: (rb, len)
-        int64_t jt[3] = {0, 0, 0};          // jobs per bin
-        int32_t *bad = nullptr;             // the orientation's symmetry flag (checked after a replay)
     } plan;
     bool capturing = false;
     hipStream_t cap_stream = nullptr;
@@ -230,7 +227,10 @@ struct Graph {
 // default's staging does not fit (per-entry appends, mask by degree).  core_k
 // > 0: the owners of the core_k highest ranks get no tasks (tc_core.hip counts
 // their triangles); g.core_k says whether the layout was built so.
+// The counters g.accum are zeroed by the caller; word 27 is set where the rows
+// of an oriented layout are not symmetric.  oriented_views does both, and waits.
 int prepare_views(Graph &g, bool oriented, int32_t hub_degree = 0, int fallback = 0, int32_t core_k = 0);
+int oriented_views(Graph &g);
 // Fills vinfo with the store's rows as given (direct layout, dm=0).
 int build_direct_vinfo(Graph &g);
 // Validation of sortedness/range, self-loop count, optional symmetry check.

@@ -474,7 +474,7 @@ int collect_timings(Graph &g, int64_t max_samples, uint64_t seed, float *feat, f
         return TC_ERR_INVALID;
     }
     if (g.st.nnz == 0) return TC_OK;
-    TC_TRY(prepare_views(g, true));
+    TC_TRY(oriented_views(g));
     if (g.ntasks == 0) return TC_OK;
     hipStream_t s = g.stream;
     const int64_t ncand = 4 * max_samples;

@@ -331,8 +331,11 @@ __device__ inline void wave_rows_of2(const int64_t *__restrict__ coff,
 // crow[c] = row holding compact entry 64c.  A row holds the starts of chunks
 // ceil(a/64) .. ceil(b/64)-1 ([a, b) its entries); a row with more than 8 of
 // them is written by its whole wave.
-__global__ void k_chunk_rows(const int64_t *__restrict__ coff, int32_t nv, int32_t *__restrict__ crow)
+// (asym, optional: set where coff exceeds what crow was sized for)
+__global__ void k_chunk_rows(const int64_t *__restrict__ coff, int32_t nv, int32_t *__restrict__ crow,
+                             const int32_t *__restrict__ asym)
 {
+    if (asym && *asym) return;
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t r0 = (int64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~(kWave - 1)); r0 < nv;
@@ -520,8 +523,9 @@ __global__ void k_orient_write_plus(const int64_t *__restrict__ coff, const int3
                                     const int64_t *__restrict__ cscan,
                                     const uint64_t *__restrict__ mask,
                                     const int32_t *__restrict__ rnk, const int64_t *__restrict__ pcoff,
-                                    int32_t nv, int64_t nnz, int32_t *__restrict__ padj)
+                                    int32_t nv, int64_t nnz, int32_t *__restrict__ padj, const int32_t *__restrict__ asym)
 {
+    if (*asym) return;
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t nchunks = ceil_div(nnz, kWave);
     const int64_t wstride = (int64_t)gridDim.x * (blockDim.x / kWave);
@@ -605,8 +609,9 @@ __global__ void k_orient_write_plus_rank(const int64_t *__restrict__ coff,
                                          const int64_t *__restrict__ cscan,
                                          const uint64_t *__restrict__ mask,
                                          const int64_t *__restrict__ pdst, int32_t nv, int64_t nnz,
-                                         int32_t *__restrict__ padj)
+                                         int32_t *__restrict__ padj, const int32_t *__restrict__ asym)
 {
+    if (*asym) return;
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t nchunks = ceil_div(nnz, kWave);
     const int64_t wstride = (int64_t)gridDim.x * (blockDim.x / kWave);
@@ -667,8 +672,9 @@ __device__ inline void bitonic_regs(int32_t (&v)[N])
 __global__ void k_sort_plus_small(const VInfo *__restrict__ vi, int32_t nv,
                                   int32_t *__restrict__ padj, int32_t *__restrict__ lst,
                                   const int64_t *__restrict__ off /* [5] */,
-                                  int32_t *__restrict__ cnt /* [5] */)
+                                  int32_t *__restrict__ cnt /* [5] */, const int32_t *__restrict__ asym)
 {
+    if (*asym) return;
     const int lane = threadIdx.x & (kWave - 1);
     const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
     // whole waves iterate together so the list appends can be aggregated
@@ -718,8 +724,9 @@ __global__ void k_sort_plus_small(const VInfo *__restrict__ vi, int32_t nv,
 // N+ parts of kThreadSort+1..64 entries: one wavefront per listed row,
 // bitonic network across the lanes.
 __global__ void k_sort_plus_wave(const VInfo *__restrict__ vi, const int32_t *__restrict__ rows,
-                                 const int32_t *__restrict__ nrows, int32_t *__restrict__ padj)
+                                 const int32_t *__restrict__ nrows, int32_t *__restrict__ padj, const int32_t *__restrict__ asym)
 {
+    if (*asym) return;
     const int lane = threadIdx.x & (kWave - 1);
     const int32_t n = *nrows;
     const int64_t wstride = (int64_t)gridDim.x * (blockDim.x / kWave);
@@ -759,8 +766,9 @@ template <int CAP, int NT>
 __global__ __launch_bounds__(NT) void k_sort_plus_block(const VInfo *__restrict__ vi,
                                                         const int32_t *__restrict__ rows,
                                                         const int32_t *__restrict__ nrows,
-                                                        int32_t *__restrict__ padj)
+                                                        int32_t *__restrict__ padj, const int32_t *__restrict__ asym)
 {
+    if (*asym) return;
     constexpr int PER = CAP / NT;
     static_assert(PER * NT == CAP && (PER & (PER - 1)) == 0, "runs of a power of two");
     __shared__ int32_t S[CAP];
@@ -856,6 +864,7 @@ __global__ void k_orient_transpose(const int64_t *__restrict__ pcoff, const int3
                                    TaskRec *__restrict__ tasks, int32_t *__restrict__ cursor,
                                    unsigned long long *__restrict__ sc, int32_t *__restrict__ bad)
 {
+    if (bad[1]) return;
     // owners from rank sc[1] up are the hubs, handled by k_orient_transpose_hubs
     const int32_t hub_lo = (int32_t)sc[1];
     unsigned long long nhub = 0;
@@ -912,6 +921,7 @@ __global__ void k_orient_transpose_hubs(
     const unsigned long long *__restrict__ sc, TaskRec *__restrict__ tasks,
     int32_t *__restrict__ bad)
 {
+    if (bad[1]) return;
     const int32_t hub_lo = (int32_t)sc[1];
     if (hub_lo >= nv) return;
     const int lane = threadIdx.x & (kWave - 1);
@@ -958,9 +968,14 @@ __global__ void k_orient_transpose_hubs(
 // it take the row-built task lists, which are correct for any owner.)  One
 // thread.
 // fixed_lo >= 0 is that rank instead (the core's first).
+// Symmetric loop-free rows have half their entries in the plus array: otherwise
+// asym is set, and the kernels after this one, whose arrays are sized for that
+// half, do nothing.
 __global__ void k_hub_lo(const VInfo *__restrict__ vi, int32_t nv, int32_t min_deg, int32_t fixed_lo,
-                         unsigned long long *__restrict__ sc)
+                         const int64_t *__restrict__ pcoff, int64_t nnz, unsigned long long *__restrict__ sc,
+                         int32_t *__restrict__ asym)
 {
+    if (2 * pcoff[nv] != nnz) *asym = 1;
     int32_t lo = fixed_lo >= 0 ? fixed_lo : 0, hi = fixed_lo >= 0 ? fixed_lo : nv;
     while (lo < hi) {
         const int32_t mid = (lo + hi) >> 1;
@@ -978,6 +993,7 @@ __global__ void k_check_cursor(const int32_t *__restrict__ cursor, const VInfo *
                                const int64_t *__restrict__ toff, int32_t nv,
                                const unsigned long long *__restrict__ sc, int32_t *__restrict__ bad)
 {
+    if (bad[1]) return;
     const int32_t hub_lo = (int32_t)sc[1];
     for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < hub_lo;
          r += (int64_t)gridDim.x * blockDim.x)
@@ -1032,9 +1048,10 @@ constexpr int64_t kTpDrop = INT64_MIN;
 // holds more than kTpWin tasks, follows such an owner, or starts its list in
 // another window than the owner before it.
 __global__ void k_tp_flags(const int64_t *__restrict__ toff, const unsigned long long *__restrict__ sc,
-                           int32_t nv, int32_t *__restrict__ flag)
+                           int32_t nv, int32_t *__restrict__ flag, const int32_t *__restrict__ asym)
 {
-    const int64_t hub_lo = (int64_t)min(sc[1], (unsigned long long)nv);
+    // (no bucket at all where the rows are not symmetric)
+    const int64_t hub_lo = *asym ? 0 : (int64_t)min(sc[1], (unsigned long long)nv);
     for (int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; w < nv;
          w += (int64_t)gridDim.x * blockDim.x) {
         int32_t f = 0;
@@ -1231,6 +1248,7 @@ __global__ __launch_bounds__(kTpThreads) void k_tp_coarse(
     unsigned long long *__restrict__ sc, unsigned long long *__restrict__ ccur,
     uint64_t *__restrict__ rec_out, int32_t *__restrict__ own_out, int32_t *__restrict__ bad)
 {
+    if (bad[1]) return;
     __shared__ TpShared S;
     __shared__ int32_t end_last;
     const int t = threadIdx.x, lane = t & (kWave - 1), wid = t / kWave;
@@ -1321,6 +1339,7 @@ __global__ __launch_bounds__(kTpThreads) void k_tp_fine(
     const int32_t *__restrict__ tmap, unsigned long long *__restrict__ fcur,
     uint64_t *__restrict__ rec_out, int32_t *__restrict__ own_out, int32_t *__restrict__ bad)
 {
+    if (bad[1]) return;
     __shared__ TpShared S;
     const int t = threadIdx.x;
     const int64_t F = ctl[0], G = ctl[1], ntiles = ctl[3];
@@ -1365,6 +1384,7 @@ __global__ __launch_bounds__(kTpThreads) void k_tp_local(const int64_t *__restri
                                                          const int32_t *__restrict__ own,
                                                          int32_t *__restrict__ bad)
 {
+    if (bad[1]) return;
     __shared__ int32_t lc[kTpWin];
     __shared__ uint64_t st[kTpLocal];
     const int t = threadIdx.x;
@@ -1410,6 +1430,7 @@ __global__ void k_tp_check(const int64_t *__restrict__ toff, const int32_t *__re
                            const unsigned long long *__restrict__ fcur, int32_t nv,
                            const unsigned long long *__restrict__ sc, int32_t *__restrict__ bad)
 {
+    if (bad[1]) return;
     const int64_t F = ctl[0], G = ctl[1], K = ctl[2];
     const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -1569,8 +1590,12 @@ __global__ void k_owner_work(const int64_t *__restrict__ coff, const int32_t *__
                              const int32_t *__restrict__ adj, const TaskRec *__restrict__ tasks,
                              int32_t nv, PlanParams P,
                              unsigned long long *__restrict__ work,
+                             unsigned long long *__restrict__ wtotal,
+                             const unsigned long long *__restrict__ fault,
                              unsigned long long *__restrict__ bstats)
 {
+    if (*fault) return;  // (set by kernels before this one: the same for all)
+    unsigned long long w_all = 0;
     const int64_t nnz = coff[P.owner_end];  // (owners from owner_end up have no jobs)
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t nchunks = ceil_div(nnz, kWave);
@@ -1610,6 +1635,7 @@ __global__ void k_owner_work(const int64_t *__restrict__ coff, const int32_t *__
                 }
             }
         }
+        w_all += w;
         // segmented (by owner row) inclusive scan of w across the wave; a
         // chunk's sum fits 32 bits (each item estimate is below 2^25)
         uint32_t x = w;
@@ -1637,6 +1663,8 @@ __global__ void k_owner_work(const int64_t *__restrict__ coff, const int32_t *__
         chunk(c, b, tl);
         if (two) chunk(c2, b2, tl2);
     }
+    const unsigned long long wpart[1] = {w_all};
+    block_add_u64<1>(wpart, wtotal);
     if (bstats) {
         // bstats layout: tasks/bytes pairs per bin, then items per bin
         const unsigned long long v[9] = {st_t[0], st_b[0], st_t[1], st_b[1], st_t[2],
@@ -1645,87 +1673,124 @@ __global__ void k_owner_work(const int64_t *__restrict__ coff, const int32_t *__
     }
 }
 
-// Jobs per owner and bin; jstats[b] (optional) gets the owner-tile entries
-// the jobs of bin b load.
+// The jobs of every bin, in arrays of their own: jc[b] (zero on entry) receives
+// their number, jstats[b] (optional) the owner-tile entries they load.  A block
+// plans kPlanOwners owners and reserves their jobs with one atomic per bin, so
+// neighbouring owners' jobs stay together and nothing is scanned over all
+// owners or read back.  *wtotal (the work of all owners) raises the grain where
+// the jobs would outgrow their arrays: at most 2^21 beyond one per owner and
+// tile.  *fault (the rows turned out not to be symmetric): no jobs.
+constexpr int kPlanThreads = 1024, kPlanPer = 4, kPlanOwners = kPlanThreads * kPlanPer;
+struct JobArrays {
+    Job *j[3];
+    int64_t cap[3];
+};
 template <bool ORIENTED>
-__global__ void k_plan_jobs(const VInfo *__restrict__ vi, const unsigned long long *__restrict__ work,
-                            int32_t nv, PlanParams P, int32_t *__restrict__ njobs /* [3][nv] */,
-                            unsigned long long *__restrict__ jstats)
+__global__ __launch_bounds__(kPlanThreads) void k_plan_jobs(
+    const VInfo *__restrict__ vi, const unsigned long long *__restrict__ work, int32_t nv, PlanParams P,
+    const unsigned long long *__restrict__ wtotal, const unsigned long long *__restrict__ fault, JobArrays J,
+    unsigned long long *__restrict__ jc, unsigned long long *__restrict__ jstats)
 {
-    const int lane = threadIdx.x & (kWave - 1);
+    __shared__ int32_t wsum[3][kPlanThreads / kWave];
+    __shared__ unsigned long long base[3];
+    if (*fault) return;  // (set by kernels before this one: the same for all)
+    const int t = threadIdx.x, lane = t & (kWave - 1), wid = t / kWave;
+    const int64_t wmin = (int64_t)(*wtotal >> 20);
+    const int64_t v0 = (int64_t)blockIdx.x * kPlanOwners + (int64_t)t * kPlanPer;
+    int32_t nj[kPlanPer], split[kPlanPer], T[kPlanPer], cnt[3] = {0, 0, 0};
+    int bin[kPlanPer];
     unsigned long long tile_items[3] = {0, 0, 0};
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t v0 = (int64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~(kWave - 1)); v0 < nv;
-         v0 += stride) {
-        const int64_t v = v0 + lane;
-        if (v >= nv) continue;
-        VInfo x = vi[v];
-        int32_t L = ORIENTED ? x.len - x.dm : x.len;
-        int32_t T = ORIENTED ? x.dm : x.len;
-        int32_t nj[3] = {0, 0, 0};
-        unsigned long long w = work[v];
-        if (L > 0 && T > 0 && w > 0 && v < P.owner_end && (ORIENTED || x.len >= 2)) {
-            int bin = owner_bin(L, P);
-            int64_t tiles = owner_tiles(L, bin, P);
-            int64_t per_tile = (int64_t)(w / (unsigned long long)tiles) + 1;
-            // a job amortises building its LDS table over at least 16 items per slot
-            // Each job ends by flushing up to one global atomic per owner slot,
-            // so a job gets at least flush_items items per slot.
-            int64_t grain = max<int64_t>((int64_t)P.job_items * P.nw[bin],
-                                         (int64_t)P.flush_items * min(L, P.lmax[bin]));
-            int64_t split = ceil_div(per_tile, grain);
-            if (split > T) split = T;
-            if (split < 1) split = 1;
-            nj[bin] = (int32_t)(split * tiles);
 #pragma unroll
-            for (int q = 0; q < 3; ++q)
-                if (q == bin) tile_items[q] += (unsigned long long)split * (unsigned long long)L;
+    for (int k = 0; k < kPlanPer; ++k) {
+        const int64_t v = v0 + k;
+        nj[k] = split[k] = T[k] = 0;
+        bin[k] = 0;
+        if (v >= nv || v >= P.owner_end) continue;
+        const VInfo x = vi[v];
+        const unsigned long long w = work[v];
+        const int32_t L = ORIENTED ? x.len - x.dm : x.len;
+        T[k] = ORIENTED ? x.dm : x.len;
+        if (L <= 0 || T[k] <= 0 || w == 0 || (!ORIENTED && x.len < 2)) continue;
+        bin[k] = owner_bin(L, P);
+        const int64_t tiles = owner_tiles(L, bin[k], P);
+        const int64_t per_tile = (int64_t)(w / (unsigned long long)tiles) + 1;
+        // a job amortises building its LDS table and, at its end, the flush of
+        // up to one global atomic per owner slot: at least flush_items items
+        // per slot
+        const int64_t grain = max(max((int64_t)P.job_items * P.nw[bin[k]],
+                                      (int64_t)P.flush_items * min(L, P.lmax[bin[k]])), wmin);
+        int64_t sp = ceil_div(per_tile, grain);
+        if (sp > T[k]) sp = T[k];
+        if (sp < 1) sp = 1;
+        split[k] = (int32_t)sp;
+        nj[k] = (int32_t)(sp * tiles);
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+            if (q == bin[k]) {
+                cnt[q] += nj[k];
+                tile_items[q] += (unsigned long long)sp * (unsigned long long)L;
+            }
+    }
+    int32_t incl[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        incl[q] = wave_incl_scan_i32(cnt[q]);
+        if (lane == kWave - 1) wsum[q][wid] = incl[q];
+    }
+    __syncthreads();
+    int32_t before[3] = {0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        int32_t all = 0;
+        for (int w = 0; w < kPlanThreads / kWave; ++w) {
+            before[q] += w < wid ? wsum[q][w] : 0;
+            all += wsum[q][w];
         }
-        njobs[v] = nj[0];
-        njobs[(int64_t)nv + v] = nj[1];
-        njobs[2 * (int64_t)nv + v] = nj[2];
+        if (t == 0) base[q] = all ? atomicAdd(&jc[q], (unsigned long long)all) : 0ull;
+    }
+    __syncthreads();
+    int64_t at[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) at[q] = (int64_t)base[q] + before[q] + incl[q] - cnt[q];
+    auto put = [&](int b, int64_t p, int64_t v, int32_t tasks, int32_t sp, int32_t q) {
+        Job j;
+        const int32_t tile = q / sp, i = q - tile * sp;
+        j.owner = (int32_t)v;
+        j.t_begin = (int32_t)(((int64_t)tasks * i) / sp);
+        j.t_end = (int32_t)(((int64_t)tasks * (i + 1)) / sp);
+        j.tile = tile;
+        Job *out = b == 0 ? J.j[0] : (b == 1 ? J.j[1] : J.j[2]);
+        const int64_t cap = b == 0 ? J.cap[0] : (b == 1 ? J.cap[1] : J.cap[2]);
+        if (p < cap) out[p] = j;
+    };
+#pragma unroll
+    for (int k = 0; k < kPlanPer; ++k) {
+        const int64_t p = bin[k] == 0 ? at[0] : (bin[k] == 1 ? at[1] : at[2]);
+        // an owner of many jobs is written by its whole wave
+        const bool wide = nj[k] > 8;
+        if (!wide)
+            for (int32_t q = 0; q < nj[k]; ++q) put(bin[k], p + q, v0 + k, T[k], split[k], q);
+        for (uint64_t wm = __ballot(wide); wm; wm &= wm - 1) {
+            const int l = __ffsll((unsigned long long)wm) - 1;
+            const int64_t lp = readlane_i64(p, l), lv = readlane_i64(v0 + k, l);
+            const int32_t lt = __builtin_amdgcn_readlane(T[k], l), ls = __builtin_amdgcn_readlane(split[k], l);
+            const int32_t ln = __builtin_amdgcn_readlane(nj[k], l), lb = __builtin_amdgcn_readlane(bin[k], l);
+            for (int32_t q = lane; q < ln; q += kWave) put(lb, lp + q, lv, lt, ls, q);
+        }
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+            if (q == bin[k]) at[q] += nj[k];
     }
     if (jstats) block_add_u64<3>(tile_items, jstats);
-}
-
-template <bool ORIENTED>
-__global__ void k_emit_jobs(const VInfo *__restrict__ vi, const int32_t *__restrict__ njobs,
-                            const int64_t *__restrict__ jscan /* [3][nv+1] */, int32_t nv,
-                            PlanParams P, Job *__restrict__ jobs0, Job *__restrict__ jobs1,
-                            Job *__restrict__ jobs2)
-{
-    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nv;
-         v += (int64_t)gridDim.x * blockDim.x) {
-        VInfo x = vi[v];
-        int32_t L = ORIENTED ? x.len - x.dm : x.len;
-        int32_t T = ORIENTED ? x.dm : x.len;
-        for (int bin = 0; bin < 3; ++bin) {
-            int32_t nj = njobs[(int64_t)bin * nv + v];
-            if (!nj) continue;
-            Job *out = bin == 0 ? jobs0 : (bin == 1 ? jobs1 : jobs2);
-            int64_t base = jscan[(int64_t)bin * (nv + 1) + v];
-            int32_t tiles = owner_tiles(L, bin, P);
-            int32_t split = nj / tiles;
-            int64_t q = 0;
-            for (int32_t t = 0; t < tiles; ++t)
-                for (int32_t s = 0; s < split; ++s) {
-                    Job j;
-                    j.owner = (int32_t)v;
-                    j.t_begin = (int32_t)(((int64_t)T * s) / split);
-                    j.t_end = (int32_t)(((int64_t)T * (s + 1)) / split);
-                    j.tile = t;
-                    out[base + q++] = j;
-                }
-        }
-    }
 }
 
 // outr[r] += 2 * (sum of pcnt over N+(r)): the task-vertex share of the
 // oriented count, one segmented wave sum per 64 entries of the plus array.
 __global__ void k_plus_row_sum(const int64_t *__restrict__ pcoff, const int32_t *__restrict__ pcrow,
                                const uint32_t *__restrict__ pcnt, int32_t nv, int64_t nplus,
-                               uint32_t *__restrict__ outr)
+                               uint32_t *__restrict__ outr, const int32_t *__restrict__ asym)
 {
+    if (*asym) return;
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t nchunks = ceil_div(nplus, kWave);
     const int64_t wstride = (int64_t)gridDim.x * (blockDim.x / kWave);
@@ -2048,12 +2113,13 @@ template <int LMAX, int NW, int MODE>
 #ifndef TC_SMALL_WAVES
 #define TC_SMALL_WAVES 7
 #endif
-__global__ __launch_bounds__(NW * kWave, LMAX <= 64 ? TC_SMALL_WAVES : LMAX <= 512 ? TC_MID_WAVES : 1) void k_count(const Job *__restrict__ jobs, int64_t njobs,
+__global__ __launch_bounds__(NW * kWave, LMAX <= 64 ? TC_SMALL_WAVES : LMAX <= 512 ? TC_MID_WAVES : 1) void k_count(const Job *__restrict__ jobs, const unsigned long long *__restrict__ njobs_dev,
                                                       CountArgs A)
 {
     // MODE: kDirect (tasks are the owner's row entries), kOriented, kByTasks
     // (direct counts by the larger row, see k_direct_tasks)
     constexpr bool ORIENTED = MODE == kOriented, TASKS = MODE != kDirect;
+    const int64_t njobs = (int64_t)*njobs_dev;
     // The owner tile lives in a bucketed two-choice hash table (BucketTableT),
     // load <= 1/2, so a lookup reads one bucket, a second only where the
     // first is full, and loops only when both are.  C counts hits per slot
@@ -2505,8 +2571,10 @@ constexpr int kLongUnroll = TC_LONG_UNROLL;
 
 template <int LMAX, int NW, bool BM>
 __global__ __launch_bounds__(NW * kWave, BM ? 6 : 4) void k_count_long(const Job *__restrict__ jobs,
-                                                           int64_t njobs, CountArgs A)
+                                                           const unsigned long long *__restrict__ njobs_dev,
+                                                           CountArgs A)
 {
+    const int64_t njobs = (int64_t)*njobs_dev;
     constexpr int NBMAX = LMAX / 2;
     constexpr int kBmWords = 2 * NBMAX;  // uint2 words in HB's space
     // one LDS block: the table (or bitmap) HB, then the counters C.  The
@@ -2718,9 +2786,11 @@ __device__ inline int32_t row_lower(const int32_t *__restrict__ row, int32_t n, 
 }
 
 template <int WORDS, int NT>
-__global__ __launch_bounds__(NT, NT == 512 ? 6 : 4) void k_direct_bits(const Job *__restrict__ jobs, int64_t njobs,
+__global__ __launch_bounds__(NT, NT == 512 ? 6 : 4) void k_direct_bits(const Job *__restrict__ jobs,
+                                                                     const unsigned long long *__restrict__ njobs_dev,
                                                                      CountArgs A)
 {
+    const int64_t njobs = (int64_t)*njobs_dev;
     constexpr int U = 8, NW = NT / kWave;
     __shared__ uint32_t bits[WORDS + 1];  // (one word past the span: the zero guard word)
     __shared__ int64_t s_job;
@@ -2839,30 +2909,31 @@ constexpr int kNW0 = 1, kNW1 = TC_MID_NW, kNW2 = 8;
 // and 128 KB, one block of 16
 constexpr int kBitsIds0 = 1 << 18, kBitsIds1 = 1 << 20;
 
+// most bounds the bin's jobs, whose number is on the device.
 // ev_long (bin 2, oriented): events recorded before and after the bitmap-tile
 // launch of k_count_long and after its hash-table-tile launch.
-int launch_bin(int bin, int mode, const Job *jobs, int64_t njobs, const CountArgs &A,
-               hipStream_t s, hipEvent_t *ev_long)
+int launch_bin(int bin, int mode, const Job *jobs, int64_t most, const unsigned long long *njobs,
+               const CountArgs &A, hipStream_t s, hipEvent_t *ev_long)
 {
     const bool oriented = mode == kOriented;
-    if (njobs <= 0) return TC_OK;
+    if (most <= 0) return TC_OK;
     int dev = 0;
     TC_HIP(hipGetDevice(&dev));
     int cus = 0;
     TC_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     // persistent grid: enough resident blocks to fill every CU
     int per_cu = bin == 0 ? 4 * TC_SMALL_WAVES / kNW0 : (bin == 1 ? 4 * TC_MID_WAVES / kNW1 : 2);
-    int64_t grid = std::min<int64_t>(njobs, (int64_t)cus * per_cu);
+    int64_t grid = std::min<int64_t>(most, (int64_t)cus * per_cu);
     if (mode == kByTasks) {
         if (bin == 0)
             hipLaunchKernelGGL((k_count<kL0, kNW0, kByTasks>), dim3((unsigned)grid), dim3(kNW0 * kWave), 0, s, jobs, njobs, A);
         else if (bin == 1)
             hipLaunchKernelGGL((k_count<kL1, kNW1, kByTasks>), dim3((unsigned)grid), dim3(kNW1 * kWave), 0, s, jobs, njobs, A);
         else if (A.nv <= kBitsIds0)
-            hipLaunchKernelGGL((k_direct_bits<kBitsIds0 / 32, 512>), dim3((unsigned)std::min<int64_t>(njobs, cus * 3)),
+            hipLaunchKernelGGL((k_direct_bits<kBitsIds0 / 32, 512>), dim3((unsigned)std::min<int64_t>(most, cus * 3)),
                                dim3(512), 0, s, jobs, njobs, A);
         else
-            hipLaunchKernelGGL((k_direct_bits<kBitsIds1 / 32, 1024>), dim3((unsigned)std::min<int64_t>(njobs, cus)),
+            hipLaunchKernelGGL((k_direct_bits<kBitsIds1 / 32, 1024>), dim3((unsigned)std::min<int64_t>(most, cus)),
                                dim3(1024), 0, s, jobs, njobs, A);
     } else if (bin == 0) {
         if (oriented)
@@ -2889,8 +2960,8 @@ int launch_bin(int bin, int mode, const Job *jobs, int64_t njobs, const CountArg
                                 A.policy == TC_POLICY_MERGEPATH;
             if (forced)
                 hipLaunchKernelGGL((k_count<kL2, kNW2, kOriented>), dim3((unsigned)grid), dim3(kNW2 * kWave), 0, s, jobs, njobs, As);
-            const int64_t gb = std::min<int64_t>(njobs, (int64_t)cus * 3);
-            const int64_t gh = std::min<int64_t>(njobs, (int64_t)cus * 2);
+            const int64_t gb = std::min<int64_t>(most, (int64_t)cus * 3);
+            const int64_t gh = std::min<int64_t>(most, (int64_t)cus * 2);
             if (ev_long) TC_HIP(hipEventRecord(ev_long[0], s));
             if (!forced)
                 hipLaunchKernelGGL((k_count_long<kL2, kNW2, true>), dim3((unsigned)gb), dim3(kNW2 * kWave), 0, s, jobs, njobs, Al);
@@ -2934,10 +3005,17 @@ int prepare_views(Graph &g, bool oriented, int32_t hub_degree, int fallback, int
         TC_TRY(scan_counts_i32(g.st.len.as<int32_t>(), coff, nv, g.tmp, s));
         TC_TRY(g.crow.ensure((size_t)(nchunks + 1) * sizeof(int32_t)));
         hipLaunchKernelGGL(k_chunk_rows, dim3(vblocks), dim3(256), 0, s, coff, nv,
-                           g.crow.as<int32_t>());
+                           g.crow.as<int32_t>(), (const int32_t *)nullptr);
         TC_HIP(hipGetLastError());
         return build_direct_vinfo(g);
     }
+
+    // Symmetric loop-free rows put half their entries into the plus array and
+    // the other half into the task array; nothing is read back on the way, and
+    // acc[27] tells in the end whether the rows were so (its halves: any fault,
+    // and one seen before the arrays are written).
+    const int64_t nplus = nnz / 2, ntasks = nnz / 2;
+    int32_t *bad = reinterpret_cast<int32_t *>(g.accum.as<unsigned long long>() + 27), *asym = bad + 1;
 
     // ---- store-order offsets and chunk rows
     TC_TRY(g.ov[0].ensure((size_t)(nv + 1) * sizeof(int64_t)));      // store-order offsets
@@ -2945,7 +3023,8 @@ int prepare_views(Graph &g, bool oriented, int32_t hub_degree, int fallback, int
     int64_t *ocoff = g.ov[0].as<int64_t>();
     int32_t *ocrow = g.ov[1].as<int32_t>();
     TC_TRY(scan_counts_i32(g.st.len.as<int32_t>(), ocoff, nv, g.tmp, s));
-    hipLaunchKernelGGL(k_chunk_rows, dim3(vblocks), dim3(256), 0, s, ocoff, nv, ocrow);
+    hipLaunchKernelGGL(k_chunk_rows, dim3(vblocks), dim3(256), 0, s, ocoff, nv, ocrow,
+                       (const int32_t *)nullptr);
     // ---- rank order: stable sort of the degrees
     TC_TRY(g.order.ensure((size_t)nv * sizeof(int32_t)));
     TC_TRY(g.rnk.ensure((size_t)nv * sizeof(int32_t)));
@@ -2961,12 +3040,16 @@ int prepare_views(Graph &g, bool oriented, int32_t hub_degree, int fallback, int
     hipLaunchKernelGGL(k_rank_keys, dim3(grid_for(nv, 256, 1024)), dim3(256), 0, s,
                        g.st.len.as<int32_t>(), nv, keys, order, sc);
     TC_HIP(hipGetLastError());
-    // sort only the bits the current maximum degree needs (one pass per 8)
-    unsigned long long hmax = g.plan.hmax;
-    if (!g.capturing) {
-        TC_HIP(hipMemcpyAsync(&hmax, sc, sizeof(hmax), hipMemcpyDeviceToHost, s));
-        TC_HIP(hipStreamSynchronize(s));
-        g.plan.hmax = hmax;
+    // sort only the bits the maximum degree needs (one pass per 8); it is read
+    // back where an update has left it unknown
+    unsigned long long hmax = (unsigned long long)g.max_degree;
+    if (!g.validated || g.degree_stale) {
+        hmax = g.plan.hmax;
+        if (!g.capturing) {
+            TC_HIP(hipMemcpyAsync(&hmax, sc, sizeof(hmax), hipMemcpyDeviceToHost, s));
+            TC_HIP(hipStreamSynchronize(s));
+            g.plan.hmax = hmax;
+        }
     }
     int kbits = std::max(1, ceil_log2_i((int64_t)hmax + 1));
     if (g.batch_voff && g.batch_ngraphs > 1) {
@@ -3036,15 +3119,33 @@ int prepare_views(Graph &g, bool oriented, int32_t hub_degree, int fallback, int
     VInfo *vi = g.vinfo.as<VInfo>();
     hipLaunchKernelGGL(k_rank_vinfo, dim3(vblocks), dim3(256), 0, s, pcoff, dpr, dmr, nv, vi);
     TC_HIP(hipGetLastError());
-    int64_t tot[2] = {g.plan.nplus, g.plan.ntasks};
-    if (!g.capturing) {
-        TC_HIP(hipMemcpyAsync(&tot[0], pcoff + nv, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-        TC_HIP(hipMemcpyAsync(&tot[1], toff + nv, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-        TC_HIP(hipStreamSynchronize(s));
-        g.plan.nplus = tot[0];
-        g.plan.ntasks = tot[1];
+    // the partitioned transpose's bound on its fine buckets (window starts,
+    // owners of more than a window and the owners after them) and its
+    // staging (16 bytes per task); the appends when either does not fit
+    const int64_t fmax = std::min<int64_t>(nv, 3 * (ntasks / kTpWin) + 1) + 1;
+    bool part = !fallback && nplus > 0 && fmax <= (int64_t)kTpMaxB * kTpMaxB;
+    if (part) {
+        const int64_t tmax = ceil_div(ntasks, kTpTile) + kTpMaxB;  // pass-2 tiles, at most
+        const size_t meta =
+            (size_t)(4 + kTpMaxB + fmax) * 8 + (size_t)(fmax + 1 + kTpMaxB + 1 + tmax) * 4;
+        part = g.ov[13].ensure((size_t)(nv + 1) * sizeof(int64_t)) == TC_OK &&
+               g.ov[14].ensure(meta) == TC_OK &&
+               g.ov[15].ensure((size_t)ntasks * sizeof(uint64_t)) == TC_OK &&
+               g.ov[16].ensure((size_t)ntasks * sizeof(int32_t)) == TC_OK &&
+               g.ov[17].ensure((size_t)ntasks * sizeof(int32_t)) == TC_OK;
+        if (!part)  // out of memory for the staging: free it again
+            for (int q = 13; q < 18; ++q) g.ov[q].release();
     }
-    const int64_t nplus = tot[0], ntasks = tot[1];
+    // the core's owners get no tasks (the split leaves out entries from rank
+    // sc[1] up, as with hubs)
+    if (part) g.core_k = core_k;
+    // hubs: owners whose task lists are built from their rows (the appends
+    // would serialise on their cursors; the partitioned transpose has no
+    // per-owner atomics and needs no hubs unless the schedule asks)
+    hipLaunchKernelGGL(k_hub_lo, dim3(1), dim3(1), 0, s, vi, nv,
+                       hub_degree > 0 ? hub_degree : part ? INT32_MAX : kHubDegree,
+                       g.core_k > 0 ? nv - g.core_k : -1, pcoff, nnz, sc, asym);
+    TC_HIP(hipGetLastError());
     TC_TRY(g.padj.ensure((size_t)std::max<int64_t>(nplus, 1) * sizeof(int32_t)));
     TC_TRY(g.tasks.ensure((size_t)std::max<int64_t>(ntasks, 1) * sizeof(TaskRec)));
     int32_t *padj = g.padj.as<int32_t>();
@@ -3053,11 +3154,11 @@ int prepare_views(Graph &g, bool oriented, int32_t hub_degree, int fallback, int
         hipLaunchKernelGGL(k_plus_dst, dim3(vblocks), dim3(256), 0, s, ocoff, cscan, mask, rnk, pcoff,
                            nv, pdst);
         hipLaunchKernelGGL(k_orient_write_plus_rank, dim3(wblocks), dim3(256), 0, s, ocoff, ocrow, tr,
-                           cscan, mask, pdst, nv, nnz, padj);
+                           cscan, mask, pdst, nv, nnz, padj, asym);
     } else
         hipLaunchKernelGGL(k_orient_write_plus, dim3(wblocks), dim3(256), 0, s, ocoff, ocrow,
                            g.st.boff.as<int64_t>(), g.st.pool.as<int32_t>(), cscan, mask, rnk, pcoff,
-                           nv, nnz, padj);
+                           nv, nnz, padj, asym);
     TC_HIP(hipGetLastError());
 
     // ---- sort every N+ part by rank
@@ -3083,21 +3184,25 @@ int prepare_views(Graph &g, bool oriented, int32_t hub_degree, int fallback, int
                        ListOffsets{{hoff[0], hoff[1], hoff[2], hoff[3], hoff[4]}},
                        reinterpret_cast<uint32_t *>(lcnt));
     hipLaunchKernelGGL(k_sort_plus_small, dim3(vblocks), dim3(256), 0, s, vi, nv, padj, lst, loff,
-                       lcnt);
+                       lcnt, asym);
     TC_HIP(hipGetLastError());
     int dev = 0, cus = 0;
     TC_HIP(hipGetDevice(&dev));
     TC_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     hipLaunchKernelGGL(k_sort_plus_wave, dim3(cus * 8), dim3(256), 0, s, vi, lst + hoff[0], lcnt + 0,
-                       padj);
+                       padj, asym);
     hipLaunchKernelGGL((k_sort_plus_block<512, 64>), dim3(cus * TC_SORT512_BLOCKS), dim3(64), 0, s,
-                       vi, lst + hoff[1], lcnt + 1, padj);
+                       vi, lst + hoff[1], lcnt + 1, padj, asym);
     hipLaunchKernelGGL((k_sort_plus_block<4096, 256>), dim3(cus * TC_SORT4096_BLOCKS), dim3(256), 0, s,
-                       vi, lst + hoff[2], lcnt + 2, padj);
+                       vi, lst + hoff[2], lcnt + 2, padj, asym);
     hipLaunchKernelGGL((k_sort_plus_block<16384, 1024>), dim3(cus), dim3(1024), 0, s, vi,
-                       lst + hoff[3], lcnt + 3, padj);
+                       lst + hoff[3], lcnt + 3, padj, asym);
     TC_HIP(hipGetLastError());
-    if (!g.capturing) {
+    // (a row of N+ has at most as many entries as its square root of nnz: none
+    // can be so long in a smaller graph)
+    if (nnz < int64_t(16384) * 16384) {
+        g.plan.huge.clear();
+    } else if (!g.capturing) {
         int32_t nhuge = 0;
         TC_HIP(hipMemcpyAsync(&nhuge, lcnt + 4, sizeof(int32_t), hipMemcpyDeviceToHost, s));
         TC_HIP(hipStreamSynchronize(s));
@@ -3132,38 +3237,11 @@ int prepare_views(Graph &g, bool oriented, int32_t hub_degree, int fallback, int
     const int64_t pchunks = ceil_div(nplus, kWave), tchunks = ceil_div(ntasks, kWave);
     TC_TRY(g.ov[10].ensure((size_t)(pchunks + 1) * sizeof(int32_t)));
     int32_t *pcrow = g.ov[10].as<int32_t>();
-    hipLaunchKernelGGL(k_chunk_rows, dim3(vblocks), dim3(256), 0, s, pcoff, nv, pcrow);
+    hipLaunchKernelGGL(k_chunk_rows, dim3(vblocks), dim3(256), 0, s, pcoff, nv, pcrow, asym);
     TC_TRY(g.crow.ensure((size_t)(tchunks + 1) * sizeof(int32_t)));
-    hipLaunchKernelGGL(k_chunk_rows, dim3(vblocks), dim3(256), 0, s, toff, nv, g.crow.as<int32_t>());
+    hipLaunchKernelGGL(k_chunk_rows, dim3(vblocks), dim3(256), 0, s, toff, nv, g.crow.as<int32_t>(),
+                       asym);
     int32_t *cursor = dmo;  // store-order |N-| is not needed any more
-    int32_t *bad = lcnt + 5;
-    // the partitioned transpose's bound on its fine buckets (window starts,
-    // owners of more than a window and the owners after them) and its
-    // staging (16 bytes per task); the appends when either does not fit
-    const int64_t fmax = std::min<int64_t>(nv, 3 * (ntasks / kTpWin) + 1) + 1;
-    bool part = !fallback && nplus > 0 && fmax <= (int64_t)kTpMaxB * kTpMaxB;
-    if (part) {
-        const int64_t tmax = ceil_div(ntasks, kTpTile) + kTpMaxB;  // pass-2 tiles, at most
-        const size_t meta =
-            (size_t)(4 + kTpMaxB + fmax) * 8 + (size_t)(fmax + 1 + kTpMaxB + 1 + tmax) * 4;
-        part = g.ov[13].ensure((size_t)(nv + 1) * sizeof(int64_t)) == TC_OK &&
-               g.ov[14].ensure(meta) == TC_OK &&
-               g.ov[15].ensure((size_t)ntasks * sizeof(uint64_t)) == TC_OK &&
-               g.ov[16].ensure((size_t)ntasks * sizeof(int32_t)) == TC_OK &&
-               g.ov[17].ensure((size_t)ntasks * sizeof(int32_t)) == TC_OK;
-        if (!part)  // out of memory for the staging: free it again
-            for (int q = 13; q < 18; ++q) g.ov[q].release();
-    }
-    // the core's owners get no tasks (the split leaves out entries from rank
-    // sc[1] up, as with hubs)
-    if (part) g.core_k = core_k;
-    // hubs: owners whose task lists are built from their rows (the appends
-    // would serialise on their cursors; the partitioned transpose has no
-    // per-owner atomics and needs no hubs unless the schedule asks)
-    hipLaunchKernelGGL(k_hub_lo, dim3(1), dim3(1), 0, s, vi, nv,
-                       hub_degree > 0 ? hub_degree : part ? INT32_MAX : kHubDegree,
-                       g.core_k > 0 ? nv - g.core_k : -1, sc);
-    TC_HIP(hipGetLastError());
     if (part) {
         int64_t *fpos = g.ov[13].as<int64_t>();
         int64_t *ctl = g.ov[14].as<int64_t>();
@@ -3176,7 +3254,7 @@ int prepare_views(Graph &g, bool oriented, int32_t hub_degree, int fallback, int
         int32_t *own1 = g.ov[16].as<int32_t>(), *own2 = g.ov[17].as<int32_t>();
         uint64_t *tasks = reinterpret_cast<uint64_t *>(g.tasks.as<TaskRec>());
         int32_t *flag = cursor;
-        hipLaunchKernelGGL(k_tp_flags, dim3(vblocks), dim3(256), 0, s, toff, sc, nv, flag);
+        hipLaunchKernelGGL(k_tp_flags, dim3(vblocks), dim3(256), 0, s, toff, sc, nv, flag, asym);
         TC_TRY(scan_counts_i32(flag, fpos, nv, g.tmp, s));
         hipLaunchKernelGGL(k_tp_bounds, dim3(vblocks), dim3(256), 0, s, flag, fpos, sc, nv, fb);
         hipLaunchKernelGGL(k_tp_plan, dim3(1), dim3(1024), 0, s, fpos, nv, fb, toff, ctl, tiles, ccur);
@@ -3210,20 +3288,27 @@ int prepare_views(Graph &g, bool oriented, int32_t hub_degree, int fallback, int
                            bad);
     }
     TC_HIP(hipGetLastError());
-    g.plan.bad = bad;
-    int32_t hbad = 0;
-    if (!g.capturing) {  // a recorded count checks the flag after its replay
-        TC_HIP(hipMemcpyAsync(&hbad, bad, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-        TC_HIP(hipStreamSynchronize(s));
-    }
-    if (hbad) {
-        g.symmetric = 0;
-        set_last_error(TC_ERR_INVALID, "oriented layout: the rows are not symmetric");
-        return TC_ERR_INVALID;
-    }
     g.ntasks = ntasks;
     g.nplus = nplus;
     g.oriented_views = true;
+    return TC_OK;
+}
+
+int oriented_views(Graph &g)
+{
+    TC_TRY(g.accum.ensure(32 * sizeof(unsigned long long)));
+    unsigned long long *acc = g.accum.as<unsigned long long>();
+    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, g.stream, acc, (int64_t)32);
+    TC_TRY(prepare_views(g, true));
+    unsigned long long fault = 0;
+    TC_HIP(hipMemcpyAsync(&fault, acc + 27, sizeof(fault), hipMemcpyDeviceToHost, g.stream));
+    TC_HIP(hipStreamSynchronize(g.stream));
+    if (fault) {
+        g.symmetric = 0;
+        g.oriented_views = false;
+        set_last_error(TC_ERR_INVALID, "oriented layout: the rows are not symmetric");
+        return TC_ERR_INVALID;
+    }
     return TC_OK;
 }
 
@@ -3271,16 +3356,18 @@ int prepare_direct_tasks(Graph &g, bool skip_lower)
     TC_TRY(scan_counts_i32(tcnt, toff, nv, g.tmp, s));
     hipLaunchKernelGGL(k_direct_tasks<true>, dim3(wblocks), dim3(256), 0, s, coff, crow, boff, len, pool, nv, nnz,
                        skip_lower ? 1 : 0, cnt, mask, toff, g.tasks.as<TaskRec>(), g.ov[16].as<int32_t>());
-    hipLaunchKernelGGL(k_chunk_rows, dim3(vblocks), dim3(256), 0, s, toff, nv, g.ov[10].as<int32_t>());
+    hipLaunchKernelGGL(k_chunk_rows, dim3(vblocks), dim3(256), 0, s, toff, nv, g.ov[10].as<int32_t>(),
+                       (const int32_t *)nullptr);
     TC_HIP(hipGetLastError());
     return TC_OK;
 }
 
 // The per-bin counters of a count (accum words, see count_pass) into stats.
-void fill_counters(tc_stats &st, const unsigned long long *hacc, const int64_t *jt, bool oriented)
+void fill_counters(tc_stats &st, const unsigned long long *hacc, bool oriented)
 {
+    const unsigned long long *jt = hacc + 28;
     for (int b = 0; b < 3; ++b) {
-        st.jobs_bin[b] = jt[b];
+        st.jobs_bin[b] = (int64_t)jt[b];
         st.tasks_bin[b] = (int64_t)hacc[4 + 2 * b];
         st.bytes_alg_bin[b] = (double)hacc[5 + 2 * b];
         st.items_bin[b] = (double)hacc[10 + b];
@@ -3331,7 +3418,8 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     // scratch: accum[0] = global, [1..3] = strategy counts, [4..9] bin tasks
     // and bytes, [10..12] items, [13..15] tile items, [16..21] long-task stats,
     // [22..24] job counters of the largest bin's two launches, [25] merge-path
-    // tasks
+    // tasks, [26] estimated work, [27] faults of the rows' symmetry, [28..30]
+    // jobs per bin
     TC_TRY(g.accum.ensure(32 * sizeof(unsigned long long)));
     unsigned long long *acc = g.accum.as<unsigned long long>();
     const bool rows = nnz > 0 && rows_eligible(g, sched);
@@ -3366,11 +3454,9 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
         int32_t *bad = reinterpret_cast<int32_t *>(acc + 27);
         TC_TRY((rows ? rows_count : dense_count)(g, outp, acc, bad, oriented, skip_lower, g.capturing ? nullptr : g.ev[2]));
         g.plan.method = method;
-        g.plan.bad = bad;
-        for (int64_t &j : g.plan.jt) j = 0;
         if (g.capturing) return TC_OK;
         TC_HIP(hipEventRecord(g.ev[7], s));
-        TC_HIP(hipMemcpyAsync(g.hcounts, acc, 28 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+        TC_HIP(hipMemcpyAsync(g.hcounts, acc, 32 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
         TC_HIP(hipStreamSynchronize(s));
         const int32_t hbad = (int32_t)(uint32_t)g.hcounts[27];
         if (oriented && hbad) {  // rows declared symmetric that are not
@@ -3385,7 +3471,7 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
         if (global) *global = g.hcounts[0];
         if (stats) {
             st.method_used = method;
-            fill_counters(st, g.hcounts, g.plan.jt, oriented);
+            fill_counters(st, g.hcounts, oriented);
             float ms = 0;
             (void)hipEventElapsedTime(&ms, g.ev[0], g.ev[7]);
             st.ms_total = ms;
@@ -3399,16 +3485,9 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     }
 
     // compact offsets, chunk rows and the (degree-partitioned) vertex views;
-    // rows declared symmetric that turn out not to be go the direct way
-    if (oriented) {
-        const int pv = prepare_views(g, true, sched.hub_degree, sched.build, core_size(g, sched));
-        if (pv == TC_ERR_INVALID && sched.method == TC_METHOD_AUTO && !g.symmetric) {
-            oriented = false;
-            method = TC_METHOD_DIRECT;
-        } else if (pv != TC_OK) {
-            return pv;
-        }
-    }
+    // rows declared symmetric that turn out not to be go the direct way, after
+    // a count that finds no jobs
+    if (oriented) TC_TRY(prepare_views(g, true, sched.hub_degree, sched.build, core_size(g, sched)));
     if (!oriented) TC_TRY(prepare_views(g, false));
     int mode = oriented ? kOriented : kDirect;
     if (!oriented && direct_by_tasks(g, sched)) {
@@ -3452,57 +3531,53 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     // flush.  Beyond kBitsIds1 ids a row is tiled by id range, which pays for
     // the largest bin only (the mid bin's lists go through LDS tables).
     P.id_tiles = 0;
-    const bool one_bits = mode == kByTasks && nv <= kBitsIds1;  // bins 1 and 2 in one launch
+    const bool one_bits = mode == kByTasks && nv <= kBitsIds1;
     if (mode == kByTasks) {
         P.id_tiles = (int32_t)ceil_div(nv, kBitsIds1);
         P.lmax[2] = INT32_MAX;
         P.nw[2] = 8;
         P.flush_items = 16;
-        if (one_bits) {
-            P.lmax[1] = INT32_MAX;
-            P.nw[1] = 8;
-        }
+        if (one_bits) P.bin_max[1] = P.bin_max[0];  // (no mid bin)
     }
     TC_TRY(g.work.ensure((size_t)nv * sizeof(unsigned long long)));
     unsigned long long *work = g.work.as<unsigned long long>();
     hipLaunchKernelGGL(k_fill_u64, dim3(grid_for(nv, 256, 65536)), dim3(256), 0, s, work, (int64_t)nv);
     if (mode != kDirect)
         hipLaunchKernelGGL(k_owner_work<true>, dim3(wblocks), dim3(256), 0, s, coff, crow, vi, adj,
-                           tasks, nv, P, work, stats ? acc + 4 : nullptr);
+                           tasks, nv, P, work, acc + 26, acc + 27, stats ? acc + 4 : nullptr);
     else
         hipLaunchKernelGGL(k_owner_work<false>, dim3(wblocks), dim3(256), 0, s, coff, crow, vi, adj,
-                           nullptr, nv, P, work, stats ? acc + 4 : nullptr);
+                           nullptr, nv, P, work, acc + 26, acc + 27, stats ? acc + 4 : nullptr);
     TC_HIP(hipGetLastError());
-    TC_TRY(g.tmp3.ensure((size_t)3 * nv * sizeof(int32_t) + (size_t)3 * (nv + 1) * sizeof(int64_t) + 16));
-    int32_t *njobs = g.tmp3.as<int32_t>();
-    int64_t *jscan = reinterpret_cast<int64_t *>(njobs + 3 * (int64_t)nv + ((3 * (int64_t)nv) & 1));
-    if (mode != kDirect)
-        hipLaunchKernelGGL(k_plan_jobs<true>, dim3(grid_for(nv, 256, 4096)), dim3(256), 0, s, vi,
-                           work, nv, P, njobs, stats ? acc + 13 : nullptr);
-    else
-        hipLaunchKernelGGL(k_plan_jobs<false>, dim3(grid_for(nv, 256, 4096)), dim3(256), 0, s, vi,
-                           work, nv, P, njobs, stats ? acc + 13 : nullptr);
-    TC_HIP(hipGetLastError());
-    for (int b = 0; b < 3; ++b)
-        TC_TRY(scan_counts_i32(njobs + (int64_t)b * nv, jscan + (int64_t)b * (nv + 1), nv, g.tmp, s));
-    int64_t jt[3] = {g.plan.jt[0], g.plan.jt[1], g.plan.jt[2]};
-    if (!g.capturing) {
-        for (int b = 0; b < 3; ++b)
-            TC_HIP(hipMemcpyAsync(&jt[b], jscan + (int64_t)b * (nv + 1) + nv, sizeof(int64_t),
-                                  hipMemcpyDeviceToHost, s));
-        TC_HIP(hipStreamSynchronize(s));
-        for (int b = 0; b < 3; ++b) g.plan.jt[b] = jt[b];
+    // the longest list there can be (|N+| <= sqrt(nnz)), and with it the most
+    // jobs a bin can have: one per owner and tile, and what its work gives, at
+    // most 2^21 (k_plan_jobs)
+    const int64_t lists = oriented ? g.nplus : nnz;
+    const int64_t lmost = oriented ? (int64_t)std::sqrt((double)nnz) + 1
+                          : g.validated && !g.degree_stale ? g.max_degree : nv;
+    JobArrays J = {};
+    const int64_t owners[3] = {nv, std::min<int64_t>(nv, lists / (P.bin_max[0] + 1)),
+                               std::min<int64_t>(nv, lists / (P.bin_max[1] + 1))};
+    int64_t total_cap = 0;
+    for (int b = 0; b < 3; ++b) {
+        const bool any = b == 0 || lmost > P.bin_max[b - 1];
+        const double more = (double)lists * (double)(lmost + 4) / ((double)P.job_items * P.nw[b]);
+        J.cap[b] = any ? owners[b] + 64 + (int64_t)std::min(more, 2097152.0) : 0;
+        if (b == 2 && any) J.cap[b] += P.id_tiles > 0 ? owners[b] * P.id_tiles : 2 * (lists / P.lmax[2]);
+        total_cap += J.cap[b];
     }
-    TC_TRY(g.jobs.ensure((size_t)(jt[0] + jt[1] + jt[2] + 1) * sizeof(Job)));
-    Job *j0 = g.jobs.as<Job>();
-    Job *j1 = j0 + jt[0];
-    Job *j2 = j1 + jt[1];
+    TC_TRY(g.jobs.ensure((size_t)total_cap * sizeof(Job)));
+    J.j[0] = g.jobs.as<Job>();
+    J.j[1] = J.j[0] + J.cap[0];
+    J.j[2] = J.j[1] + J.cap[1];
+    unsigned long long *jc = acc + 28;
+    const dim3 pgrid((unsigned)ceil_div(nv, kPlanOwners)), pblock(kPlanThreads);
     if (mode != kDirect)
-        hipLaunchKernelGGL(k_emit_jobs<true>, dim3(grid_for(nv, 256, 65536)), dim3(256), 0, s, vi,
-                           njobs, jscan, nv, P, j0, j1, j2);
+        hipLaunchKernelGGL(k_plan_jobs<true>, pgrid, pblock, 0, s, vi, work, nv, P, acc + 26, acc + 27, J, jc,
+                           stats ? acc + 13 : nullptr);
     else
-        hipLaunchKernelGGL(k_emit_jobs<false>, dim3(grid_for(nv, 256, 65536)), dim3(256), 0, s, vi,
-                           njobs, jscan, nv, P, j0, j1, j2);
+        hipLaunchKernelGGL(k_plan_jobs<false>, pgrid, pblock, 0, s, vi, work, nv, P, acc + 26, acc + 27, J, jc,
+                           stats ? acc + 13 : nullptr);
     TC_HIP(hipGetLastError());
     TC_HIP(rec(g.ev[2]));
 
@@ -3555,24 +3630,21 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
                            g.outr.as<uint32_t>(), (int64_t)nv, 0u);
         A.outr = g.outr.as<uint32_t>();
     }
-    if (oriented && jt[2] > 0) {
-        TC_TRY(g.hjobs.ensure((size_t)jt[2] * sizeof(int64_t)));
+    if (oriented && J.cap[2] > 0) {
+        TC_TRY(g.hjobs.ensure((size_t)J.cap[2] * sizeof(int64_t)));
         A.hjobs = g.hjobs.as<int64_t>();
     }
-    const Job *jl[3] = {j0, j1, j2};
     for (int b = 0; b < 3; ++b) {
         TC_HIP(rec(g.ev[3 + b]));
-        // bit rows of any list: the mid and largest bins' jobs in one launch
-        if (one_bits && b == 1) continue;
-        const int64_t nj = one_bits && b == 2 ? jt[1] + jt[2] : jt[b];
-        TC_TRY(launch_bin(b, mode, one_bits && b == 2 ? jl[1] : jl[b], nj, A, s, g.capturing ? nullptr : &g.ev[8]));
+        TC_TRY(launch_bin(b, mode, J.j[b], J.cap[b], jc + b, A, s, g.capturing ? nullptr : &g.ev[8]));
     }
     TC_HIP(rec(g.ev[6]));  // end of the bin kernels
     if (oriented && g.core_k > 0) TC_TRY(core_count(g, acc, reinterpret_cast<int32_t *>(acc + 27), A.gid));
     if (oriented && nplus > 0) {
         hipLaunchKernelGGL(k_plus_row_sum, dim3(grid_for(ceil_div(nplus, kWave), 4, 1 << 16)),
                            dim3(256), 0, s, g.ov[6].as<int64_t>(), g.ov[10].as<int32_t>(),
-                           g.pcnt.as<uint32_t>(), nv, nplus, g.outr.as<uint32_t>());
+                           g.pcnt.as<uint32_t>(), nv, nplus, g.outr.as<uint32_t>(),
+                           reinterpret_cast<const int32_t *>(acc + 27) + 1);
         TC_HIP(hipGetLastError());
     }
     if (oriented) {
@@ -3583,21 +3655,23 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     g.plan.method = method;
     if (g.capturing) return TC_OK;  // results are read after the replay
     TC_HIP(hipEventRecord(g.ev[7], s));
-    TC_HIP(hipEventSynchronize(g.ev[7]));
-
-    unsigned long long hacc[28];
-    TC_HIP(hipMemcpy(hacc, acc, sizeof(hacc), hipMemcpyDeviceToHost));
-    if (oriented && g.core_k > 0 && hacc[27]) {  // rows declared symmetric that are not
+    const unsigned long long *hacc = g.hcounts;
+    TC_HIP(hipMemcpyAsync(g.hcounts, acc, 32 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+    TC_HIP(hipStreamSynchronize(s));
+    if (oriented && hacc[27]) {  // rows declared symmetric that are not
         g.symmetric = 0;
         if (sched.method == TC_METHOD_ORIENTED) {
             set_last_error(TC_ERR_INVALID, "oriented layout: the rows are not symmetric");
             return TC_ERR_INVALID;
         }
+        if (g.batch_per_graph)
+            hipLaunchKernelGGL(k_fill_u64, dim3(grid_for(g.batch_ngraphs, 256, 4096)), dim3(256), 0, s,
+                               g.batch_per_graph, (int64_t)g.batch_ngraphs);
         return count_pass(g, out, global, sched, stats, skip_lower);  // the direct way
     }
     if (global) *global = hacc[0];
     if (stats) {
-        fill_counters(st, hacc, jt, oriented);
+        fill_counters(st, hacc, oriented);
         float ms = 0;
         (void)hipEventElapsedTime(&ms, g.ev[0], g.ev[7]);
         st.ms_total = ms;
@@ -3609,7 +3683,7 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
             (void)hipEventElapsedTime(&ms, g.ev[3 + b], g.ev[4 + b]);
             st.ms_bin[b] = ms;
         }
-        if (oriented && jt[2] > 0) {
+        if (oriented && hacc[30] > 0) {
             for (int k = 0; k < 2; ++k) {
                 (void)hipEventElapsedTime(&ms, g.ev[8 + k], g.ev[9 + k]);
                 st.ms_long[k] = ms;
@@ -3653,12 +3727,10 @@ int count_replay(Graph &g, uint64_t *global, tc_stats *stats)
     TC_HIP(hipGraphLaunch(g.cexec, s));
     TC_HIP(hipEventRecord(g.ev[7], s));
     TC_HIP(hipEventSynchronize(g.ev[7]));
-    unsigned long long hacc[28];
-    int32_t bad = 0;
-    TC_HIP(hipMemcpy(hacc, g.accum.p, sizeof(hacc), hipMemcpyDeviceToHost));
-    if (g.plan.method == TC_METHOD_ORIENTED && g.plan.bad)
-        TC_HIP(hipMemcpy(&bad, g.plan.bad, sizeof(bad), hipMemcpyDeviceToHost));
-    if (bad || (g.plan.method == TC_METHOD_ORIENTED && hacc[27])) {  // cannot happen for an unchanged store that counted before
+    const unsigned long long *hacc = g.hcounts;
+    TC_HIP(hipMemcpyAsync(g.hcounts, g.accum.p, 32 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+    TC_HIP(hipStreamSynchronize(s));
+    if (g.plan.method == TC_METHOD_ORIENTED && hacc[27]) {  // cannot happen for an unchanged store that counted before
         g.symmetric = 0;
         g.touch();
         set_last_error(TC_ERR_INVALID, "oriented layout: the rows are not symmetric");
@@ -3667,7 +3739,7 @@ int count_replay(Graph &g, uint64_t *global, tc_stats *stats)
     if (global) *global = hacc[0];
     if (stats) {
         tc_stats st = {};
-        fill_counters(st, hacc, g.plan.jt, g.plan.method == TC_METHOD_ORIENTED);
+        fill_counters(st, hacc, g.plan.method == TC_METHOD_ORIENTED);
         float ms = 0;
         (void)hipEventElapsedTime(&ms, g.ev[0], g.ev[7]);
         st.ms_total = ms;
