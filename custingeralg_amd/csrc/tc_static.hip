@@ -1786,15 +1786,40 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan_jobs(
 
 // outr[r] += 2 * (sum of pcnt over N+(r)): the task-vertex share of the
 // oriented count, one segmented wave sum per 64 entries of the plus array.
-__global__ void k_plus_row_sum(const int64_t *__restrict__ pcoff, const int32_t *__restrict__ pcrow,
-                               const uint32_t *__restrict__ pcnt, int32_t nv, int64_t nplus,
-                               uint32_t *__restrict__ outr, const int32_t *__restrict__ asym)
+// HUBS: the entries that point to the last hubs ranks hold third-vertex hits
+// (k_count) and are credited to that rank instead, summed in LDS.  Those ranks
+// are what most lists end in: credited from k_count one by one, their few cache
+// lines were much of its middle bin (R-MAT 20 1460 -> 850 us, 3M ragged vertices
+// 5690 -> 5300; R-MAT 24, where fewer third vertices are hubs, 15.4 ms either
+// way), for one more read of the entries here.  Not for batched graphs: each has
+// hubs of its own, too many for one block's sums.
+constexpr int kSumThreads = 512;
+constexpr int32_t kSumHubs = 4096;
+
+template <bool HUBS>
+__global__ __launch_bounds__(kSumThreads) void k_plus_row_sum(const int64_t *__restrict__ pcoff,
+                                                              const int32_t *__restrict__ pcrow,
+                                                              const int32_t *__restrict__ padj,
+                                                              const uint32_t *__restrict__ pcnt, int32_t nv,
+                                                              int64_t nplus, int32_t hubs,
+                                                              uint32_t *__restrict__ outr,
+                                                              const int32_t *__restrict__ asym)
 {
     if (*asym) return;
+    __shared__ uint32_t hub[HUBS ? kSumHubs : 1];
+    const int32_t hub_lo = nv - hubs;
+    if (HUBS) {
+        for (int q = threadIdx.x; q < hubs; q += blockDim.x) hub[q] = 0u;
+        __syncthreads();
+    }
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t nchunks = ceil_div(nplus, kWave);
     const int64_t wstride = (int64_t)gridDim.x * (blockDim.x / kWave);
-    auto chunk = [&](int64_t e, int32_t r, uint32_t x) {
+    auto chunk = [&](int64_t e, int32_t r, uint32_t x, int32_t w) {
+        if (HUBS && x && w >= hub_lo) {
+            atomicAdd(&hub[w - hub_lo], x);
+            x = 0u;
+        }
 #pragma unroll
         for (int d = 1; d < kWave; d <<= 1) {
             const uint32_t y = __shfl_up(x, d, kWave);
@@ -1814,10 +1839,17 @@ __global__ void k_plus_row_sum(const int64_t *__restrict__ pcoff, const int32_t 
         const int64_t e = c * kWave + lane, e2 = c2 * kWave + lane;
         const uint32_t x = e < nplus ? pcnt[e] : 0u;
         const uint32_t x2 = (two && e2 < nplus) ? pcnt[e2] : 0u;
+        const int32_t w = HUBS && e < nplus ? padj[e] : 0;
+        const int32_t w2 = HUBS && two && e2 < nplus ? padj[e2] : 0;
         int32_t r, r2;
         wave_rows_of2(pcoff, pcrow, nv, c, two ? c2 : c, nplus, r, r2);
-        chunk(e, r, x);
-        if (two) chunk(e2, r2, x2);
+        chunk(e, r, x, w);
+        if (two) chunk(e2, r2, x2, w2);
+    }
+    if (HUBS) {
+        __syncthreads();
+        for (int q = threadIdx.x; q < hubs; q += blockDim.x)
+            if (const uint32_t x = hub[q]) atomicAdd(&outr[hub_lo + q], 2u * x);
     }
 }
 
@@ -1893,6 +1925,9 @@ struct CountArgs {
     // to the hash-table launch, [2] that launch's next entry of the list
     unsigned long long *job_ctr;
     int32_t nv;
+    // oriented, one graph: first rank of the core, whose third-vertex counts go
+    // to pcnt (INT32_MAX: none)
+    int32_t hub_lo;
     int64_t *hjobs;  // room for every job of the largest bin (or null)
 };
 
@@ -2525,16 +2560,19 @@ __global__ __launch_bounds__(NW * kWave, LMAX <= 64 ? TC_SMALL_WAVES : LMAX <= 5
         unsigned long long hjob = 0;
         for (int w = 0; w < NW; ++w) hjob += red[w];
         if (ORIENTED) {
-            if (by_pos) {
-                for (int i = threadIdx.x; i < L; i += nthr) {
-                    const uint32_t ci = C[i];
-                    if (ci) atomicAdd(&A.out[A.order[Sg[i]]], 2u * ci);
-                }
-            } else {
-                for (int i = threadIdx.x; i < kSlots << nbb; i += nthr) {
-                    const uint32_t ci = C[i];
-                    if (ci) atomicAdd(&A.out[A.order[T.id_at(i)]], 2u * ci);
-                }
+            // third vertices; a hub's count goes to the owner's entry of it (no
+            // task's: a core owner has none), for k_plus_row_sum to credit
+            const bool whole = J.t_begin == 0 && J.t_end == vo.dm;  // the owner's only job
+            for (int i = threadIdx.x; i < L; i += nthr) {
+                const int32_t w = Sg[i];
+                const uint32_t ci = C[by_pos ? i : lookup(w)];
+                if (!ci) continue;
+                if (w < A.hub_lo)
+                    atomicAdd(&A.out[A.order[w]], 2u * ci);
+                else if (whole)
+                    A.pcnt[obase + s0 + i] = ci;
+                else
+                    atomicAdd(&A.pcnt[obase + s0 + i], ci);
             }
         }
         const int32_t owner_v = ORIENTED ? A.order[J.owner] : J.owner;
@@ -3590,6 +3628,8 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     A.toff = mode != kDirect ? coff : nullptr;
     A.cred = mode == kByTasks ? g.ov[16].as<int32_t>() : nullptr;
     A.nv = nv;
+    const int32_t hubs = oriented && !g.batch_voff && g.core_k <= kSumHubs ? g.core_k : 0;
+    A.hub_lo = hubs > 0 ? nv - hubs : INT32_MAX;
     A.order = oriented ? g.order.as<int32_t>() : nullptr;
     A.out = outp;
     A.global = acc;
@@ -3641,9 +3681,13 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     TC_HIP(rec(g.ev[6]));  // end of the bin kernels
     if (oriented && g.core_k > 0) TC_TRY(core_count(g, acc, reinterpret_cast<int32_t *>(acc + 27), A.gid));
     if (oriented && nplus > 0) {
-        hipLaunchKernelGGL(k_plus_row_sum, dim3(grid_for(ceil_div(nplus, kWave), 4, 1 << 16)),
-                           dim3(256), 0, s, g.ov[6].as<int64_t>(), g.ov[10].as<int32_t>(),
-                           g.pcnt.as<uint32_t>(), nv, nplus, g.outr.as<uint32_t>(),
+        // (hubs: blocks of 16K entries at least, so that the sums of a block are
+        // worth adding up)
+        const auto sum = hubs > 0 ? k_plus_row_sum<true> : k_plus_row_sum<false>;
+        const int64_t per = hubs > 0 ? 16384 : kSumThreads;
+        hipLaunchKernelGGL(sum, dim3(grid_for(nplus, per, hubs > 0 ? 1024 : 32768)), dim3(kSumThreads), 0, s,
+                           g.ov[6].as<int64_t>(), g.ov[10].as<int32_t>(), g.padj.as<int32_t>(),
+                           g.pcnt.as<uint32_t>(), nv, nplus, hubs, g.outr.as<uint32_t>(),
                            reinterpret_cast<const int32_t *>(acc + 27) + 1);
         TC_HIP(hipGetLastError());
     }

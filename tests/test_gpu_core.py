@@ -50,6 +50,15 @@ def test_rmat(scale, ef):
     _check(*O.rmat_graph(scale, ef, 12), policy=T.POLICY_LEARNED)
 
 
+@pytest.mark.parametrize("kw", [dict(job_items=64), dict(job_items=1 << 20), dict(small_max=16, mid_max=64),
+                                dict(policy=T.POLICY_MERGE), dict(policy=T.POLICY_HASH)])
+def test_owners_in_one_and_several_jobs(kw):
+    """Third-vertex counts of core vertices, stored by an owner's only job and
+    added by several."""
+    _check(*_planted(20000, 600, 3), **kw)
+    _check(*O.rmat_graph(15, 16, 13), **kw)
+
+
 def test_recorded_counts():
     off, adj = _planted(20000, 600, 5)
     ref = O.custinger_count(off, adj)
