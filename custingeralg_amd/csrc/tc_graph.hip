@@ -273,83 +273,180 @@ __global__ void k_copy_rows(const int64_t *__restrict__ off, const int32_t *__re
     }
 }
 
-__device__ inline int32_t row_search_g(const int64_t *__restrict__ coff, int64_t e, int32_t lo,
-                                       int32_t hi)
+// Rows that hold the compact entries e[0..N) (the same in every lane): 64 rows
+// probed at a time, the N searches in lockstep.
+template <int N>
+__device__ inline void wave_row_search(const int64_t *__restrict__ coff, int32_t nv, const int64_t (&e)[N],
+                                       int32_t (&row)[N])
 {
-    while (lo < hi) {
-        int32_t mid = lo + ((hi - lo + 1) >> 1);
-        if (coff[mid] <= e) lo = mid; else hi = mid - 1;
+    const int lane = threadIdx.x & (kWave - 1);
+#pragma unroll
+    for (int q = 0; q < N; ++q) row[q] = 0;
+    for (int32_t n = nv; n > 1;) {
+        const int32_t step = (n + kWave - 1) / kWave;
+        int64_t v[N];
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
+            const int64_t r = (int64_t)row[q] + (int64_t)lane * step;
+            v[q] = (int64_t)lane * step < n && r < nv ? coff[r] : INT64_MAX;
+        }
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
+            const uint64_t m = __ballot(v[q] <= e[q]);
+            row[q] += m ? (63 - __clzll((long long)m)) * step : 0;
+        }
+        n = step;
     }
-    return lo;
 }
 
 // Validation over compact entries: [0] unsorted/dup, [1] out of range,
 // [2] self loops, [3] missing reverse entries, [4] max degree, [5] entries
 // that leave their graph (gid: the graph of every vertex, or null).
-__global__ void k_validate(const int64_t *__restrict__ coff, const int64_t *__restrict__ boff,
-                           const int32_t *__restrict__ len, const int32_t *__restrict__ pool,
-                           int32_t nv, int64_t nnz, int check_sym, const int32_t *__restrict__ gid,
-                           unsigned long long *__restrict__ res)
-{
-    const int lane = threadIdx.x & (kWave - 1);
-    const int64_t nchunks = ceil_div(nnz, kWave);
-    const int64_t wstride = (int64_t)gridDim.x * (blockDim.x / kWave);
-    unsigned long long bad = 0, oor = 0, loops = 0, miss = 0, cross = 0;
-    for (int64_t c = (int64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave; c < nchunks;
-         c += wstride) {
-        int64_t e = c * kWave + lane;
-        int64_t e0 = c * kWave, elast = min(e0 + kWave, nnz) - 1;
-        int32_t rf = 0, rl = 0;
-        if (lane == 0) rf = row_search_g(coff, e0, 0, nv - 1);
-        if (lane == 1) rl = row_search_g(coff, elast, 0, nv - 1);
-        rf = __shfl(rf, 0);
-        rl = __shfl(rl, 1);
-        if (e > elast) continue;
-        int32_t a = row_search_g(coff, e, rf, rl);
-        int64_t k = e - coff[a];
-        int64_t addr = boff[a] + k;
-        int32_t b = pool[addr];
-        if (b < 0 || b >= nv) {
-            ++oor;
-            continue;
-        }
-        if (k > 0 && pool[addr - 1] >= b) ++bad;
-        if (b == a) ++loops;
-        if (gid && gid[a] != gid[b]) ++cross;
-        if (check_sym) {
-            const int32_t *lst = pool + boff[b];
-            int32_t lo = 0, hi = len[b];
-            while (lo < hi) {
-                int32_t mid = (lo + hi) >> 1;
-                if (lst[mid] < a) lo = mid + 1; else hi = mid;
-            }
-            if (!(lo < len[b] && lst[lo] == a)) ++miss;
-        }
-    }
-    for (int d = 32; d > 0; d >>= 1) {
-        bad += __shfl_xor(bad, d);
-        oor += __shfl_xor(oor, d);
-        loops += __shfl_xor(loops, d);
-        miss += __shfl_xor(miss, d);
-        cross += __shfl_xor(cross, d);
-    }
-    if (lane == 0) {
-        if (bad) atomicAdd(&res[0], bad);
-        if (oor) atomicAdd(&res[1], oor);
-        if (loops) atomicAdd(&res[2], loops);
-        if (miss) atomicAdd(&res[3], miss);
-        if (cross) atomicAdd(&res[5], cross);
-    }
-}
+//
+// Symmetry: an entry (a, b) is looked for in the other row where that is the
+// shorter one (ties: the lower id), and [6] counts those entries.  If none
+// misses its reverse, the rows are symmetric exactly when the other entries are
+// as many.  Half the searches, and none in a hub's row for its leaves' entries.
+// Bound by the cache lines of the rows searched, one or two per search (250K
+// R-MAT vertices at edge factor 16: 429 -> 250 us; 1.2M entries, each to a higher
+// id: 53 -> 22).  A wave takes two chunks of 64 entries in lockstep;
+// one or four took 8% longer.
+constexpr int kValThreads = 512;
 
-__global__ void k_max_len(const int32_t *__restrict__ len, int32_t nv, unsigned long long *res)
+__global__ __launch_bounds__(kValThreads) void k_validate(
+    const int64_t *__restrict__ coff, const int64_t *__restrict__ boff, const int32_t *__restrict__ len,
+    const int32_t *__restrict__ pool, int32_t nv, int64_t nnz, int check_sym, const int32_t *__restrict__ gid,
+    unsigned long long *__restrict__ res)
 {
-    unsigned long long m = 0;
-    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nv;
-         v += (int64_t)gridDim.x * blockDim.x)
-        m = max(m, (unsigned long long)len[v]);
-    for (int d = 32; d > 0; d >>= 1) m = max(m, (unsigned long long)__shfl_xor(m, d));
-    if ((threadIdx.x & 63) == 0) atomicMax(res, m);
+    constexpr int U = 2;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int64_t npairs = ceil_div(nnz, U * kWave);
+    const int64_t wstride = (int64_t)gridDim.x * (blockDim.x / kWave);
+    uint32_t bad = 0, oor = 0, loops = 0, miss = 0, cross = 0, down = 0;
+    int32_t most = 0;
+    for (int64_t c = (int64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave; c < npairs;
+         c += wstride) {
+        const int64_t e0 = c * U * kWave;
+        int64_t edge[U + 1];
+        int32_t row[U + 1];
+#pragma unroll
+        for (int u = 0; u <= U; ++u) edge[u] = min(e0 + u * kWave, nnz - 1);
+        wave_row_search<U + 1>(coff, nv, edge, row);
+        int64_t e[U];
+        int32_t a[U], top[U];
+        bool go = false;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            e[u] = min(e0 + u * kWave + lane, nnz - 1);
+            a[u] = row[u];
+            top[u] = max(row[u], row[u + 1]);
+            go = go || a[u] < top[u];
+        }
+        while (go) {
+            go = false;
+            int64_t v[U];
+            int32_t mid[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                mid[u] = a[u] + ((top[u] - a[u] + 1) >> 1);
+                v[u] = coff[mid[u]];
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (a[u] < top[u]) {
+                    if (v[u] <= e[u]) a[u] = mid[u]; else top[u] = mid[u] - 1;
+                }
+                go = go || a[u] < top[u];
+            }
+        }
+        int32_t b[U], la[U], lb[U], lo[U], hi[U];
+        int64_t at[U];
+        bool in[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t k = e[u] - coff[a[u]], addr = boff[a[u]] + k;
+            la[u] = len[a[u]];
+            b[u] = pool[addr];
+            const int32_t before = k > 0 ? pool[addr - 1] : -1;
+            in[u] = e0 + u * kWave + lane < nnz;
+            if (in[u]) {
+                if (b[u] < 0 || b[u] >= nv) {
+                    ++oor;
+                    in[u] = false;
+                } else {
+                    bad += k > 0 && before >= b[u];
+                    loops += b[u] == a[u];
+                }
+            }
+        }
+        if (gid) {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (in[u] && gid[a[u]] != gid[b[u]]) ++cross;
+        }
+        if (!check_sym) continue;
+        go = false;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            lb[u] = in[u] ? len[b[u]] : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            in[u] = in[u] && b[u] != a[u] && (lb[u] < la[u] || (lb[u] == la[u] && b[u] < a[u]));
+            at[u] = in[u] ? boff[b[u]] : 0;
+            lo[u] = 0;
+            hi[u] = in[u] ? lb[u] : 0;
+            go = go || hi[u] > 0;
+        }
+        while (go) {
+            go = false;
+            int32_t x[U], mid[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                mid[u] = (lo[u] + hi[u]) >> 1;
+                x[u] = lo[u] < hi[u] ? pool[at[u] + mid[u]] : 0;
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (lo[u] < hi[u]) {
+                    if (x[u] < a[u])
+                        lo[u] = mid[u] + 1;
+                    else
+                        hi[u] = x[u] == a[u] ? -1 : mid[u];  // (-1: found)
+                }
+                go = go || lo[u] < hi[u];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            down += in[u];
+            miss += in[u] && hi[u] != -1;
+        }
+    }
+    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nv; v += (int64_t)gridDim.x * blockDim.x)
+        most = max(most, len[v]);
+    __shared__ unsigned long long part[kValThreads / kWave][7];
+    const uint32_t mine[7] = {bad, oor, loops, miss, (uint32_t)most, cross, down};
+#pragma unroll
+    for (int q = 0; q < 7; ++q) {
+        unsigned long long x = mine[q];
+        if (q == 4)
+            for (int d = 32; d > 0; d >>= 1) x = max(x, __shfl_xor(x, d));
+        else
+            x = wave_sum<unsigned long long>(x);
+        if (lane == 0) part[threadIdx.x / kWave][q] = x;
+    }
+    __syncthreads();
+    if (threadIdx.x < 7) {
+        unsigned long long x = 0;
+        const bool top = threadIdx.x == 4;
+        for (int w = 0; w < kValThreads / kWave; ++w) {
+            const unsigned long long p = part[w][threadIdx.x];
+            x = top ? max(x, p) : x + p;
+        }
+        if (top && x) atomicMax(&res[4], x);
+        if (!top && x) atomicAdd(&res[threadIdx.x], x);
+    }
 }
 
 __global__ void k_zero_u64(unsigned long long *p, int n)
@@ -384,16 +481,10 @@ int validate_graph(Graph &g, bool check_symmetry, int64_t *bad_rows)
         TC_TRY(g.coff.ensure((size_t)(nv + 1) * sizeof(int64_t)));
         int64_t *coff = g.coff.as<int64_t>();
         TC_TRY(scan_counts_i32(g.st.len.as<int32_t>(), coff, nv, g.tmp, s));
-        if (nnz > 0) {
-            int64_t nchunks = ceil_div(nnz, kWave);
-            hipLaunchKernelGGL(k_validate, dim3(grid_for(nchunks, 4, 1 << 16)), dim3(256), 0, s, coff,
-                               g.st.boff.as<int64_t>(), g.st.len.as<int32_t>(),
-                               g.st.pool.as<int32_t>(), nv, nnz, check_symmetry ? 1 : 0,
-                               g.batch_voff ? g.dgid.as<int32_t>() : nullptr, res);
-            TC_HIP(hipGetLastError());
-        }
-        hipLaunchKernelGGL(k_max_len, dim3(grid_for(nv, 256, 4096)), dim3(256), 0, s,
-                           g.st.len.as<int32_t>(), nv, res + 4);
+        hipLaunchKernelGGL(k_validate, dim3(grid_for(std::max<int64_t>(nnz, nv), 2 * kValThreads, 1024)),
+                           dim3(kValThreads), 0, s, coff, g.st.boff.as<int64_t>(), g.st.len.as<int32_t>(),
+                           g.st.pool.as<int32_t>(), nv, nnz, check_symmetry ? 1 : 0,
+                           g.batch_voff ? g.dgid.as<int32_t>() : nullptr, res);
         TC_HIP(hipGetLastError());
     }
     unsigned long long h[16];
@@ -409,7 +500,7 @@ int validate_graph(Graph &g, bool check_symmetry, int64_t *bad_rows)
     }
     g.validated = true;
     g.self_loops = (int64_t)h[2];
-    if (check_symmetry) g.symmetric = h[3] == 0 ? 1 : 0;
+    if (check_symmetry) g.symmetric = h[3] == 0 && 2 * h[6] + h[2] == (unsigned long long)nnz ? 1 : 0;
     g.max_degree = (int32_t)h[4];
     g.degree_stale = false;
     // bit matrices hold a graph's own columns only
