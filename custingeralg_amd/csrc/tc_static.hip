@@ -1582,10 +1582,13 @@ __device__ inline int owner_bin(int32_t L, const PlanParams &P)
 }
 
 // Per-owner estimated work (sum over its tasks); per-bin stats.
-template <bool ORIENTED>
 // Entries are the task array (oriented) or the store rows (direct), with
-// their row offsets coff and chunk rows crow.
-__global__ void k_owner_work(const int64_t *__restrict__ coff, const int32_t *__restrict__ crow,
+// their row offsets coff and chunk rows crow.  Two blocks of 16 waves per CU:
+// each adds to the one total of all owners, and 4096 blocks of 4 waves spent
+// most of their time in that (250K R-MAT vertices 64 -> 20 us, R-MAT 20 96 -> 54).
+constexpr int kWorkThreads = 1024, kWorkBlocks = 512;
+template <bool ORIENTED>
+__global__ __launch_bounds__(kWorkThreads) void k_owner_work(const int64_t *__restrict__ coff, const int32_t *__restrict__ crow,
                              const VInfo *__restrict__ vi,
                              const int32_t *__restrict__ adj, const TaskRec *__restrict__ tasks,
                              int32_t nv, PlanParams P,
@@ -3548,9 +3551,7 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     const TaskRec *tasks = mode != kDirect ? g.tasks.as<TaskRec>() : nullptr;
     // planning walks the task array (oriented, by tasks) or the store rows (direct)
     const int64_t nchunks = ceil_div(oriented ? g.ntasks : nnz, kWave);
-    // 4 waves of 256 threads; 16 blocks per CU keep the chip busy and bound
-    // the number of per-block statistics atomics
-    const int wblocks = grid_for(nchunks, 4, 4096);
+    const int wblocks = grid_for(nchunks, 2 * kWorkThreads / kWave, kWorkBlocks);
 
     // ---- planning: work per owner, jobs per bin
     PlanParams P;
@@ -3581,10 +3582,10 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     unsigned long long *work = g.work.as<unsigned long long>();
     hipLaunchKernelGGL(k_fill_u64, dim3(grid_for(nv, 256, 65536)), dim3(256), 0, s, work, (int64_t)nv);
     if (mode != kDirect)
-        hipLaunchKernelGGL(k_owner_work<true>, dim3(wblocks), dim3(256), 0, s, coff, crow, vi, adj,
+        hipLaunchKernelGGL(k_owner_work<true>, dim3(wblocks), dim3(kWorkThreads), 0, s, coff, crow, vi, adj,
                            tasks, nv, P, work, acc + 26, acc + 27, stats ? acc + 4 : nullptr);
     else
-        hipLaunchKernelGGL(k_owner_work<false>, dim3(wblocks), dim3(256), 0, s, coff, crow, vi, adj,
+        hipLaunchKernelGGL(k_owner_work<false>, dim3(wblocks), dim3(kWorkThreads), 0, s, coff, crow, vi, adj,
                            nullptr, nv, P, work, acc + 26, acc + 27, stats ? acc + 4 : nullptr);
     TC_HIP(hipGetLastError());
     // the longest list there can be (|N+| <= sqrt(nnz)), and with it the most
