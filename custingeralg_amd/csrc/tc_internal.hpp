@@ -273,6 +273,20 @@ void graph_destroy(Graph *g);
 tc_schedule default_schedule();
 
 // ------------------------------------------------------- reductions --
+__device__ inline void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ inline int64_t readlane_i64(int64_t x, int lane)
+{
+    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)(uint64_t)x, lane);
+    const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)((uint64_t)x >> 32), lane);
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
 template <class T> __device__ inline T wave_sum(T x)
 {
 #pragma unroll

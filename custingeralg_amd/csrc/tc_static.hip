@@ -51,13 +51,6 @@ template <int LMAX> constexpr int big_task_min()
 #endif
 constexpr int kBigUnroll = TC_BIG_UNROLL;  // loads in flight per lane on long tasks
 
-__device__ inline int64_t readlane_i64(int64_t x, int lane)
-{
-    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)(uint64_t)x, lane);
-    const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)((uint64_t)x >> 32), lane);
-    return (int64_t)(((uint64_t)hi << 32) | lo);
-}
-
 // Bucketed two-choice hash table in LDS.  Bucket b holds up to S ids (S = 4:
 // 16-byte buckets, S = 2: 8-byte buckets) in slots S b .. S b + S - 1, filled
 // as a prefix (inserts claim the first empty slot by CAS), -1 when empty.  An
@@ -244,13 +237,6 @@ struct TileBitmap {
 };
 
 // ------------------------------------------------------------ helpers --
-
-__device__ inline void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 __device__ inline int32_t wave_incl_scan_i32(int32_t x)
 {

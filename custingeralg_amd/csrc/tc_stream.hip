@@ -32,21 +32,18 @@ constexpr int kRowThreads = 1024;
 #define TC_DELTA_BLOCKS 4096
 #endif
 constexpr int kDeltaBlocks = TC_DELTA_BLOCKS;  // k_delta_lb's largest grid (4 waves per block)
-// Edges of a batch above the one-block size whose lists are both long and of
-// similar length are intersected by merge path, in segments of kMergeSeg
-// merge positions, instead of one binary search per entry.
-#ifndef TC_MERGE_MIN
-#define TC_MERGE_MIN 256
-#endif
-#ifndef TC_MERGE_RATIO
-#define TC_MERGE_RATIO 16
-#endif
-#ifndef TC_MERGE_SEG
-#define TC_MERGE_SEG 4096
-#endif
-constexpr int32_t kMergeMin = TC_MERGE_MIN;      // the shorter list at least this long
-constexpr int32_t kMergeRatio = TC_MERGE_RATIO;  // the longer at most this many times as long
-constexpr int32_t kMergeSeg = TC_MERGE_SEG;
+// Edges of a batch above the one-block size whose lists are both long and not too
+// unlike are intersected in segments of kMergeSeg merge positions (k_delta_merge)
+// instead of one binary search per entry (k_delta_lb).  The search costs 13 steps
+// of scattered reads per entry of the shorter list, a segment reads both lists:
+// at a million pairs of 4M R-MAT vertices 64 entries and a ratio of 64 took
+// 14.7 ms, 256 and 16 (what merging window by window wanted) 16.2, 32 and 64 15.1.
+// A segment's fixed cost is hidden by many others only: batches below
+// kMergeMany pairs took 3% longer with 64 than with 128 on uniform rows of 64.
+constexpr int32_t kMergeMin = 64, kMergeMinFew = 128;  // the shorter list at least this long
+constexpr int64_t kMergeMany = 1 << 17;
+constexpr int32_t kMergeRatio = 64;  // the longer at most this many times as long
+constexpr int32_t kMergeSeg = 4096;
 // The insertion's pool reservation, words of a device control block: the
 // pool's first free entry and capacity (set by the host per batch), whether
 // the rows that move fit (else no row is touched, and the host grows the
@@ -878,9 +875,9 @@ __global__ void k_set_ctl(unsigned long long *__restrict__ ctl, unsigned long lo
 // With msegs given, an edge whose lists are both long and of similar length
 // (merge_edge) gets no items but msegs[t] merge-path segments of kMergeSeg
 // positions (k_delta_merge).
-__device__ inline bool merge_edge(int32_t mn, int32_t mx)
+__device__ inline bool merge_edge(int32_t mn, int32_t mx, int64_t n)
 {
-    return mn >= kMergeMin && (int64_t)mx <= (int64_t)kMergeRatio * mn;
+    return mn >= (n >= kMergeMany ? kMergeMin : kMergeMinFew) && (int64_t)mx <= (int64_t)kMergeRatio * mn;
 }
 
 __global__ void k_delta_items(const int32_t *__restrict__ pa, const int32_t *__restrict__ pb,
@@ -897,7 +894,7 @@ __global__ void k_delta_items(const int32_t *__restrict__ pa, const int32_t *__r
         if (t < lim && (sel == nullptr || sel[t])) {
             const int32_t la = len[pa[t]], lb = len[pb[t]];
             const int32_t mn = min(la, lb), mx = max(la, lb);
-            if (msegs && merge_edge(mn, mx))
+            if (msegs && merge_edge(mn, mx, n))
                 sg = (int32_t)ceil_div((int64_t)mn + mx, kMergeSeg);
             else
                 it = mn;
@@ -1020,74 +1017,294 @@ __global__ __launch_bounds__(kThreads) void k_delta_lb(
 // lists (the entries of X among the first d positions, by binary search).
 // The segment's X entries meet their equals, if any, in Y[iy0 .. iy1]: an
 // entry x = X[i] at merge position i + j (j entries of Y below it) lies in
-// the segment, so iy0 <= j <= iy1.  The parts are merged window by window by
-// the whole wave: each lane finds its x's co-rank in the 64-entry Y window
-// by a six-step search over the lanes; only values up to m = min(last x,
-// last y) are settled by a pair of windows, and each window then moves past
-// its entries <= m.  Every x is in one segment, so every common neighbour is
-// counted once; its credits are those of k_delta_lb.  Called per wave.
-__global__ __launch_bounds__(kThreads) void k_delta_merge(
+// the segment, so iy0 <= j <= iy1.  Every x is in one segment, so every common
+// neighbour is counted once; its credits are those of k_delta_lb.
+//
+// A wave takes a segment: its Y entries set a bit each in a hashed bit set of
+// its own in LDS, and its X entries test theirs.  The few that pass (the common
+// neighbours, and one in ten of the others) are queued and, 128 at a time,
+// looked for in Y: among the marks of its groups of 16 first, in LDS, then in
+// the group, all of it loaded at once.  Bound by the latency of the rows' reads
+// (0.5 GB of rows, 10 GB of reads): 8 windows in flight per wave.
+//
+// Credits of third vertices meet on a few hubs (4096 vertices hold half of a
+// million-pair batch's): a block keeps the ids that come first to each slot of a
+// table in LDS and their sums, and only what finds its slot taken goes to out at
+// once.
+//
+// Four launches for a million pairs of 4M R-MAT vertices and their undoing:
+// merged window by window through lane exchanges 14.0 ms; bit sets 9.1 (half the
+// blocks' size and an 8-byte credit slot), the whole-CU block 7.4, runs of
+// segments from all over the batch 6.6 (2.6 of it the queue, 0.8 the credits).
+constexpr int kMergeThreads = 1024, kMergeBlocks = 256;
+constexpr int kMergeWaves = kMergeThreads / kWave;
+constexpr int kMergeRuns = 8;
+constexpr int kSetBits = 15;     // bits of a wave's set: 4 KB
+constexpr int kMergeGroup = 16;  // entries of Y between two of the set's marks: 64 B
+constexpr int kCreditBits = 13;  // slots of a block's credit table: 32 KB
+constexpr uint32_t kMergeHash = 0x9E3779B1u;
+
+// x with x * kMergeHash = h
+__device__ inline uint32_t merge_unhash(uint32_t h)
+{
+    uint32_t inv = kMergeHash;  // (Newton: 3, 6, 12, 24, 48 bits)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) inv *= 2u - kMergeHash * inv;
+    return h * inv;
+}
+
+// Largest t in [0, n) with pre[t] <= i (pre[0] = 0), by the whole wave.
+__device__ inline int64_t wave_edge_of(const int64_t *__restrict__ pre, int64_t i, int64_t n)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    int64_t lo = 0;
+    while (n > 1) {
+        const int64_t step = (n + kWave - 1) / kWave;
+        const int64_t q = lane * step < n ? lane * step : 0;
+        const uint64_t m = __ballot(lane * step < n && pre[lo + q] <= i);
+        const int64_t j = m ? 63 - __clzll((long long)m) : 0;
+        lo += j * step;
+        n = min(step, n - j * step);
+    }
+    return lo;
+}
+
+// X entries among the first dd positions of the merge of X and Y (X first on
+// ties), by the whole wave.
+__device__ inline int32_t wave_split(const int32_t *__restrict__ X, int32_t nx, const int32_t *__restrict__ Y,
+                                     int32_t ny, int64_t dd)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    int32_t lo = (int32_t)max<int64_t>(0, dd - ny), hi = (int32_t)min<int64_t>(dd, nx);
+    while (lo < hi) {
+        const int32_t step = (hi - lo + kWave - 1) / kWave;
+        const int64_t q = (int64_t)lo + (int64_t)(lane + 1) * step - 1;
+        const uint64_t m = __ballot(q < hi && X[q < hi ? q : lo] <= Y[dd - 1 - (q < hi ? q : lo)]);
+        lo += (int32_t)__popcll(m) * step;  // (true for the first lanes only)
+        hi = min(hi, lo + step - 1);
+    }
+    return min(lo, hi);
+}
+
+struct MergeShared {
+    uint32_t set[kMergeWaves][1 << (kSetBits - 5)];
+    int32_t mark[kMergeWaves][kMergeSeg / kMergeGroup + 4];  // the first entry of every group of Y
+    int32_t qx[kMergeWaves][3 * kWave];                      // candidates: x
+    uint16_t qi[kMergeWaves][3 * kWave];                     // and its place in X's part
+    // credits: (the hash of x below its slot number, sum of the credits, 13 bits)
+    uint32_t credit[1 << kCreditBits];
+};
+
+__global__ __launch_bounds__(kMergeThreads, 4) void k_delta_merge(
     const int32_t *__restrict__ pa, const int32_t *__restrict__ pb,
     const int64_t *__restrict__ mpre, int64_t n, const int32_t *__restrict__ pool,
     const int64_t *__restrict__ boff, const int32_t *__restrict__ len,
     const uint8_t *__restrict__ flag, int32_t sign, uint32_t *__restrict__ out,
     uint32_t *__restrict__ ecnt, unsigned long long *__restrict__ gsum)
 {
-    const int lane = threadIdx.x & (kWave - 1);
+    constexpr int U = 8;  // windows of 64 entries in flight
+    constexpr uint32_t kFree = 0xFFFFFFFFu, kSumMask = (1u << kCreditBits) - 1, kDrain = 1u << (kCreditBits - 1);
+    static_assert(kDrain > 2 * kMergeThreads, "a slot's sum stays in its field");
+    __shared__ MergeShared S;
+    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+    for (int q = threadIdx.x; q < 1 << kCreditBits; q += kMergeThreads) S.credit[q] = kFree;
+    __syncthreads();
+    uint32_t *set = S.set[wid];
+    int32_t *mark = S.mark[wid], *qx = S.qx[wid];
+    uint16_t *qi = S.qi[wid];
+    auto hash = [](int32_t x) { return ((uint32_t)x * kMergeHash) >> (32 - kSetBits); };
+    auto credit = [&](int32_t x, uint32_t c) {
+        const uint32_t h = (uint32_t)x * kMergeHash;
+        uint32_t *at = &S.credit[h >> (32 - kCreditBits)];
+        const uint32_t tag = h << kCreditBits;  // (its low bits: an empty sum)
+        uint32_t w = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (w == kFree) w = atomicCAS(at, kFree, tag);
+        if (w != kFree && (w ^ tag) > kSumMask) {
+            atomicAdd(&out[x], (uint32_t)sign * c);
+            return;
+        }
+        const uint32_t before = atomicAdd(at, c) & kSumMask;
+        // a full slot is drained by the one that filled it; until then the others
+        // take back what they added, so that it never reaches the next field
+        if (before + c >= kDrain) {
+            const uint32_t back = before < kDrain ? kDrain : c;
+            atomicSub(at, back);
+            atomicAdd(&out[x], (uint32_t)sign * back);
+        }
+    };
     const int64_t total = mpre[n];
-    const int64_t nwaves = (int64_t)gridDim.x * (blockDim.x / kWave);
-    int64_t local = 0;
-    for (int64_t g = (int64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave; g < total;
-         g += nwaves) {
-        const int64_t t = edge_of(mpre, g, 0, n - 1);
-        const int64_t d0 = (g - mpre[t]) * kMergeSeg;
-        const int32_t s = pa[t], d = pb[t];
-        const int32_t ls = len[s], ld = len[d];
-        const bool s_short = ls <= ld;
-        const int32_t nx = s_short ? ls : ld, ny = s_short ? ld : ls;
-        const int64_t xb = s_short ? boff[s] : boff[d], yb = s_short ? boff[d] : boff[s];
-        const int32_t *X = pool + xb, *Y = pool + yb;
-        const int64_t d1 = min(d0 + kMergeSeg, (int64_t)nx + ny);
-        int32_t split = 0;
-        if (lane < 2) {  // X entries among the first dd merge positions
-            const int64_t dd = lane ? d1 : d0;
-            int32_t lo = (int32_t)max<int64_t>(0, dd - ny), hi = (int32_t)min<int64_t>(dd, nx);
-            while (lo < hi) {
-                const int32_t mid = (lo + hi) >> 1;
-                if (X[mid] <= Y[dd - 1 - mid]) lo = mid + 1; else hi = mid;
-            }
-            split = lo;
+    const int64_t nwaves = (int64_t)gridDim.x * kMergeWaves, wave = (int64_t)blockIdx.x * kMergeWaves + wid;
+    // runs of segments, so that an edge is looked up once per run; every wave gets
+    // kMergeRuns of them from all over the batch, whose hubs are neighbours
+    const int64_t per = (total + nwaves * kMergeRuns - 1) / (nwaves * kMergeRuns);
+    int64_t local = 0, g0 = wave * per, g1 = min(g0 + per, total);
+    int64_t t0 = g0 < total ? wave_edge_of(mpre, g0, n) : n;
+    while (g0 < total) {
+        // 64 edges: what is known of each in its lane
+        const int64_t t = t0 + lane;
+        const int64_t m0 = t < n ? mpre[t] : INT64_MAX, m1 = t < n ? mpre[t + 1] : INT64_MAX;
+        const int64_t k0 = max(m0, g0), k1 = min(m1, g1);
+        const bool mine = t < n && k0 < k1;
+        int32_t enx = 0, eny = 0;
+        int64_t exb = 0, eyb = 0;
+        if (mine) {
+            const int32_t s = pa[t], d = pb[t];
+            const int32_t ls = len[s], ld = len[d];
+            const int64_t bs = boff[s], bd = boff[d];
+            enx = min(ls, ld);
+            eny = max(ls, ld);
+            exb = ls <= ld ? bs : bd;
+            eyb = ls <= ld ? bd : bs;
         }
-        int32_t ix = __shfl(split, 0, kWave);
-        const int32_t ix1 = __shfl(split, 1, kWave);
-        int32_t iy = (int32_t)(d0 - ix);
-        const int32_t iy1 = (int32_t)min<int64_t>(d1 - ix1 + 1, ny);  // (one past iy1, inclusive)
-        uint32_t msum = 0;
-        while (ix < ix1 && iy < iy1) {
-            const int32_t cx = min(kWave, ix1 - ix), cy = min(kWave, iy1 - iy);
-            const int32_t x = lane < cx ? X[ix + lane] : INT32_MAX;
-            const int32_t y = lane < cy ? Y[iy + lane] : INT32_MAX;
-            const int32_t m = min(__shfl(x, cx - 1, kWave), __shfl(y, cy - 1, kWave));
-            int32_t r = 0;  // window entries y < x among lanes 0..62
+        for (uint64_t em = __ballot(mine); em; em &= em - 1) {
+            const int j = __ffsll((unsigned long long)em) - 1;
+            const int64_t xb = readlane_i64(exb, j), yb = readlane_i64(eyb, j);
+            const int32_t nx = __builtin_amdgcn_readlane(enx, j), ny = __builtin_amdgcn_readlane(eny, j);
+            const int64_t first = readlane_i64(m0, j), ka = readlane_i64(k0, j), kb = readlane_i64(k1, j);
+            uint32_t msum = 0;
+            int32_t ix1 = wave_split(pool + xb, nx, pool + yb, ny, (ka - first) * kMergeSeg);
+            for (int64_t k = ka; k < kb; ++k) {
+                const int64_t d0 = (k - first) * kMergeSeg, d1 = min(d0 + kMergeSeg, (int64_t)nx + ny);
+                const int32_t ix = ix1;
+                ix1 = wave_split(pool + xb, nx, pool + yb, ny, d1);
+                const int32_t iy = (int32_t)(d0 - ix);
+                const int32_t iy1 = (int32_t)min<int64_t>(d1 - ix1 + 1, ny);  // (one past the last, inclusive)
+                if (ix >= ix1 || iy >= iy1) continue;
+                const int32_t cx = ix1 - ix;  // (at most kMergeSeg)
+                const int32_t *X = pool + xb + ix;
+                // places in Y's part are counted from the aligned 16 bytes it begins in
+                const int32_t yo = (int32_t)((yb + iy) & 3), ye = yo + iy1 - iy;
+                const int32_t *Y = pool + yb + iy - yo;
+                for (int q = lane; q < 1 << (kSetBits - 7); q += kWave)
+                    reinterpret_cast<uint4 *>(set)[q] = make_uint4(0u, 0u, 0u, 0u);
+                wave_sync();
+                for (int32_t q0 = 0; q0 < ye; q0 += U * kWave) {
+                    int32_t y[U];
 #pragma unroll
-            for (int st = kWave / 2; st > 0; st >>= 1) {
-                const int32_t q = __shfl(y, r + st - 1, kWave);
-                r += (q < x) ? st : 0;
+                    for (int u = 0; u < U; ++u) {
+                        const int32_t q = q0 + u * kWave + lane;
+                        y[u] = q >= yo && q < ye ? Y[q] : -1;
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        const int32_t q = q0 + u * kWave + lane;
+                        const uint32_t h = hash(y[u]);
+                        if (y[u] >= 0) atomicOr(&set[h >> 5], 1u << (h & 31));
+                        // (the first group's mark is below any x)
+                        if (q < ye && q % kMergeGroup == 0) mark[q / kMergeGroup] = q ? y[u] : -1;
+                    }
+                }
+                wave_sync();
+                const int32_t groups = (ye + kMergeGroup - 1) / kMergeGroup;
+                auto settle = [&](int32_t m) {  // the first m of the queue, two per lane
+                    wave_sync();
+                    int32_t x[2], lo[2], hi[2], at[2];
+                    int fx[2];
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        const int32_t q = u * kWave + lane;
+                        x[u] = q < m ? qx[q] : -1;
+                        fx[u] = q < m ? flag[xb + ix + qi[q]] : 0;
+                        lo[u] = 0;
+                        hi[u] = groups - 1;
+                    }
+                    // the last group whose mark is <= x
+                    for (int32_t span = groups; span > 1; span = (span + 1) >> 1) {
+#pragma unroll
+                        for (int u = 0; u < 2; ++u) {
+                            const int32_t mid = (lo[u] + hi[u] + 1) >> 1;
+                            if (mark[mid] <= x[u]) lo[u] = mid; else hi[u] = max(mid - 1, lo[u]);
+                        }
+                    }
+                    int4 v[2][4];
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        lo[u] *= kMergeGroup;
+#pragma unroll
+                        for (int k = 0; k < 4; ++k)
+                            v[u][k] = x[u] >= 0 && lo[u] + 4 * k < ye
+                                          ? reinterpret_cast<const int4 *>(Y)[lo[u] / 4 + k]
+                                          : make_int4(-1, -1, -1, -1);
+                    }
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        at[u] = -1;
+                        auto test = [&](int32_t y, int32_t q) {
+                            if (y == x[u] && q >= yo && q < ye) at[u] = q;
+                        };
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            test(v[u][k].x, lo[u] + 4 * k);
+                            test(v[u][k].y, lo[u] + 4 * k + 1);
+                            test(v[u][k].z, lo[u] + 4 * k + 2);
+                            test(v[u][k].w, lo[u] + 4 * k + 3);
+                        }
+                        at[u] = x[u] >= 0 ? at[u] : -1;
+                    }
+                    int fy[2];
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) fy[u] = at[u] >= 0 ? flag[yb + iy - yo + at[u]] : 0;
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        if (at[u] < 0) continue;
+                        const int cw = 2 - fx[u] - fy[u];
+                        if (cw) credit(x[u], (uint32_t)cw);
+                        local += sign * cw;
+                        msum += cw == 2 ? 2u : 1u;
+                    }
+                    wave_sync();
+                };
+                int32_t held = 0;
+                for (int32_t i0 = 0; i0 < cx; i0 += U * kWave) {
+                    int32_t x[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        const int32_t i = i0 + u * kWave + lane;
+                        x[u] = i < cx ? X[i] : -1;
+                    }
+                    bool in[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        const uint32_t h = hash(x[u]);
+                        in[u] = x[u] >= 0 && ((set[h >> 5] >> (h & 31)) & 1u);
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        const uint64_t m = __ballot(in[u]);
+                        if (in[u]) {
+                            const int32_t at = held + __popcll(m & ((1ull << lane) - 1));
+                            qx[at] = x[u];
+                            qi[at] = (uint16_t)(i0 + u * kWave + lane);
+                        }
+                        held += __popcll(m);
+                        if (held >= 2 * kWave) {
+                            settle(2 * kWave);
+                            held -= 2 * kWave;
+                            if (lane < held) {
+                                qx[lane] = qx[2 * kWave + lane];
+                                qi[lane] = qi[2 * kWave + lane];
+                            }
+                        }
+                    }
+                }
+                if (held) settle(held);
             }
-            const int32_t yr = __shfl(y, r, kWave);  // (every lane takes part)
-            if (x <= m && yr == x) {
-                const int fs = flag[xb + ix + lane], fl = flag[yb + iy + r];
-                const int bs = s_short ? fs : fl, bd = s_short ? fl : fs;
-                const int cw = 2 - bs - bd;
-                if (cw) atomicAdd(&out[x], (uint32_t)(sign * cw));
-                local += sign * cw;
-                msum += (bs | bd) ? 1u : 2u;
-            }
-            ix += __popcll(__ballot(x <= m));
-            iy += __popcll(__ballot(y <= m));
+            msum = wave_sum<uint32_t>(msum);
+            if (lane == 0 && msum) atomicAdd(&ecnt[t0 + j], msum);
         }
-        msum = wave_sum<uint32_t>(msum);
-        if (lane == 0 && msum) atomicAdd(&ecnt[t], msum);
+        t0 += kWave;
+        if (readlane_i64(m1, kWave - 1) >= g1) {  // (past the last edge too) the next run
+            g0 += nwaves * per;
+            g1 = min(g0 + per, total);
+            if (g0 < total) t0 = wave_edge_of(mpre, g0, n);
+        }
+    }
+    __syncthreads();
+    for (uint32_t q = threadIdx.x; q < 1u << kCreditBits; q += kMergeThreads) {
+        const uint32_t w = S.credit[q];
+        if (w != kFree && (w & kSumMask))
+            atomicAdd(&out[merge_unhash(q << (32 - kCreditBits) | w >> kCreditBits)],
+                      (uint32_t)sign * (w & kSumMask));
     }
     const unsigned long long part[1] = {(unsigned long long)local};
     block_add_u64<1>(part, gsum);  // two's complement: a negative sum wraps
@@ -1635,7 +1852,8 @@ int run_delta(Graph &g, const int32_t *pa, const int32_t *pb, const int32_t *sel
                        g.st.pool.as<int32_t>(), g.st.boff.as<int64_t>(), g.st.len.as<int32_t>(),
                        g.flagpool.as<uint8_t>(), sign, out, ecnt, gsum);
     if (merges)
-        hipLaunchKernelGGL(k_delta_merge, dim3(dblocks), dim3(kThreads), 0, s, pa, pb, mpre, n,
+        hipLaunchKernelGGL(k_delta_merge, dim3(std::min(dblocks, kMergeBlocks)), dim3(kMergeThreads),
+                           0, s, pa, pb, mpre, n,
                            g.st.pool.as<int32_t>(), g.st.boff.as<int64_t>(), g.st.len.as<int32_t>(),
                            g.flagpool.as<uint8_t>(), sign, out, ecnt, gsum);
     hipLaunchKernelGGL(k_delta_edges, dim3(grid_for(n, 256, 4096)), dim3(256), 0, s, pa, pb, n, ecnt,
