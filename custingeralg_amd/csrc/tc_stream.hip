@@ -914,6 +914,22 @@ __device__ inline int64_t edge_of(const int64_t *__restrict__ pre, int64_t i, in
     return lo;
 }
 
+// Largest t in [0, n) with pre[t] <= i (pre[0] = 0), by the whole wave.
+__device__ inline int64_t wave_edge_of(const int64_t *__restrict__ pre, int64_t i, int64_t n)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    int64_t lo = 0;
+    while (n > 1) {
+        const int64_t step = (n + kWave - 1) / kWave;
+        const int64_t q = lane * step < n ? lane * step : 0;
+        const uint64_t m = __ballot(lane * step < n && pre[lo + q] <= i);
+        const int64_t j = m ? 63 - __clzll((long long)m) : 0;
+        lo += j * step;
+        n = min(step, n - j * step);
+    }
+    return lo;
+}
+
 // Each wave takes two chunks of 64 items per pass (c and c + the grid's wave
 // count) and runs their two binary searches interleaved, so every lane keeps
 // two independent load chains in flight.
@@ -938,10 +954,7 @@ __global__ __launch_bounds__(kThreads) void k_delta_lb(
     auto setup = [&](int64_t c, Item &it) {
         const int64_t i0 = c * kWave;
         it.ilast = min(i0 + kWave, total) - 1;
-        int64_t tb = 0;
-        if (lane == 0) tb = edge_of(pre, i0, 0, n - 1);
-        if (lane == 1) tb = edge_of(pre, it.ilast, 0, n - 1);
-        const int64_t tfirst = __shfl(tb, 0, kWave), tlast = __shfl(tb, 1, kWave);
+        const int64_t tfirst = wave_edge_of(pre, i0, n), tlast = wave_edge_of(pre, it.ilast, n);
         it.i = i0 + lane;
         it.valid = it.i <= it.ilast;
         it.t = it.valid ? edge_of(pre, it.i, tfirst, tlast) : tlast;
@@ -1051,22 +1064,6 @@ __device__ inline uint32_t merge_unhash(uint32_t h)
 #pragma unroll
     for (int k = 0; k < 4; ++k) inv *= 2u - kMergeHash * inv;
     return h * inv;
-}
-
-// Largest t in [0, n) with pre[t] <= i (pre[0] = 0), by the whole wave.
-__device__ inline int64_t wave_edge_of(const int64_t *__restrict__ pre, int64_t i, int64_t n)
-{
-    const int lane = threadIdx.x & (kWave - 1);
-    int64_t lo = 0;
-    while (n > 1) {
-        const int64_t step = (n + kWave - 1) / kWave;
-        const int64_t q = lane * step < n ? lane * step : 0;
-        const uint64_t m = __ballot(lane * step < n && pre[lo + q] <= i);
-        const int64_t j = m ? 63 - __clzll((long long)m) : 0;
-        lo += j * step;
-        n = min(step, n - j * step);
-    }
-    return lo;
 }
 
 // X entries among the first dd positions of the merge of X and Y (X first on
@@ -1846,13 +1843,15 @@ int run_delta(Graph &g, const int32_t *pa, const int32_t *pb, const int32_t *sel
         hipLaunchKernelGGL(k_zero_u32, dim3(grid_for(n, 256, 65536)), dim3(256), 0, s, ecnt, n);
     }
     // a grid by the batch size (the item total is known on the device only;
-    // the waves loop over the chunks)
-    const int dblocks = (int)std::min<int64_t>(kDeltaBlocks, std::max<int64_t>(16, n / 4));
+    // the waves loop over the chunks): two waves per edge, so that a small batch
+    // of hubs is searched in one pass of the grid (1000 pairs of 4M R-MAT vertices,
+    // four launches: n / 4 blocks 98 us, n / 2 or n 76)
+    const int dblocks = (int)std::min<int64_t>(kDeltaBlocks, std::max<int64_t>(32, n / 2));
     hipLaunchKernelGGL(k_delta_lb, dim3(dblocks), dim3(kThreads), 0, s, pa, pb, pre, n,
                        g.st.pool.as<int32_t>(), g.st.boff.as<int64_t>(), g.st.len.as<int32_t>(),
                        g.flagpool.as<uint8_t>(), sign, out, ecnt, gsum);
     if (merges)
-        hipLaunchKernelGGL(k_delta_merge, dim3(std::min(dblocks, kMergeBlocks)), dim3(kMergeThreads),
+        hipLaunchKernelGGL(k_delta_merge, dim3((int)std::min<int64_t>(kMergeBlocks, std::max<int64_t>(16, n / 4))), dim3(kMergeThreads),
                            0, s, pa, pb, mpre, n,
                            g.st.pool.as<int32_t>(), g.st.boff.as<int64_t>(), g.st.len.as<int32_t>(),
                            g.flagpool.as<uint8_t>(), sign, out, ecnt, gsum);
