@@ -1543,6 +1543,8 @@ struct PlanParams {
     int32_t lmax[3];     // owner-list capacity of each bin's kernel
     int32_t nw[3];       // wavefronts per block of each bin's kernel
     int32_t bin_max[2];  // |owner| <= bin_max[0] -> bin 0, <= bin_max[1] -> bin 1, else 2
+    // owners from wide_lo up with wide_tasks: above wide_max -> bin 2 as well
+    int32_t wide_lo, wide_max, wide_tasks;
     int32_t job_items;   // target estimated items per job (per wavefront)
     int32_t flush_items; // minimum items per owner slot in a job
     int32_t owner_end;   // owners from here up get no jobs (the core's)
@@ -1562,9 +1564,10 @@ __device__ inline int32_t est_items(int32_t L, int32_t pl)
     return (int32_t)min<int64_t>(pl, bs) + 4;
 }
 
-__device__ inline int owner_bin(int32_t L, const PlanParams &P)
+__device__ inline int owner_bin(int32_t v, int32_t L, int32_t tasks, const PlanParams &P)
 {
-    return L <= P.bin_max[0] ? 0 : (L <= P.bin_max[1] ? 1 : 2);
+    const bool wide = v >= P.wide_lo && L > P.wide_max && tasks >= P.wide_tasks;
+    return L <= P.bin_max[0] ? 0 : (L <= P.bin_max[1] && !wide ? 1 : 2);
 }
 
 // Per-owner estimated work (sum over its tasks); per-bin stats.
@@ -1613,7 +1616,7 @@ __global__ __launch_bounds__(kWorkThreads) void k_owner_work(const int64_t *__re
                 }
                 if (ok) {
                     w = (uint32_t)est_items(min(L, P.lmax[2]), pl);
-                    const int bin = owner_bin(L, P);
+                    const int bin = owner_bin(b, L, ORIENTED ? vb.dm : vb.len, P);
 #pragma unroll
                     for (int q = 0; q < 3; ++q)
                         if (bin == q) {
@@ -1700,7 +1703,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan_jobs(
         const int32_t L = ORIENTED ? x.len - x.dm : x.len;
         T[k] = ORIENTED ? x.dm : x.len;
         if (L <= 0 || T[k] <= 0 || w == 0 || (!ORIENTED && x.len < 2)) continue;
-        bin[k] = owner_bin(L, P);
+        bin[k] = owner_bin((int32_t)v, L, T[k], P);
         const int64_t tiles = owner_tiles(L, bin[k], P);
         const int64_t per_tile = (int64_t)(w / (unsigned long long)tiles) + 1;
         // a job amortises building its LDS table and, at its end, the flush of
@@ -2925,6 +2928,9 @@ tc_schedule default_schedule()
 namespace {
 
 constexpr int kL0 = 64, kL1 = 512, kL2 = 4096;
+// (the ranks that k_count_long's bitmap holds, its guard word left)
+constexpr int32_t kWideMin = 128, kWideTasks = 64, kWideSpan = (kL2 - 1) * 32;
+constexpr int64_t kWideNnz = int64_t(3) << 24;
 // owners of at least this degree get their task lists from their own rows
 // (k_orient_transpose_hubs) instead of by appends
 constexpr int kHubDegree = 65536;  // with the appends
@@ -3552,6 +3558,25 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     P.job_items = std::max(sched.job_items, 256);
     P.flush_items = sched.flush_items > 0 ? sched.flush_items : 1024;
     P.owner_end = nv - (oriented ? g.core_k : 0);
+    // Owners whose rows fit k_count_long's bitmap by their rank (a row of N+ spans
+    // at most the ranks above its owner) go to the largest bin from kWideMin
+    // entries on: it streams 1300 G entries a second against the mid bin's 440,
+    // whose bitmap holds an eighth of the ranks, and hash tables beyond (3M ragged
+    // vertices 12.2 -> 10.3 ms; 96, 192, 256, 384 entries: 10.3, 10.3, 10.6, 10.7).
+    // Its jobs of eight waves need a large graph to fill the chip: R-MAT graphs of
+    // 8M to 48M entries took 1.01 to 1.12 times as long, of 63M and more 0.84 to
+    // 0.96.  Without enough tasks the bitmap is not repaid; the largest bin's hash
+    // tables are no gain either (R-MAT 24 with all rows from 256 on 131 -> 149 ms),
+    // nor are batched graphs, whose cores lie behind all other ranks.
+    P.wide_lo = INT32_MAX;
+    P.wide_max = P.bin_max[1];
+    P.wide_tasks = kWideTasks;
+    if (oriented && !g.batch_voff && nnz >= kWideNnz && P.bin_max[1] > kWideMin &&
+        (sched.policy == TC_POLICY_HASH || sched.policy == TC_POLICY_LEARNED ||
+         (sched.policy == TC_POLICY_FIXED && sched.ratio_x16 <= 0 && sched.mpath_min <= 0))) {
+        P.wide_lo = std::max(nv - kWideSpan, 0);
+        P.wide_max = kWideMin;
+    }
     // by tasks: bit rows hold any list whole, and a job of theirs ends without a
     // flush.  Beyond kBitsIds1 ids a row is tiled by id range, which pays for
     // the largest bin only (the mid bin's lists go through LDS tables).
@@ -3582,10 +3607,10 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
                           : g.validated && !g.degree_stale ? g.max_degree : nv;
     JobArrays J = {};
     const int64_t owners[3] = {nv, std::min<int64_t>(nv, lists / (P.bin_max[0] + 1)),
-                               std::min<int64_t>(nv, lists / (P.bin_max[1] + 1))};
+                               std::min<int64_t>(nv, lists / (P.wide_max + 1))};
     int64_t total_cap = 0;
     for (int b = 0; b < 3; ++b) {
-        const bool any = b == 0 || lmost > P.bin_max[b - 1];
+        const bool any = b == 0 || lmost > (b == 1 ? P.bin_max[0] : P.wide_max);
         const double more = (double)lists * (double)(lmost + 4) / ((double)P.job_items * P.nw[b]);
         J.cap[b] = any ? owners[b] + 64 + (int64_t)std::min(more, 2097152.0) : 0;
         if (b == 2 && any) J.cap[b] += P.id_tiles > 0 ? owners[b] * P.id_tiles : 2 * (lists / P.lmax[2]);

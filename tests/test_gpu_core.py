@@ -121,3 +121,23 @@ def test_batched_cores(sizes):
         assert np.array_equal(pv.to_host(), ref)
         assert np.array_equal(pg.to_host(), want)
     bg.close()
+
+
+def test_rows_of_129_to_512_in_the_largest_bin():
+    """A graph large enough that rows of the middle bin's lengths near the top of
+    the rank order go to the largest one: schedules that bin them otherwise
+    agree."""
+    off, adj = O.rmat_graph(21, 16, 5)
+    assert len(adj) >= 3 << 24
+    g = T.cuStinger(off, adj, assume_symmetric=True)
+    a, ga, sa = T.static_count(g, T.default_schedule())
+    b, gb, sb = T.static_count(g, T.default_schedule(mid_max=128))
+    h, gh, _ = T.static_count(g, T.default_schedule(policy=T.POLICY_HASH))
+    m, gm, _ = T.static_count(g, T.default_schedule(mpath_min=1 << 20))  # (kept in the middle bin)
+    g.close()
+    for x, gx in ((b, gb), (h, gh), (m, gm)):
+        assert np.array_equal(a, x) and ga == gx
+    assert int(a.astype(np.uint64).sum()) == ga
+    assert sum(sa["tasks_bin"]) == sum(sb["tasks_bin"]) and 0 < sa["tasks_bin"][2] <= sb["tasks_bin"][2]
+    total, _ = O.forward_count(off, adj)
+    assert ga == 6 * total
