@@ -20,11 +20,16 @@ namespace {
 constexpr int kGroup = 8;                    // lanes per bit row: 128 bytes a load
 constexpr int kGroups = kWave / kGroup;
 constexpr int kCoreCols = kGroup * 4 * 32;   // columns per such load
-// Columns: 4096 for one graph (2 MB of bit rows, an XCD's L2 holds them),
+// Columns: 4096 for one graph (2 MB of bit rows, an XCD's L2 holds them), 8192 (8
+// MB) from 200M entries on, where the lists that they take the place of are the
+// longer part: R-MAT 24 (edge factor 16) 131.5 -> 125.8 ms, 4M vertices with edge
+// factor 32 22.6 -> 21.4, with 16 (130M entries) 10.9 -> 11.0, 1M 2.85 -> 2.90.
 // 2048 for each of batched graphs (1024 graphs of 1k to 64k vertices: 24.2 ms
 // a count, against 26.2 with 1024, 25.5 with 3072 and 26.3 with 4096, whose
 // matrices cost more to build)
 constexpr int kCoreOne = 4, kCoreBatch = 2;  // loads per lane and bit row
+constexpr int kCoreLarge = 8;
+constexpr int64_t kCoreLargeNnz = int64_t(3) << 26;
 constexpr int kCoreThreads = 512;
 constexpr int kCoreWaves = kCoreThreads / kWave;
 constexpr int kGroupRow = 16;                // rows of S(a) up to this long go four to a wave
@@ -314,7 +319,7 @@ __device__ inline unsigned long long core_rows(CoreShared<Q> &S, const CoreArgs 
 // block.  Bound by L2 reads of bit rows (2 MB for 4096 columns: an XCD's L2
 // holds all of it; 18.7 TB/s at R-MAT 24).
 template <int Q>
-__global__ __launch_bounds__(kCoreThreads, Q <= 2 ? 7 : 6) void k_core_count(CoreArgs A)
+__global__ __launch_bounds__(kCoreThreads, Q <= 2 ? 7 : Q <= 4 ? 6 : 2) void k_core_count(CoreArgs A)
 {
     __shared__ CoreShared<Q> S;
     if (*A.fault) return;  // (set before this kernel: the same for all)
@@ -467,7 +472,8 @@ int32_t core_size(const Graph &g, const tc_schedule &sched)
         sched.mpath_min > 0 || sched.hub_degree > 0 || sched.build != 0)
         return 0;
     if (g.batch_voff) return g.core_total;
-    return g.st.nv > 4 * kCoreOne * kCoreCols ? kCoreOne * kCoreCols : 0;
+    const int32_t k = (g.st.nnz >= kCoreLargeNnz ? kCoreLarge : kCoreOne) * kCoreCols;
+    return g.st.nv > 4 * k ? k : 0;
 }
 
 namespace {
@@ -518,9 +524,10 @@ int core_count(Graph &g, unsigned long long *acc, int32_t *bad, const int32_t *g
     int dev = 0, cus = 0;
     TC_HIP(hipGetDevice(&dev));
     TC_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    return core_launch<kCoreOne>(g, A, bad, nullptr,
-                                 std::min<int64_t>(ceil_div(nv, kCoreThreads),
-                                                   std::max<int64_t>(3 * cus, ceil_div(nv, 1 << 15))));
+    const int64_t grid = std::min<int64_t>(ceil_div(nv, kCoreThreads),
+                                           std::max<int64_t>(3 * cus, ceil_div(nv, 1 << 15)));
+    return k > kCoreOne * kCoreCols ? core_launch<kCoreLarge>(g, A, bad, nullptr, grid)
+                                    : core_launch<kCoreOne>(g, A, bad, nullptr, grid);
 }
 
 }  // namespace tc

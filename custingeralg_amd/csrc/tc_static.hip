@@ -1778,17 +1778,17 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan_jobs(
 
 // outr[r] += 2 * (sum of pcnt over N+(r)): the task-vertex share of the
 // oriented count, one segmented wave sum per 64 entries of the plus array.
-// HUBS: the entries that point to the last hubs ranks hold third-vertex hits
-// (k_count) and are credited to that rank instead, summed in LDS.  Those ranks
+// HUBS > 0: the entries that point to the last hubs (at most HUBS) ranks hold
+// third-vertex hits (k_count) and are credited to that rank instead, summed in
+// LDS.  Those ranks
 // are what most lists end in: credited from k_count one by one, their few cache
 // lines were much of its middle bin (R-MAT 20 1460 -> 850 us, 3M ragged vertices
 // 5690 -> 5300; R-MAT 24, where fewer third vertices are hubs, 15.4 ms either
 // way), for one more read of the entries here.  Not for batched graphs: each has
 // hubs of its own, too many for one block's sums.
 constexpr int kSumThreads = 512;
-constexpr int32_t kSumHubs = 4096;
 
-template <bool HUBS>
+template <int32_t HUBS>
 __global__ __launch_bounds__(kSumThreads) void k_plus_row_sum(const int64_t *__restrict__ pcoff,
                                                               const int32_t *__restrict__ pcrow,
                                                               const int32_t *__restrict__ padj,
@@ -1798,7 +1798,7 @@ __global__ __launch_bounds__(kSumThreads) void k_plus_row_sum(const int64_t *__r
                                                               const int32_t *__restrict__ asym)
 {
     if (*asym) return;
-    __shared__ uint32_t hub[HUBS ? kSumHubs : 1];
+    __shared__ uint32_t hub[HUBS ? HUBS : 1];
     const int32_t hub_lo = nv - hubs;
     if (HUBS) {
         for (int q = threadIdx.x; q < hubs; q += blockDim.x) hub[q] = 0u;
@@ -3640,7 +3640,7 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     A.toff = mode != kDirect ? coff : nullptr;
     A.cred = mode == kByTasks ? g.ov[16].as<int32_t>() : nullptr;
     A.nv = nv;
-    const int32_t hubs = oriented && !g.batch_voff && g.core_k <= kSumHubs ? g.core_k : 0;
+    const int32_t hubs = oriented && !g.batch_voff && g.core_k <= 8192 ? g.core_k : 0;
     A.hub_lo = hubs > 0 ? nv - hubs : INT32_MAX;
     A.order = oriented ? g.order.as<int32_t>() : nullptr;
     A.out = outp;
@@ -3695,7 +3695,7 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     if (oriented && nplus > 0) {
         // (hubs: blocks of 16K entries at least, so that the sums of a block are
         // worth adding up)
-        const auto sum = hubs > 0 ? k_plus_row_sum<true> : k_plus_row_sum<false>;
+        const auto sum = hubs == 0 ? k_plus_row_sum<0> : hubs <= 4096 ? k_plus_row_sum<4096> : k_plus_row_sum<8192>;
         const int64_t per = hubs > 0 ? 16384 : kSumThreads;
         hipLaunchKernelGGL(sum, dim3(grid_for(nplus, per, hubs > 0 ? 1024 : 32768)), dim3(kSumThreads), 0, s,
                            g.ov[6].as<int64_t>(), g.ov[10].as<int32_t>(), g.padj.as<int32_t>(),

@@ -141,3 +141,14 @@ def test_rows_of_129_to_512_in_the_largest_bin():
     assert sum(sa["tasks_bin"]) == sum(sb["tasks_bin"]) and 0 < sa["tasks_bin"][2] <= sb["tasks_bin"][2]
     total, _ = O.forward_count(off, adj)
     assert ga == 6 * total
+
+
+def test_core_of_the_largest_graphs():
+    """From 200M entries on the core has 8192 ranks; a forced policy has none."""
+    g = T.rmat_graph_device(22, 28, 7)
+    assert g.info()["nnz"] >= 3 << 26
+    a, ga, _ = T.static_count(g, T.default_schedule())
+    h, gh, _ = T.static_count(g, T.default_schedule(policy=T.POLICY_HASH))
+    g.close()
+    assert np.array_equal(a, h) and ga == gh
+    assert ga % 6 == 0
