@@ -1479,13 +1479,12 @@ __device__ inline DirectEntry direct_entry(const int64_t *__restrict__ coff, con
     return d;
 }
 
-// WRITE = false: cnt[x] = tasks of owner x (zero on entry), and every entry's
-// place among them to place[e], if given.  WRITE = true: the tasks themselves,
-// at those places, or (place null: 4 bytes an entry did not fit) with cnt as the
-// cursors, zero on entry.  A row's own tasks in a chunk take one atomic; the
-// others one each, and those are what bounds a pass: written at places kept from
-// the first one, the second takes 62 us instead of 195 (4M entries, 2^18 R-MAT
-// vertices).
+// WRITE = false: cnt[x] = tasks of owner x (zero on entry).  WRITE = true: the
+// tasks themselves, at the places of k_direct_places, or (place null: 4 bytes an
+// entry did not fit) with cnt as the cursors, zero on entry.  With cursors a row's
+// own tasks in a chunk take one atomic and the others one each, and those are what
+// bounds a pass: at known places it takes 62 us instead of 195 (4M entries, 2^18
+// R-MAT vertices).
 constexpr uint32_t kNoTask = 0xFFFFFFFFu;
 template <bool WRITE>
 __global__ void k_direct_tasks(const int64_t *__restrict__ coff, const int32_t *__restrict__ crow,
@@ -1526,13 +1525,95 @@ __global__ void k_direct_tasks(const int64_t *__restrict__ coff, const int32_t *
             slot = __shfl(slot, s0, kWave) + __popcll(mine & lt);
             if (other) slot = atomicAdd(&cnt[direct_slot(d.owner, mask)], 1);
             at = d.ok ? 2u * (uint32_t)slot + own : kNoTask;
-            if (!WRITE && place && e < nnz) place[e] = at;
         }
         if (WRITE && d.ok) {
             const int64_t p = toff[d.owner] + (at >> 1);
             tasks[p] = TaskRec::make(boff[d.list], len[d.list]);
             cred[p] = v;
         }
+    }
+}
+
+// cnt[x] = tasks of owner x (zero on entry), place[e] = 2 * (entry e's place among
+// them) + (whether it is its own row's task), or kNoTask.  A block first counts
+// the tasks of the owners of its 4096 entries in a table in LDS and then adds each
+// owner's sum to its counter: an atomic per task on the hubs' counters took 190 us
+// (4M entries, 2^18 R-MAT vertices), this 82.
+constexpr int kPlaceThreads = 1024, kPlaceChunks = 4;
+constexpr int kPlaceTile = kPlaceThreads * kPlaceChunks, kPlaceBits = 13;
+
+__global__ __launch_bounds__(kPlaceThreads) void k_direct_places(
+    const int64_t *__restrict__ coff, const int32_t *__restrict__ crow, const int64_t *__restrict__ boff,
+    const int32_t *__restrict__ len, const int32_t *__restrict__ pool, int32_t nv, int64_t nnz, int skip_lower,
+    int32_t *__restrict__ cnt, uint32_t mask, uint32_t *__restrict__ place)
+{
+    static_assert((1 << kPlaceBits) >= 2 * kPlaceTile, "half of the table stays empty");
+    constexpr int U = kPlaceChunks, W = kPlaceThreads / kWave;
+    __shared__ int32_t key[1 << kPlaceBits];
+    __shared__ uint32_t sum[1 << kPlaceBits];
+    const int t = threadIdx.x, lane = t & (kWave - 1), wid = t / kWave;
+    const int64_t nchunks = ceil_div(nnz, kWave), ntiles = ceil_div(nnz, kPlaceTile);
+    const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
+    auto slot_of = [&](int32_t x) {
+        uint32_t h = ((uint32_t)x * 0x9E3779B1u) >> (32 - kPlaceBits);
+        for (;;) {
+            const int32_t k = atomicCAS(&key[h], -1, x);
+            if (k == -1 || k == x) return h;
+            h = (h + 1) & ((1u << kPlaceBits) - 1);
+        }
+    };
+    for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        for (int q = t; q < 1 << kPlaceBits; q += kPlaceThreads) {
+            key[q] = -1;
+            sum[q] = 0u;
+        }
+        __syncthreads();
+        uint32_t at[U], loc[U];  // (slot * 2 + the row's own task), place among the tile's of the owner
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t c = (tile * W + wid) * U + u;
+            at[u] = kNoTask;
+            loc[u] = 0;
+            if (c >= nchunks) continue;  // (the whole wave)
+            const int32_t v = wave_row_of(coff, crow, nv, c, nnz);
+            const DirectEntry d = direct_entry(coff, boff, len, pool, v, c * kWave + lane, nnz, skip_lower);
+            const bool own = d.ok && d.owner == v;
+            // the lanes of this lane's row (rows are runs of lanes)
+            const int32_t before = __shfl_up(v, 1, kWave);
+            const uint64_t starts = __ballot(lane == 0 || before != v);
+            const int s0 = 63 - __clzll((long long)(starts & (lt | (1ull << lane))));
+            const uint64_t after = starts & ~(lt | (1ull << lane));
+            const int s1 = after ? __ffsll((unsigned long long)after) - 1 : kWave;
+            const uint64_t seg = (s1 == kWave ? ~0ull : (1ull << s1) - 1) & ~((1ull << s0) - 1);
+            const uint64_t mine = __ballot(own) & seg;
+            // a row's own tasks by the row's first lane, the others one by one
+            const bool first = lane == s0 && mine;
+            uint32_t h = 0, l = 0;
+            if (first) {
+                h = slot_of(v);
+                l = atomicAdd(&sum[h], (uint32_t)__popcll(mine));
+            }
+            const uint32_t rh = __shfl(h, s0, kWave), rl = __shfl(l, s0, kWave);
+            if (own) {
+                h = rh;
+                l = rl + (uint32_t)__popcll(mine & lt);
+            } else if (d.ok) {
+                h = slot_of(d.owner);
+                l = atomicAdd(&sum[h], 1u);
+            }
+            at[u] = d.ok ? 2u * h + own : kNoTask;
+            loc[u] = l;
+        }
+        __syncthreads();
+        for (int q = t; q < 1 << kPlaceBits; q += kPlaceThreads)
+            if (sum[q]) sum[q] = (uint32_t)atomicAdd(&cnt[direct_slot(key[q], mask)], (int32_t)sum[q]);
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t e = ((tile * W + wid) * U + u) * kWave + lane;
+            if (e < nnz) place[e] = at[u] == kNoTask ? kNoTask : 2u * (sum[at[u] >> 1] + loc[u]) + (at[u] & 1u);
+        }
+        __syncthreads();
     }
 }
 
@@ -3400,8 +3481,12 @@ int prepare_direct_tasks(Graph &g, bool skip_lower)
     const int32_t *crow = g.crow.as<int32_t>(), *len = g.st.len.as<int32_t>(), *pool = g.st.pool.as<int32_t>();
     hipLaunchKernelGGL(k_fill_u32, dim3(vblocks), dim3(256), 0, s, reinterpret_cast<uint32_t *>(cnt),
                        (int64_t)slots, 0u);
-    hipLaunchKernelGGL(k_direct_tasks<false>, dim3(wblocks), dim3(256), 0, s, coff, crow, boff, len, pool, nv, nnz,
-                       skip_lower ? 1 : 0, cnt, mask, place, nullptr, nullptr, nullptr);
+    if (place)
+        hipLaunchKernelGGL(k_direct_places, dim3(grid_for(nnz, kPlaceTile, 512)), dim3(kPlaceThreads), 0, s, coff,
+                           crow, boff, len, pool, nv, nnz, skip_lower ? 1 : 0, cnt, mask, place);
+    else
+        hipLaunchKernelGGL(k_direct_tasks<false>, dim3(wblocks), dim3(256), 0, s, coff, crow, boff, len, pool, nv,
+                           nnz, skip_lower ? 1 : 0, cnt, mask, place, nullptr, nullptr, nullptr);
     TC_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_direct_task_vinfo, dim3(vblocks), dim3(256), 0, s, boff, len, cnt, mask, nv,
                        g.vinfo.as<VInfo>(), tcnt);

@@ -81,3 +81,28 @@ def test_batched_asymmetric():
     assert st["method_used"] == T.METHOD_DIRECT
     assert np.array_equal(pv, ref)
     assert np.array_equal(pg, np.add.reduceat(ref.astype(np.uint64), voff[:-1]))
+
+
+@pytest.mark.parametrize("entries", [1, 63, 65, 4095, 4096, 4097, 8192, 20481])
+@pytest.mark.parametrize("owners", ["one", "all different"])
+def test_places_around_the_tiles(entries, owners):
+    """Entry counts around the 4096 whose owners a block counts together: tasks
+    of one owner only, and of as many as there are entries."""
+    n = 70000
+    rng = np.random.default_rng(entries)
+    if owners == "one":  # rows of two entries, both to vertices with longer rows
+        src = np.repeat(np.arange(10, 10 + (entries + 1) // 2), 2)[:entries]
+        dst = np.tile([3, 4], (entries + 1) // 2)[:entries]
+        hub = np.repeat([3, 4], 5)
+        key = np.unique(np.concatenate([src * n + dst, hub * n + np.tile(np.arange(60000, 60005), 2)]))
+    else:
+        src = rng.choice(n, entries, replace=False)
+        dst = (src + rng.integers(1, n, entries)) % n
+        key = np.unique(np.concatenate([src * n + dst, src * n + (src + 1) % n]))
+    off = np.concatenate([[0], np.cumsum(np.bincount(key // n, minlength=n))]).astype(np.int64)
+    adj = (key % n).astype(np.int32)
+    ref = O.custinger_count(off, adj)
+    g = T.cuStinger(off, adj)
+    pv, glob, st = T.static_count(g, T.default_schedule(method=T.METHOD_DIRECT))
+    g.close()
+    assert np.array_equal(pv, ref) and glob == int(ref.astype(np.uint64).sum())
