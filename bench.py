@@ -232,8 +232,8 @@ def bench_static(T, args) -> dict:
     # the dominant count kernel by event time: the small and mid bins' kernels,
     # or the largest bin's hash-task kernel on bitmap / hash-table tiles (the
     # rest of the largest bin is a short pass over its other tasks)
-    kernels = [("k_count<64,1,true> (bin 0)", st["ms_bin"][0], st["stream_bytes_bin"][0]),
-               ("k_count<512,2,true> (bin 1)", st["ms_bin"][1], st["stream_bytes_bin"][1]),
+    kernels = [("k_count<64,1,1> (bin 0)", st["ms_bin"][0], st["stream_bytes_bin"][0]),
+               ("k_count<512,2,1> (bin 1)", st["ms_bin"][1], st["stream_bytes_bin"][1]),
                ("k_count_long<4096,8,true> (bin 2, bitmap tiles)", st["ms_long"][0],
                 st["stream_bytes_long"][0]),
                ("k_count_long<4096,8,false> (bin 2, hash-table tiles)", st["ms_long"][1],

@@ -131,7 +131,8 @@ typedef struct {
     int32_t method;        /* TC_METHOD_*                                           */
     int32_t policy;        /* TC_POLICY_*                                           */
     int32_t small_max;     /* rows with |N+| <= small_max use one wave per job      */
-    int32_t mid_max;       /* rows with |N+| <= mid_max use the mid bin              */
+    int32_t mid_max;       /* rows with |N+| <= mid_max use the mid bin (on large     */
+                           /*   graphs, the largest where its bitmap suits them)     */
     int32_t job_items;     /* target items per job (prefix-sum partition grain)      */
     int32_t ratio_x16;     /* fixed heuristic: merge when long*16 <= short*ratio_x16 */
                            /*   and long <= 96 (0, the default: never merge)         */
@@ -166,6 +167,9 @@ typedef struct {
     double ms_count;        /* intersection kernels                           */
     double ms_bin[4];       /* per bin (small, mid, large, direct)            */
     double bytes_alg_bin[4];/* algorithmic bytes 4*(L_u+L_v) per bin          */
+    /* Task, job and byte counters are of the task lists: a count (or the part of
+       it) that runs on bit rows or row by row has none, and is in ms_count only.
+       Direct counts keep all rows above the small bin in bin 2. */
     int64_t tasks_bin[4];   /* intersection tasks per bin                     */
     int64_t jobs_bin[4];
     int64_t strategy_tasks[3]; /* tasks run as merge / bsearch / hash         */
