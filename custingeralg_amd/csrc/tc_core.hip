@@ -100,33 +100,89 @@ __global__ __launch_bounds__(256) void k_core_rows(const VInfo *__restrict__ vi,
     }
 }
 
-// The lower half: every 64 x 64 block on or above the diagonal is transposed
-// in registers (lane = row) and stored below it.  The waves of a graph's nblk
-// thread blocks take its bit blocks in turn.
-template <int Q>
-__global__ __launch_bounds__(256) void k_core_transpose(CoreGraph one, const CoreGraph *__restrict__ graphs,
-                                                        int32_t nblk, uint32_t *__restrict__ mat)
+// A 64 x 64 block of bits, a row per lane, transposed.
+__device__ inline uint64_t transpose_64(uint64_t x)
 {
     const int lane = threadIdx.x & (kWave - 1);
-    const CoreGraph D = graphs ? graphs[blockIdx.x / nblk] : one;
+    auto step = [&](int s, uint64_t m0) {
+        const uint64_t y = shfl_xor_u64(x, s);
+        x = (lane & s) == 0 ? (x & m0) | ((y & m0) << s) : (x & ~m0) | ((y & ~m0) >> s);
+    };
+    step(32, 0x00000000FFFFFFFFull);
+    step(16, 0x0000FFFF0000FFFFull);
+    step(8, 0x00FF00FF00FF00FFull);
+    step(4, 0x0F0F0F0F0F0F0F0Full);
+    step(2, 0x3333333333333333ull);
+    step(1, 0x5555555555555555ull);
+    return x;
+}
+
+// The lower half: every 64 x 64 block on or above the diagonal is transposed
+// in registers (lane = row) and stored below it.  One graph: its few blocks are
+// dealt to all waves (7 us with 4096 ranks, 36 as below).
+template <int Q>
+__global__ __launch_bounds__(256) void k_core_transpose(CoreGraph D, uint32_t *__restrict__ mat)
+{
+    const int lane = threadIdx.x & (kWave - 1);
     constexpr int32_t stride = Q * (kCoreCols / 64);
     uint64_t *m = reinterpret_cast<uint64_t *>(mat) + (int64_t)D.kpre * stride;
     const int32_t k = D.k, nb = (k + 63) / 64;
-    const int32_t wpb = blockDim.x / kWave, nw = nblk * wpb;
-    for (int32_t q = (int32_t)(blockIdx.x % nblk) * wpb + threadIdx.x / kWave; q < nb * nb; q += nw) {
+    const int32_t wpb = blockDim.x / kWave, nw = (int32_t)gridDim.x * wpb;
+    for (int32_t q = (int32_t)blockIdx.x * wpb + threadIdx.x / kWave; q < nb * nb; q += nw) {
         const int32_t i = q / nb, j = q % nb;
         if (j < i) continue;
         const int32_t ri = 64 * i + lane, rj = 64 * j + lane;
         const uint64_t x0 = ri < k ? m[(int64_t)ri * stride + j] : 0ull;
-        uint64_t x = x0;
-        for (int s = 32; s > 0; s >>= 1) {
-            const uint64_t m0 = s == 32 ? 0x00000000FFFFFFFFull : s == 16 ? 0x0000FFFF0000FFFFull
-                              : s == 8 ? 0x00FF00FF00FF00FFull : s == 4 ? 0x0F0F0F0F0F0F0F0Full
-                              : s == 2 ? 0x3333333333333333ull : 0x5555555555555555ull;
-            const uint64_t y = shfl_xor_u64(x, s);
-            x = (lane & s) == 0 ? (x & m0) | ((y & m0) << s) : (x & ~m0) | ((y & ~m0) >> s);
-        }
+        const uint64_t x = transpose_64(x0);
         if (rj < k) m[(int64_t)rj * stride + i] = i == j ? x | x0 : x;
+    }
+}
+
+// Batched graphs: a 1024 x 1024 block of bits per thread block, wave i the 64 x 64
+// blocks of its 64 rows, and the results go through LDS, so that rows are read and
+// written as whole 128-byte lines (1024 cores: 8 bytes of a line at a time 0.88
+// ms, this 0.39).
+template <int Q>
+__global__ __launch_bounds__(1024) void k_core_transpose_batch(const CoreGraph *__restrict__ graphs,
+                                                               uint32_t *__restrict__ mat)
+{
+    constexpr int W = kCoreCols / 64;              // words of such a block's row
+    constexpr int kPairs = Q * (Q + 1) / 2;        // blocks on or above the diagonal
+    static_assert(W == 16, "a wave per 64 rows");
+    __shared__ uint64_t tile[kCoreCols][W + 1];
+    const int t = threadIdx.x, lane = t & (kWave - 1), wid = t / kWave;
+    const CoreGraph D = graphs[blockIdx.x / kPairs];
+    int I = 0, J = (int)(blockIdx.x % kPairs);
+    while (J >= Q - I) J -= Q - I++;
+    J += I;
+    constexpr int32_t stride = Q * W;
+    uint64_t *m = reinterpret_cast<uint64_t *>(mat) + (int64_t)D.kpre * stride;
+    const int32_t k = D.k;
+    if (J * kCoreCols >= k) return;  // (the whole block: no such rows or columns)
+    const int32_t r = I * kCoreCols + 64 * wid + lane;
+    uint64_t x[W];
+    const ulonglong2 *src = reinterpret_cast<const ulonglong2 *>(m + (int64_t)(r < k ? r : 0) * stride + J * W);
+#pragma unroll
+    for (int j = 0; j < W; j += 2) {
+        const ulonglong2 v = r < k ? src[j / 2] : make_ulonglong2(0ull, 0ull);
+        x[j] = v.x;
+        x[j + 1] = v.y;
+    }
+#pragma unroll
+    for (int j = 0; j < W; ++j) {
+        if (I == J && j < wid) continue;  // (below the diagonal: the whole wave)
+        const uint64_t y = transpose_64(x[j]);
+        tile[64 * j + lane][wid] = I == J && j == wid ? y | x[j] : y;
+    }
+    __syncthreads();
+    for (int q = t; q < kCoreCols * W / 2; q += 1024) {
+        const int row = q / (W / 2), c = 2 * (q % (W / 2)), last = I == J ? row / 64 : W - 1;
+        if (J * kCoreCols + row >= k || c > last) continue;
+        uint64_t *dst = m + (int64_t)(J * kCoreCols + row) * stride + I * W + c;
+        if (c < last)
+            *reinterpret_cast<ulonglong2 *>(dst) = make_ulonglong2(tile[row][c], tile[row][c + 1]);
+        else
+            *dst = tile[row][c];
     }
 }
 
@@ -488,11 +544,13 @@ int core_launch(Graph &g, CoreArgs A, int32_t *bad, const int32_t *gid, int64_t 
     uint32_t *mat = g.cmat.as<uint32_t>();
     A.mat = mat;
     A.pcount = mat + words;
-    const int32_t graphs = A.graphs ? g.batch_ngraphs : 1, nblk = A.graphs ? 8 : 512;
     hipLaunchKernelGGL(k_core_rows<Q>, dim3(grid_for(k, 4)), dim3(256), 0, s, A.vi, A.padj, A.core_lo, k, A.one,
                        A.graphs, gid, mat, A.pcount, A.fault);
-    hipLaunchKernelGGL(k_core_transpose<Q>, dim3((unsigned)(nblk * (int64_t)graphs)), dim3(256), 0, s, A.one,
-                       A.graphs, nblk, mat);
+    if constexpr (Q == kCoreBatch)
+        hipLaunchKernelGGL(k_core_transpose_batch<Q>, dim3((unsigned)((int64_t)g.batch_ngraphs * (Q * (Q + 1) / 2))),
+                           dim3(1024), 0, s, A.graphs, mat);
+    else
+        hipLaunchKernelGGL(k_core_transpose<Q>, dim3(512), dim3(256), 0, s, A.one, mat);
     hipLaunchKernelGGL(k_core_count<Q>, dim3((unsigned)grid), dim3(kCoreThreads), 0, s, A);
     hipLaunchKernelGGL(k_core_check, dim3(grid_for(k, 256)), dim3(256), 0, s, A.vi, A.core_lo, k, A.pcount, bad);
     TC_HIP(hipGetLastError());
