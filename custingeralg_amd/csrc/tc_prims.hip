@@ -330,7 +330,7 @@ __global__ __launch_bounds__(1024) void k_sort_reg(uint64_t *__restrict__ keys, 
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int i0 = 128 * w + lane, i1 = i0 + 64;
     uint64_t v0 = i0 < n ? keys[i0] : ~0ull, v1 = i1 < n ? keys[i1] : ~0ull;
-    block_bitonic_2048(v0, v1, buf);
+    block_bitonic_2048(v0, v1, buf, n);
     if (i0 < n) keys[i0] = v0;
     if (i1 < n) keys[i1] = v1;
 }

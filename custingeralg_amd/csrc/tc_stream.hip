@@ -1572,7 +1572,7 @@ __global__ __launch_bounds__(1024) void k_small_front(
     uint64_t v0 = key(i0), v1 = key(i1);
     const unsigned long long part[1] = {nd};
     block_add_u64<1>(part, ndel);
-    block_bitonic_2048(v0, v1, buf);
+    block_bitonic_2048(v0, v1, buf, Bc);
     buf[0][i0] = v0;
     buf[0][i1] = v1;
     __syncthreads();
@@ -1671,7 +1671,7 @@ __global__ __launch_bounds__(1024) void k_small_insert(
     __syncthreads();
     uint64_t v0 = buf[0][i0], v1 = buf[0][i1];
     __syncthreads();
-    block_bitonic_2048(v0, v1, buf);
+    block_bitonic_2048(v0, v1, buf, nd);
     if (i0 < B2) dk[i0] = v0;
     if (i1 < B2) dk[i1] = v1;
     buf[0][i0] = v0;

@@ -82,3 +82,34 @@ def test_one_vertex_in_every_list():
     bu, bv = _new_pairs(n, off, adj, a[keep], b[keep])
     assert len(bu) > 1_000_000
     _insert_and_undo(n, off, adj, bu, bv)
+
+
+@pytest.mark.parametrize("pairs", [1, 2, 31, 63, 64, 65, 127, 128, 129, 256, 257, 511, 513, 1023, 1024])
+@pytest.mark.parametrize("capture", [0, 1])
+def test_small_batches_of_every_sort_size(pairs, capture):
+    """Batches whose pairs, and whose directed entries, fill the one-block sort
+    up to and past each power of two."""
+    n = 3000
+    rng = np.random.default_rng(pairs)
+    off, adj = O.canon_csr(n, rng.integers(0, n, 9 * n).astype(np.int32), rng.integers(0, n, 9 * n).astype(np.int32))
+    bu, bv = _new_pairs(n, off, adj, rng.integers(0, n, 4 * pairs + 8), rng.integers(0, n, 4 * pairs + 8))
+    pick = rng.permutation(len(bu))[:pairs]
+    bu, bv = np.ascontiguousarray(bu[pick]), np.ascontiguousarray(bv[pick])
+    base = O.custinger_count(off, adj)
+    want_off, want_adj = O.apply_batch_csr(n, off, adj, ins_u=bu, ins_v=bv,
+                                           del_u=np.zeros(0, np.int32), del_v=np.zeros(0, np.int32))
+    now = O.custinger_count(want_off, want_adj)
+    g = T.cuStinger(off, adj, slack_pct=100)
+    sched = T.default_schedule(capture=capture)
+    ins = np.zeros(pairs, np.uint8)
+    delta = T.DeviceArray(n, np.uint32).zero()
+    for _ in range(3 if capture else 1):
+        T.batch_apply(g, bu, bv, ins, delta, sched)
+        assert np.array_equal(base + delta.to_host(), now)
+        got_off, got_adj = g.to_csr()
+        assert np.array_equal(got_off, want_off) and np.array_equal(got_adj, want_adj)
+        T.batch_apply(g, bu, bv, 1 - ins, delta, sched)
+        assert not delta.to_host().any()
+        got_off, got_adj = g.to_csr()
+        assert np.array_equal(got_off, off) and np.array_equal(got_adj, adj)
+    g.close()
