@@ -785,7 +785,7 @@ void graph_destroy(Graph *g)
     DevBuf *bufs[] = {&g->st.boff, &g->st.len, &g->st.cap, &g->st.pool, &g->vinfo, &g->padj,
                       &g->coff, &g->crow, &g->work, &g->jobs, &g->tmp, &g->tmp2, &g->tmp3, &g->tmp4,
                       &g->accum, &g->bsrc, &g->bdst, &g->bflag, &g->bkeys, &g->bkeys2,
-                      &g->bvals2, &g->boffb, &g->bdel, &g->flagpool, &g->vmark, &g->order,
+                      &g->bvals2, &g->boffb, &g->bdel, &g->hrow, &g->flagpool, &g->vmark, &g->order,
                       &g->rnk, &g->tasks, &g->pcnt, &g->hjobs, &g->outr, &g->dmat, &g->ditems,
                       &g->dgraphs, &g->dgid, &g->cmat, &g->cgraphs, &g->cblocks};
     for (DevBuf *b : bufs) b->release(idle);

@@ -151,6 +151,7 @@ struct Graph {
     DevBuf bsrc, bdst, bflag, bkeys, bkeys2, bvals2, boffb, bdel;
     // streaming: per-entry "in the current batch" flags parallel to the pool,
     // per-vertex marks, and batch scratch
+    DevBuf hrow;  // small batches: copies of the long rows they merge into
     DevBuf flagpool, vmark;
     DevBuf sb[28];
     // capacity of a row that outgrows its block: len * grow_mul_x16 / 16 +

@@ -337,6 +337,23 @@ __global__ void k_unmark(const int32_t *__restrict__ queue, int64_t n0, const in
         mark[queue[i]] = 0;
 }
 
+// Batches of the one-block size: rows of kSplitRow entries or more are merged by
+// blocks of their own for every kSplitChunk entries, from a copy of the row
+// (k_split_copy, k_split_merge), as long as the copies fit kSplitMax chunks; one
+// block alone is held to one CU's 25 GB/s (rows of 10^5 entries, 1000 pairs: 42 us,
+// 6 + 8 so, with 13 for the shorter rows).  Larger batches fill the chip with one block per row.
+constexpr int32_t kSplitRow = 8192, kSplitChunk = 4096;
+// (two launches more: graphs whose longest row is below this took 3 to 6% longer)
+constexpr int32_t kSplitLongest = 65536;
+constexpr int kSplitThreads = 512, kSplitPer = kSplitChunk / kSplitThreads;
+constexpr int64_t kSplitMax = 1024;
+
+// Whether segment s has copies: hpre, the chunks of the rows before each segment.
+__device__ inline bool split_row(const int64_t *__restrict__ hpre, int64_t s, int64_t hcap)
+{
+    return hcap > 0 && hpre[s + 1] > hpre[s] && hpre[s + 1] <= hcap;
+}
+
 // Entries per thread per pass of the row kernels: every pass issues all its
 // loads before it writes, so a long row costs its length / (threads * entries
 // per thread) round trips instead of one per thread-width chunk.
@@ -714,7 +731,8 @@ __global__ __launch_bounds__(256) void k_merge_rows(
     const uint64_t *__restrict__ keys, int bv, const int32_t *__restrict__ need,
     const int64_t *__restrict__ nscan, const unsigned long long *__restrict__ ctl,
     int64_t *__restrict__ boff, int32_t *__restrict__ len, int32_t *__restrict__ cap,
-    int32_t *__restrict__ pool, uint8_t *__restrict__ flag, int64_t *__restrict__ newpos)
+    int32_t *__restrict__ pool, uint8_t *__restrict__ flag, int64_t *__restrict__ newpos,
+    const int64_t *__restrict__ hpre, int64_t hcap)
 {
     constexpr int kKeys = 256;
     __shared__ int32_t ys[256 / kWave][kWave * kRowPer];
@@ -729,16 +747,17 @@ __global__ __launch_bounds__(256) void k_merge_rows(
     for (int64_t s = (int64_t)blockIdx.x * (blockDim.x / kWave) + wid; s < nseg; s += wstride) {
         const int32_t v = sv[s];
         const int32_t lo = len[v];
-        if (lo >= kBigRow) continue;  // k_merge_rows_block
+        const bool split = split_row(hpre, s, hcap);  // k_split_merge has merged it
+        if (lo >= kBigRow && !split) continue;         // k_merge_rows_block
         const int64_t b0 = sbeg[s];
         const int32_t cn = (int32_t)(((s + 1 < nseg) ? sbeg[s + 1] : n) - b0);
         const int64_t ob = boff[v];
         const bool move = need[s] > 0;
         const int64_t db = move ? pool_used + nscan[s] : ob;
-        if (lo > 0) {
+        if (lo > 0 && !split) {
             merge_row<kWave, kRowPer>(ob, db, lo, keys, b0, cn, m, pool, flag, newpos, ys[wid],
                                       kl[wid], kKeys, sh[wid]);
-        } else {  // an empty row: the new entries in order
+        } else if (!split) {  // an empty row: the new entries in order
             for (int32_t i = lane; i < cn; i += kWave) {
                 pool[db + i] = (int32_t)(keys[b0 + i] & m);
                 flag[db + i] = 1;
@@ -789,7 +808,7 @@ __global__ __launch_bounds__(kRowThreads) void k_merge_rows_block(
     int64_t *__restrict__ boff,
     int32_t *__restrict__ len, int32_t *__restrict__ cap, int32_t *__restrict__ pool,
     uint8_t *__restrict__ flag, int64_t *__restrict__ newpos, const int32_t *__restrict__ big,
-    const unsigned long long *__restrict__ nbig)
+    const unsigned long long *__restrict__ nbig, const int64_t *__restrict__ hpre, int64_t hcap)
 {
     constexpr int kKeys = 4096;
     __shared__ int32_t ys[kRowThreads * kRowPerBlock];
@@ -805,7 +824,7 @@ __global__ __launch_bounds__(kRowThreads) void k_merge_rows_block(
         const int64_t s = big ? big[k] : k;
         const int32_t v = sv[s];
         const int32_t lo = len[v];
-        if (lo < kBigRow) continue;
+        if (lo < kBigRow || split_row(hpre, s, hcap)) continue;
         const int64_t b0 = sbeg[s];
         const int32_t cn = (int32_t)(((s + 1 < nseg) ? sbeg[s + 1] : n) - b0);
         const int64_t ob = boff[v];
@@ -928,6 +947,103 @@ __device__ inline int64_t wave_edge_of(const int64_t *__restrict__ pre, int64_t 
         n = min(step, n - j * step);
     }
     return lo;
+}
+
+// The split rows' chunks copied: chunk q of all to scratch + q * kSplitChunk.
+__global__ __launch_bounds__(256) void k_split_copy(const int32_t *__restrict__ sv, const int64_t *__restrict__ hpre,
+                                                    int64_t hcap, const int64_t *__restrict__ boff,
+                                                    const int32_t *__restrict__ len,
+                                                    const int32_t *__restrict__ pool,
+                                                    int32_t *__restrict__ scratch)
+{
+    const int64_t total = min(hpre[kRegSort], hcap);
+    for (int64_t q = blockIdx.x; q < total; q += gridDim.x) {
+        const int64_t s = wave_edge_of(hpre, q, kRegSort);
+        if (!split_row(hpre, s, hcap)) continue;
+        const int32_t v = sv[s], j0 = (int32_t)(q - hpre[s]) * kSplitChunk;
+        const int32_t n = min(kSplitChunk, len[v] - j0);
+        const int32_t *src = pool + boff[v] + j0;
+        int32_t *dst = scratch + q * kSplitChunk;
+#pragma unroll 8
+        for (int32_t i = threadIdx.x; i < n; i += 256) dst[i] = src[i];
+    }
+}
+
+// merge_row by chunks of the copy, one block each: the old entries of a chunk and
+// the new ones above its first entry (below it too in the first chunk) up to the
+// next chunk's first.  The row's length and place are set by k_merge_rows.
+__global__ __launch_bounds__(kSplitThreads) void k_split_merge(
+    const int32_t *__restrict__ sv, const int64_t *__restrict__ sbeg, int64_t nseg0,
+    const int64_t *__restrict__ nsegd, int64_t n0, const int64_t *__restrict__ nd,
+    const uint64_t *__restrict__ keys, int bv, const int32_t *__restrict__ need,
+    const int64_t *__restrict__ nscan, const unsigned long long *__restrict__ ctl,
+    const int64_t *__restrict__ boff, const int32_t *__restrict__ len, int32_t *__restrict__ pool,
+    uint8_t *__restrict__ flag, int64_t *__restrict__ newpos, const int64_t *__restrict__ hpre, int64_t hcap,
+    const int32_t *__restrict__ scratch)
+{
+    __shared__ int32_t ys[kSplitChunk];
+    __shared__ int32_t kl[kRegSort];
+    __shared__ int32_t sh[2];
+    if (!ctl[kCtlFits]) return;
+    const int t = threadIdx.x;
+    const int64_t nseg = bound(nseg0, nsegd), n = bound(n0, nd);
+    const int64_t total = min(hpre[kRegSort], hcap);
+    const uint64_t m = (1ull << bv) - 1;
+    for (int64_t q = blockIdx.x; q < total; q += gridDim.x) {
+        const int64_t s = wave_edge_of(hpre, q, kRegSort);
+        if (!split_row(hpre, s, hcap)) continue;  // (the same in the whole block)
+        const int32_t v = sv[s], lo = len[v];
+        const int64_t b0 = sbeg[s];
+        const int32_t cn = (int32_t)(((s + 1 < nseg) ? sbeg[s + 1] : n) - b0);  // (at most kRegSort)
+        const int64_t ob = boff[v];
+        const bool inplace = need[s] <= 0;
+        const int64_t db = inplace ? ob : (int64_t)ctl[kCtlBase] + nscan[s];
+        const int32_t j0 = (int32_t)(q - hpre[s]) * kSplitChunk, jn = min(kSplitChunk, lo - j0);
+        const int32_t *src = scratch + q * kSplitChunk;
+        int32_t y[kSplitPer], A[kSplitPer];
+#pragma unroll
+        for (int k = 0; k < kSplitPer; ++k) y[k] = k * kSplitThreads + t < jn ? src[k * kSplitThreads + t] : 0;
+        const int32_t next = j0 + jn < lo ? src[kSplitChunk] : 0;
+        for (int32_t i = t; i < cn; i += kSplitThreads) kl[i] = (int32_t)(keys[b0 + i] & m);
+#pragma unroll
+        for (int k = 0; k < kSplitPer; ++k)
+            if (k * kSplitThreads + t < jn) ys[k * kSplitThreads + t] = y[k];
+        __syncthreads();
+        auto below = [&](int32_t x) {  // new entries below x
+            int32_t a = 0, b = cn;
+            while (a < b) {
+                const int32_t mid = (a + b) >> 1;
+                if (kl[mid] < x) a = mid + 1; else b = mid;
+            }
+            return a;
+        };
+#pragma unroll
+        for (int k = 0; k < kSplitPer; ++k) A[k] = k * kSplitThreads + t < jn ? below(y[k]) : 0;
+        if (t == 0) sh[0] = j0 > 0 ? A[0] : 0;
+        if (t == kSplitThreads - 1) sh[1] = j0 + jn < lo ? below(next) : cn;
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kSplitPer; ++k) {
+            const int32_t j = k * kSplitThreads + t;
+            if (j < jn && (A[k] > 0 || !inplace)) {
+                pool[db + j0 + j + A[k]] = y[k];
+                flag[db + j0 + j + A[k]] = 0;
+            }
+        }
+        for (int32_t i = sh[0] + t; i < sh[1]; i += kSplitThreads) {
+            const int32_t x = kl[i];
+            int32_t a = 0, b = jn;  // entries of the chunk below x
+            while (a < b) {
+                const int32_t mid = (a + b) >> 1;
+                if (ys[mid] < x) a = mid + 1; else b = mid;
+            }
+            const int64_t d = db + i + j0 + a;
+            pool[d] = x;
+            flag[d] = 1;
+            newpos[b0 + i] = d;
+        }
+        __syncthreads();  // the tables are rewritten by the next chunk
+    }
 }
 
 // Each wave takes two chunks of 64 items per pass (c and c + the grid's wave
@@ -1621,7 +1737,7 @@ __global__ __launch_bounds__(1024) void k_small_insert(
     int32_t mul_x16, int32_t add, int32_t *__restrict__ absent, int64_t *__restrict__ ndir,
     uint64_t *__restrict__ dk, int32_t *__restrict__ sv, int64_t *__restrict__ sbeg,
     int64_t *__restrict__ nseg_out, int32_t *__restrict__ need, int64_t *__restrict__ nscan,
-    int64_t *__restrict__ nmoved, unsigned long long *__restrict__ ctl)
+    int64_t *__restrict__ nmoved, unsigned long long *__restrict__ ctl, int64_t *__restrict__ hpre)
 {
     __shared__ uint64_t buf[2][kRegSort];
     __shared__ int32_t segb[kRegSort + 1];  // segment starts
@@ -1700,14 +1816,15 @@ __global__ __launch_bounds__(1024) void k_small_insert(
     }
     __syncthreads();
     // block sizes of the rows that outgrow their blocks (rows s = t, 1024 + t)
-    int64_t c[2];
+    int64_t c[2], hc[2];
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
         const int s = q * 1024 + t;
-        c[q] = 0;
+        c[q] = hc[q] = 0;
         if (s < nseg) {
-            const int32_t r = segv[s];
-            const int64_t nl = (int64_t)len[r] + (segb[s + 1] - segb[s]);
+            const int32_t r = segv[s], lr = len[r];
+            if (lr >= kSplitRow) hc[q] = ceil_div(lr, kSplitChunk);
+            const int64_t nl = (int64_t)lr + (segb[s + 1] - segb[s]);
             if (nl > cap[r]) {
                 if (mul_x16 > 0) {
                     c[q] = nl * mul_x16 / 16 + add;
@@ -1724,11 +1841,17 @@ __global__ __launch_bounds__(1024) void k_small_insert(
     scan_rows_2048(c[0], c[1], e0, e1, grow, ws64);
     if (t < B2) nscan[t] = e0;
     if (1024 + t < B2) nscan[1024 + t] = e1;
-    int64_t mv0, mv1, moved;
-    scan_rows_2048(c[0] != 0, c[1] != 0, mv0, mv1, moved, ws64);
+    // the moved rows (low words) and the split rows' chunks (high words) together
+    int64_t mh0, mh1, both;
+    scan_rows_2048(hc[0] << 32 | (c[0] != 0), hc[1] << 32 | (c[1] != 0), mh0, mh1, both, ws64);
+    if (hpre) {
+        hpre[t] = mh0 >> 32;
+        hpre[1024 + t] = mh1 >> 32;
+        if (t == 0) hpre[kRegSort] = both >> 32;
+    }
     if (t == 0) {
         nscan[B2] = grow;
-        *nmoved = moved;
+        *nmoved = (int64_t)(uint32_t)both;
         if (ctl) {  // k_pool_reserve
             ctl[kCtlGrow] = (unsigned long long)grow;
             const unsigned long long used = ctl[kCtlPoolUsed];
@@ -1992,6 +2115,21 @@ int batch_apply(Graph &g, const int32_t *u, const int32_t *v, const uint8_t *is_
     const int gB = grid_for(Bc, 256, 65536), gB2 = grid_for(B2, 256, 65536);
     const bool small = Bc <= kSmallPairs;  // one-block bookkeeping
 
+    // (no room for the copies: one block per row)
+    int64_t *hpre = nullptr;
+    int32_t *scratch = nullptr;
+    // (the longest row as last known: it decides the speed only)
+    int64_t hcap = small && g.max_degree >= kSplitLongest ? std::min<int64_t>(kSplitMax, (int64_t)(g.st.pool.bytes / sizeof(int32_t)) / kSplitChunk) : 0;
+    if (hcap > 0) {
+        const size_t head_bytes = (kRegSort + 1) * sizeof(int64_t) + 8;
+        if (g.hrow.ensure(head_bytes + (size_t)hcap * kSplitChunk * sizeof(int32_t)) == TC_OK) {
+            hpre = g.hrow.as<int64_t>();
+            scratch = reinterpret_cast<int32_t *>(g.hrow.as<char>() + head_bytes);
+        } else {
+            hcap = 0;
+        }
+    }
+
     uint32_t *out = delta;
     if (count && !out) {
         TC_TRY(g.tmp4.ensure((size_t)std::max(nv, 1) * sizeof(uint32_t)));
@@ -2025,11 +2163,19 @@ int batch_apply(Graph &g, const int32_t *u, const int32_t *v, const uint8_t *is_
                            sv, sbeg, B2, nseg, B2, ndir, dk, bv, need, nscan, ctl,
                            g.st.boff.as<int64_t>(), g.st.len.as<int32_t>(), g.st.cap.as<int32_t>(),
                            g.st.pool.as<int32_t>(), g.flagpool.as<uint8_t>(), newpos,
-                           small ? nullptr : head, small ? nullptr : acc + 28);
+                           small ? nullptr : head, small ? nullptr : acc + 28, hpre, hcap);
+        if (hcap > 0) {
+            const dim3 chunks((unsigned)std::min<int64_t>(hcap, 1024));
+            hipLaunchKernelGGL(k_split_copy, chunks, dim3(256), 0, st, sv, hpre, hcap, g.st.boff.as<int64_t>(),
+                               g.st.len.as<int32_t>(), g.st.pool.as<int32_t>(), scratch);
+            hipLaunchKernelGGL(k_split_merge, chunks, dim3(kSplitThreads), 0, st, sv, sbeg, B2, nseg, B2, ndir, dk,
+                               bv, need, nscan, ctl, g.st.boff.as<int64_t>(), g.st.len.as<int32_t>(),
+                               g.st.pool.as<int32_t>(), g.flagpool.as<uint8_t>(), newpos, hpre, hcap, scratch);
+        }
         hipLaunchKernelGGL(k_merge_rows, dim3(grid_for(B2, 4, 65536)), dim3(256), 0, st, sv, sbeg, B2,
                            nseg, B2, ndir, dk, bv, need, nscan, ctl, g.st.boff.as<int64_t>(),
                            g.st.len.as<int32_t>(), g.st.cap.as<int32_t>(), g.st.pool.as<int32_t>(),
-                           g.flagpool.as<uint8_t>(), newpos);
+                           g.flagpool.as<uint8_t>(), newpos, hpre, hcap);
         TC_HIP(hipGetLastError());
         if (count) {
             TC_HIP(rec(first ? 11 : 14, st));
@@ -2113,7 +2259,7 @@ int batch_apply(Graph &g, const int32_t *u, const int32_t *v, const uint8_t *is_
             hipLaunchKernelGGL(k_small_insert, dim3(1), dim3(1024), 0, st, ia, ib, pres, Bc, nI, bv,
                                directed ? 1 : 0, pad, g.st.len.as<int32_t>(), g.st.cap.as<int32_t>(),
                                g.grow_mul_x16, g.grow_add, absent, ndir, dk, sv, sbeg, hpos + B2, need,
-                               nscan, nmoved, ctl);
+                               nscan, nmoved, ctl, hpre);
         } else {
             hipLaunchKernelGGL(k_not, dim3(gB), dim3(256), 0, st, pres, Bc, nI, absent);
             TC_TRY(scan_counts_i32(absent, sidx, Bc, g.tmp, st));
@@ -2149,11 +2295,11 @@ int batch_apply(Graph &g, const int32_t *u, const int32_t *v, const uint8_t *is_
             const unsigned char *c = static_cast<const unsigned char *>(p);
             for (size_t i = 0; i < n; ++i) key = (key ^ c[i]) * 1099511628211ull;
         };
-        const int64_t kv[8] = {Bc, directed, count, track_sym, bv, g.grow_mul_x16, g.grow_add, 0};
+        const int64_t kv[8] = {Bc, directed, count, track_sym, bv, g.grow_mul_x16, g.grow_add, hcap};
         mix(kv, sizeof(kv));
         const void *ptrs[] = {out, g.st.pool.p, g.flagpool.p, g.st.boff.p, g.st.len.p, g.st.cap.p,
                               g.vmark.p, g.accum.p, g.tmp.p, g.bsrc.p, g.bdst.p, g.bdel.p, g.boffb.p,
-                              g.lbuf[0].p, g.lbuf[1].p, g.lbuf[2].p, g.lbuf[3].p, g.lbuf[4].p};
+                              g.lbuf[0].p, g.lbuf[1].p, g.lbuf[2].p, g.lbuf[3].p, g.lbuf[4].p, g.hrow.p};
         mix(ptrs, sizeof(ptrs));
         for (const DevBuf &b : g.sb) mix(&b.p, sizeof(b.p));
         key |= 1ull;

@@ -113,3 +113,30 @@ def test_small_batches_of_every_sort_size(pairs, capture):
         got_off, got_adj = g.to_csr()
         assert np.array_equal(got_off, off) and np.array_equal(got_adj, adj)
     g.close()
+
+
+@pytest.mark.parametrize("slack", [0, 100])
+def test_small_batches_into_rows_of_several_chunks(slack):
+    """Rows around the length that several blocks merge and around their chunks,
+    with new entries first, last and at chunk borders, in place and moved, more of
+    them than the copies have room for."""
+    n = 80000
+    rng = np.random.default_rng(slack)
+    lens = [8191, 8192, 8193, 12287, 12288, 12289, 40000, 66000] + [8193] * 40
+    hubs = np.arange(100, 100 + len(lens))
+    u, v = [], []
+    for h, k in zip(hubs, lens):
+        cand = rng.permutation(np.arange(200, n - 200))[:k]
+        u.append(np.full(k, h))
+        v.append(cand)
+    off, adj = O.canon_csr(n, np.concatenate(u).astype(np.int32), np.concatenate(v).astype(np.int32))
+    pu, pv = [], []
+    for h in hubs:
+        row = adj[off[h]:off[h + 1]]
+        near = [0, 1, n - 1, n - 2] + [int(row[q]) + 1 for q in (4094, 4095, 4096, 8190) if q < len(row)]
+        near += list(rng.integers(0, n, 6))
+        pu += [h] * len(near)
+        pv += near
+    bu, bv = _new_pairs(n, off, adj, np.array(pu), np.array(pv))
+    bu, bv = bu[:1024], bv[:1024]
+    _insert_and_undo(n, off, adj, bu, bv, slack)
