@@ -22,7 +22,7 @@
 // the learned table.  Jobs come from a prefix-sum partition of the estimated
 // work per owner (the load-balance layer, include/load_balance.cuh:77-102),
 // binned by owner-list length (small / mid / large+tiled).
-#include "tc_internal.hpp"
+#include "tc_plan.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -1638,37 +1638,6 @@ __global__ void k_direct_task_vinfo(const int64_t *__restrict__ boff, const int3
 
 // ------------------------------------------------------------- planning --
 
-struct PlanParams {
-    int32_t lmax[3];     // owner-list capacity of each bin's kernel
-    int32_t nw[3];       // wavefronts per block of each bin's kernel
-    int32_t bin_max[2];  // |owner| <= bin_max[0] -> bin 0, <= bin_max[1] -> bin 1, else 2
-    // owners from wide_lo up with wide_tasks: above wide_max -> bin 2 as well
-    int32_t wide_lo, wide_max, wide_tasks;
-    int32_t job_items;   // target estimated items per job (per wavefront)
-    int32_t flush_items; // minimum items per owner slot in a job
-    int32_t owner_end;   // owners from here up get no jobs (the core's)
-    int32_t id_tiles;    // > 0: owners of bin 2 are tiled by id range, into this many
-};
-
-__device__ inline int32_t owner_tiles(int32_t L, int bin, const PlanParams &P)
-{
-    return bin == 2 && P.id_tiles > 0 ? P.id_tiles : (int32_t)ceil_div(L, P.lmax[bin]);
-}
-
-__device__ inline int32_t est_items(int32_t L, int32_t pl)
-{
-    // cheapest of streaming the task list (pl) and searching the owner list (L*log pl)
-    const int32_t lg = max(1, 32 - __clz(pl));  // smallest lg >= 1 with 2^lg > pl
-    int64_t bs = (int64_t)L * lg;
-    return (int32_t)min<int64_t>(pl, bs) + 4;
-}
-
-__device__ inline int owner_bin(int32_t v, int32_t L, int32_t tasks, const PlanParams &P)
-{
-    const bool wide = v >= P.wide_lo && L > P.wide_max && tasks >= P.wide_tasks;
-    return L <= P.bin_max[0] ? 0 : (L <= P.bin_max[1] && !wide ? 1 : 2);
-}
-
 // Per-owner estimated work (sum over its tasks); per-bin stats.
 // Entries are the task array (oriented) or the store rows (direct), with
 // their row offsets coff and chunk rows crow.  Two blocks of 16 waves per CU:
@@ -1786,7 +1755,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan_jobs(
     __shared__ unsigned long long base[3];
     if (*fault) return;  // (set by kernels before this one: the same for all)
     const int t = threadIdx.x, lane = t & (kWave - 1), wid = t / kWave;
-    const int64_t wmin = (int64_t)(*wtotal >> 20);
+    const int64_t wmin = plan_wmin(*wtotal);
     const int64_t v0 = (int64_t)blockIdx.x * kPlanOwners + (int64_t)t * kPlanPer;
     int32_t nj[kPlanPer], split[kPlanPer], T[kPlanPer], cnt[3] = {0, 0, 0};
     int bin[kPlanPer];
@@ -1803,23 +1772,13 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan_jobs(
         T[k] = ORIENTED ? x.dm : x.len;
         if (L <= 0 || T[k] <= 0 || w == 0 || (!ORIENTED && x.len < 2)) continue;
         bin[k] = owner_bin((int32_t)v, L, T[k], P);
-        const int64_t tiles = owner_tiles(L, bin[k], P);
-        const int64_t per_tile = (int64_t)(w / (unsigned long long)tiles) + 1;
-        // a job amortises building its LDS table and, at its end, the flush of
-        // up to one global atomic per owner slot: at least flush_items items
-        // per slot
-        const int64_t grain = max(max((int64_t)P.job_items * P.nw[bin[k]],
-                                      (int64_t)P.flush_items * min(L, P.lmax[bin[k]])), wmin);
-        int64_t sp = ceil_div(per_tile, grain);
-        if (sp > T[k]) sp = T[k];
-        if (sp < 1) sp = 1;
-        split[k] = (int32_t)sp;
-        nj[k] = (int32_t)(sp * tiles);
+        split[k] = owner_split(L, T[k], w, bin[k], wmin, P);
+        nj[k] = split[k] * owner_tiles(L, bin[k], P);
 #pragma unroll
         for (int q = 0; q < 3; ++q)
             if (q == bin[k]) {
                 cnt[q] += nj[k];
-                tile_items[q] += (unsigned long long)sp * (unsigned long long)L;
+                tile_items[q] += (unsigned long long)split[k] * (unsigned long long)L;
             }
     }
     int32_t incl[3];
@@ -1971,8 +1930,6 @@ __global__ void k_graph_of(const int64_t *__restrict__ voff, int32_t G,
 }
 
 // ---------------------------------------------------------- count kernel --
-
-enum { kDirect = 0, kOriented = 1, kByTasks = 2 };
 
 struct CountArgs {
     const int32_t *adj;
@@ -2240,12 +2197,12 @@ template <int LMAX, int NW, int MODE>
 #define TC_SMALL_WAVES 7
 #endif
 __global__ __launch_bounds__(NW * kWave, LMAX <= 64 ? TC_SMALL_WAVES : LMAX <= 512 ? TC_MID_WAVES : 1) void k_count(const Job *__restrict__ jobs, const unsigned long long *__restrict__ njobs_dev,
-                                                      CountArgs A)
+                                                      int64_t cap, CountArgs A)
 {
     // MODE: kDirect (tasks are the owner's row entries), kOriented, kByTasks
     // (direct counts by the larger row, see k_direct_tasks)
     constexpr bool ORIENTED = MODE == kOriented, TASKS = MODE != kDirect;
-    const int64_t njobs = (int64_t)*njobs_dev;
+    const int64_t njobs = min((int64_t)*njobs_dev, cap);
     // The owner tile lives in a bucketed two-choice hash table (BucketTableT),
     // load <= 1/2, so a lookup reads one bucket, a second only where the
     // first is full, and loops only when both are.  C counts hits per slot
@@ -2701,9 +2658,9 @@ constexpr int kLongUnroll = TC_LONG_UNROLL;
 template <int LMAX, int NW, bool BM>
 __global__ __launch_bounds__(NW * kWave, BM ? 6 : 4) void k_count_long(const Job *__restrict__ jobs,
                                                            const unsigned long long *__restrict__ njobs_dev,
-                                                           CountArgs A)
+                                                           int64_t cap, CountArgs A)
 {
-    const int64_t njobs = (int64_t)*njobs_dev;
+    const int64_t njobs = min((int64_t)*njobs_dev, cap);
     constexpr int NBMAX = LMAX / 2;
     constexpr int kBmWords = 2 * NBMAX;  // uint2 words in HB's space
     // one LDS block: the table (or bitmap) HB, then the counters C.  The
@@ -2917,9 +2874,9 @@ __device__ inline int32_t row_lower(const int32_t *__restrict__ row, int32_t n, 
 template <int WORDS, int NT>
 __global__ __launch_bounds__(NT, NT == 512 ? 6 : 4) void k_direct_bits(const Job *__restrict__ jobs,
                                                                      const unsigned long long *__restrict__ njobs_dev,
-                                                                     CountArgs A)
+                                                                     int64_t cap, CountArgs A)
 {
-    const int64_t njobs = (int64_t)*njobs_dev;
+    const int64_t njobs = min((int64_t)*njobs_dev, cap);
     constexpr int U = 8, NW = NT / kWave;
     __shared__ uint32_t bits[WORDS + 1];  // (one word past the span: the zero guard word)
     __shared__ int64_t s_job;
@@ -3026,22 +2983,11 @@ tc_schedule default_schedule()
 
 namespace {
 
-constexpr int kL0 = 64, kL1 = 512, kL2 = 4096;
-// (the ranks that k_count_long's bitmap holds, its guard word left)
-constexpr int32_t kWideMin = 128, kWideTasks = 64, kWideSpan = (kL2 - 1) * 32;
-constexpr int64_t kWideNnz = int64_t(3) << 24;
 // owners of at least this degree get their task lists from their own rows
 // (k_orient_transpose_hubs) instead of by appends
 constexpr int kHubDegree = 65536;  // with the appends
-#ifndef TC_MID_NW
-#define TC_MID_NW 2
-#endif
-constexpr int kNW0 = 1, kNW1 = TC_MID_NW, kNW2 = 8;
-// ids of a bit row in LDS (k_direct_bits): 32 KB, four blocks of 8 waves a CU,
-// and 128 KB, one block of 16
-constexpr int kBitsIds0 = 1 << 18, kBitsIds1 = 1 << 20;
 
-// most bounds the bin's jobs, whose number is on the device.
+// most: room for the bin's jobs, whose number is on the device.
 // ev_long (bin 2, oriented): events recorded before and after the bitmap-tile
 // launch of k_count_long and after its hash-table-tile launch.
 int launch_bin(int bin, int mode, const Job *jobs, int64_t most, const unsigned long long *njobs,
@@ -3058,25 +3004,25 @@ int launch_bin(int bin, int mode, const Job *jobs, int64_t most, const unsigned 
     int64_t grid = std::min<int64_t>(most, (int64_t)cus * per_cu);
     if (mode == kByTasks) {
         if (bin == 0)
-            hipLaunchKernelGGL((k_count<kL0, kNW0, kByTasks>), dim3((unsigned)grid), dim3(kNW0 * kWave), 0, s, jobs, njobs, A);
+            hipLaunchKernelGGL((k_count<kL0, kNW0, kByTasks>), dim3((unsigned)grid), dim3(kNW0 * kWave), 0, s, jobs, njobs, most, A);
         else if (bin == 1)
-            hipLaunchKernelGGL((k_count<kL1, kNW1, kByTasks>), dim3((unsigned)grid), dim3(kNW1 * kWave), 0, s, jobs, njobs, A);
+            hipLaunchKernelGGL((k_count<kL1, kNW1, kByTasks>), dim3((unsigned)grid), dim3(kNW1 * kWave), 0, s, jobs, njobs, most, A);
         else if (A.nv <= kBitsIds0)
             hipLaunchKernelGGL((k_direct_bits<kBitsIds0 / 32, 512>), dim3((unsigned)std::min<int64_t>(most, cus * 3)),
-                               dim3(512), 0, s, jobs, njobs, A);
+                               dim3(512), 0, s, jobs, njobs, most, A);
         else
             hipLaunchKernelGGL((k_direct_bits<kBitsIds1 / 32, 1024>), dim3((unsigned)std::min<int64_t>(most, cus)),
-                               dim3(1024), 0, s, jobs, njobs, A);
+                               dim3(1024), 0, s, jobs, njobs, most, A);
     } else if (bin == 0) {
         if (oriented)
-            hipLaunchKernelGGL((k_count<kL0, kNW0, kOriented>), dim3((unsigned)grid), dim3(kNW0 * kWave), 0, s, jobs, njobs, A);
+            hipLaunchKernelGGL((k_count<kL0, kNW0, kOriented>), dim3((unsigned)grid), dim3(kNW0 * kWave), 0, s, jobs, njobs, most, A);
         else
-            hipLaunchKernelGGL((k_count<kL0, kNW0, kDirect>), dim3((unsigned)grid), dim3(kNW0 * kWave), 0, s, jobs, njobs, A);
+            hipLaunchKernelGGL((k_count<kL0, kNW0, kDirect>), dim3((unsigned)grid), dim3(kNW0 * kWave), 0, s, jobs, njobs, most, A);
     } else if (bin == 1) {
         if (oriented)
-            hipLaunchKernelGGL((k_count<kL1, kNW1, kOriented>), dim3((unsigned)grid), dim3(kNW1 * kWave), 0, s, jobs, njobs, A);
+            hipLaunchKernelGGL((k_count<kL1, kNW1, kOriented>), dim3((unsigned)grid), dim3(kNW1 * kWave), 0, s, jobs, njobs, most, A);
         else
-            hipLaunchKernelGGL((k_count<kL1, kNW1, kDirect>), dim3((unsigned)grid), dim3(kNW1 * kWave), 0, s, jobs, njobs, A);
+            hipLaunchKernelGGL((k_count<kL1, kNW1, kDirect>), dim3((unsigned)grid), dim3(kNW1 * kWave), 0, s, jobs, njobs, most, A);
     } else {
         if (oriented) {
             // short tasks here, long hash tasks in k_count_long (bitmap and
@@ -3091,18 +3037,18 @@ int launch_bin(int bin, int mode, const Job *jobs, int64_t most, const unsigned 
             const bool forced = A.policy == TC_POLICY_MERGE || A.policy == TC_POLICY_BSEARCH ||
                                 A.policy == TC_POLICY_MERGEPATH;
             if (forced)
-                hipLaunchKernelGGL((k_count<kL2, kNW2, kOriented>), dim3((unsigned)grid), dim3(kNW2 * kWave), 0, s, jobs, njobs, As);
+                hipLaunchKernelGGL((k_count<kL2, kNW2, kOriented>), dim3((unsigned)grid), dim3(kNW2 * kWave), 0, s, jobs, njobs, most, As);
             const int64_t gb = std::min<int64_t>(most, (int64_t)cus * 3);
             const int64_t gh = std::min<int64_t>(most, (int64_t)cus * 2);
             if (ev_long) TC_HIP(hipEventRecord(ev_long[0], s));
             if (!forced)
-                hipLaunchKernelGGL((k_count_long<kL2, kNW2, true>), dim3((unsigned)gb), dim3(kNW2 * kWave), 0, s, jobs, njobs, Al);
+                hipLaunchKernelGGL((k_count_long<kL2, kNW2, true>), dim3((unsigned)gb), dim3(kNW2 * kWave), 0, s, jobs, njobs, most, Al);
             if (ev_long) TC_HIP(hipEventRecord(ev_long[1], s));
             if (!forced)
-                hipLaunchKernelGGL((k_count_long<kL2, kNW2, false>), dim3((unsigned)gh), dim3(kNW2 * kWave), 0, s, jobs, njobs, Al);
+                hipLaunchKernelGGL((k_count_long<kL2, kNW2, false>), dim3((unsigned)gh), dim3(kNW2 * kWave), 0, s, jobs, njobs, most, Al);
             if (ev_long) TC_HIP(hipEventRecord(ev_long[2], s));
         } else
-            hipLaunchKernelGGL((k_count<kL2, kNW2, kDirect>), dim3((unsigned)grid), dim3(kNW2 * kWave), 0, s, jobs, njobs, A);
+            hipLaunchKernelGGL((k_count<kL2, kNW2, kDirect>), dim3((unsigned)grid), dim3(kNW2 * kWave), 0, s, jobs, njobs, most, A);
     }
     TC_HIP(hipGetLastError());
     return TC_OK;
@@ -3650,49 +3596,7 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     const int wblocks = grid_for(nchunks, 2 * kWorkThreads / kWave, kWorkBlocks);
 
     // ---- planning: work per owner, jobs per bin
-    PlanParams P;
-    P.lmax[0] = kL0;
-    P.lmax[1] = kL1;
-    P.lmax[2] = kL2;
-    P.nw[0] = kNW0;
-    P.nw[1] = kNW1;
-    P.nw[2] = kNW2;
-    P.bin_max[0] = std::min(std::max(sched.small_max, 1), kL0);
-    P.bin_max[1] = std::min(std::max(sched.mid_max, P.bin_max[0]), kL1);
-    P.job_items = std::max(sched.job_items, 256);
-    P.flush_items = sched.flush_items > 0 ? sched.flush_items : 1024;
-    P.owner_end = nv - (oriented ? g.core_k : 0);
-    // Owners whose rows fit k_count_long's bitmap by their rank (a row of N+ spans
-    // at most the ranks above its owner) go to the largest bin from kWideMin
-    // entries on: it streams 1300 G entries a second against the mid bin's 440,
-    // whose bitmap holds an eighth of the ranks, and hash tables beyond (3M ragged
-    // vertices 12.2 -> 10.3 ms; 96, 192, 256, 384 entries: 10.3, 10.3, 10.6, 10.7).
-    // Its jobs of eight waves need a large graph to fill the chip: R-MAT graphs of
-    // 8M to 48M entries took 1.01 to 1.12 times as long, of 63M and more 0.84 to
-    // 0.96.  Without enough tasks the bitmap is not repaid; the largest bin's hash
-    // tables are no gain either (R-MAT 24 with all rows from 256 on 131 -> 149 ms),
-    // nor are batched graphs, whose cores lie behind all other ranks.
-    P.wide_lo = INT32_MAX;
-    P.wide_max = P.bin_max[1];
-    P.wide_tasks = kWideTasks;
-    if (oriented && !g.batch_voff && nnz >= kWideNnz && P.bin_max[1] > kWideMin &&
-        (sched.policy == TC_POLICY_HASH || sched.policy == TC_POLICY_LEARNED ||
-         (sched.policy == TC_POLICY_FIXED && sched.ratio_x16 <= 0 && sched.mpath_min <= 0))) {
-        P.wide_lo = std::max(nv - kWideSpan, 0);
-        P.wide_max = kWideMin;
-    }
-    // by tasks: bit rows hold any list whole, and a job of theirs ends without a
-    // flush.  Beyond kBitsIds1 ids a row is tiled by id range, which pays for
-    // the largest bin only (the mid bin's lists go through LDS tables).
-    P.id_tiles = 0;
-    const bool one_bits = mode == kByTasks && nv <= kBitsIds1;
-    if (mode == kByTasks) {
-        P.id_tiles = (int32_t)ceil_div(nv, kBitsIds1);
-        P.lmax[2] = INT32_MAX;
-        P.nw[2] = 8;
-        P.flush_items = 16;
-        if (one_bits) P.bin_max[1] = P.bin_max[0];  // (no mid bin)
-    }
+    const PlanParams P = plan_params(sched, mode, g.batch_voff != nullptr, nv, nnz, g.core_k);
     TC_TRY(g.work.ensure((size_t)nv * sizeof(unsigned long long)));
     unsigned long long *work = g.work.as<unsigned long long>();
     hipLaunchKernelGGL(k_fill_u64, dim3(grid_for(nv, 256, 65536)), dim3(256), 0, s, work, (int64_t)nv);
@@ -3703,23 +3607,11 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
         hipLaunchKernelGGL(k_owner_work<false>, dim3(wblocks), dim3(kWorkThreads), 0, s, coff, crow, vi, adj,
                            nullptr, nv, P, work, acc + 26, acc + 27, stats ? acc + 4 : nullptr);
     TC_HIP(hipGetLastError());
-    // the longest list there can be (|N+| <= sqrt(nnz)), and with it the most
-    // jobs a bin can have: one per owner and tile, and what its work gives, at
-    // most 2^21 (k_plan_jobs)
     const int64_t lists = oriented ? g.nplus : nnz;
-    const int64_t lmost = oriented ? (int64_t)std::sqrt((double)nnz) + 1
-                          : g.validated && !g.degree_stale ? g.max_degree : nv;
+    const int64_t lmost = longest_list(oriented, nv, nnz, g.validated && !g.degree_stale ? g.max_degree : nv);
     JobArrays J = {};
-    const int64_t owners[3] = {nv, std::min<int64_t>(nv, lists / (P.bin_max[0] + 1)),
-                               std::min<int64_t>(nv, lists / (P.wide_max + 1))};
-    int64_t total_cap = 0;
-    for (int b = 0; b < 3; ++b) {
-        const bool any = b == 0 || lmost > (b == 1 ? P.bin_max[0] : P.wide_max);
-        const double more = (double)lists * (double)(lmost + 4) / ((double)P.job_items * P.nw[b]);
-        J.cap[b] = any ? owners[b] + 64 + (int64_t)std::min(more, 2097152.0) : 0;
-        if (b == 2 && any) J.cap[b] += P.id_tiles > 0 ? owners[b] * P.id_tiles : 2 * (lists / P.lmax[2]);
-        total_cap += J.cap[b];
-    }
+    plan_caps(P, nv, lists, lmost, J.cap);
+    const int64_t total_cap = J.cap[0] + J.cap[1] + J.cap[2];
     TC_TRY(g.jobs.ensure((size_t)total_cap * sizeof(Job)));
     J.j[0] = g.jobs.as<Job>();
     J.j[1] = J.j[0] + J.cap[0];
@@ -3829,6 +3721,11 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
                                g.batch_per_graph, (int64_t)g.batch_ngraphs);
         return count_pass(g, out, global, sched, stats, skip_lower);  // the direct way
     }
+    for (int b = 0; b < 3; ++b)
+        if ((int64_t)hacc[28 + b] > J.cap[b]) {  // (plan_caps bounds them: a fault of the planner)
+            set_last_error(TC_ERR_CAPACITY, "static count: more jobs than their array holds");
+            return TC_ERR_CAPACITY;
+        }
     if (global) *global = hacc[0];
     if (stats) {
         fill_counters(st, hacc, oriented);

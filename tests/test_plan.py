@@ -1,0 +1,68 @@
+"""The capacities of the job arrays against the jobs that the planner's rule
+gives, on the host: row lengths around every bin's bounds, in each mode."""
+from __future__ import annotations
+
+import ctypes as C
+import os
+
+import numpy as np
+import pytest
+
+import custingeralg_amd as T
+import oracle as O
+
+_LIB = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "libplan_test.so")
+DIRECT, ORIENTED, BY_TASKS = 0, 1, 2
+
+
+def _plan(mode, off, adj, skip_lower=0, **sched):
+    lib = C.CDLL(_LIB)
+    s = T.default_schedule(**sched)
+    jobs, caps = (C.c_int64 * 3)(), (C.c_int64 * 3)()
+    off, adj = np.ascontiguousarray(off, np.int64), np.ascontiguousarray(adj, np.int32)
+    lib.plan_probe(C.c_int32(mode), C.byref(s), C.c_int32(len(off) - 1), C.c_void_p(off.ctypes.data),
+                   C.c_void_p(adj.ctypes.data), C.c_int32(skip_lower), jobs, caps)
+    return list(jobs), list(caps)
+
+
+def _rows(n, lens, seed, sym=False):
+    """Rows of the given lengths at the first vertices, their entries drawn from the
+    first 2 len(lens) vertices or more, and short rows elsewhere."""
+    rng = np.random.default_rng(seed)
+    top = max(max(lens) + 1, 2 * len(lens))
+    rows = [rng.permutation(min(top, n))[:k] for k in lens]
+    u = np.concatenate([np.full(len(r), i) for i, r in enumerate(rows)] + [np.arange(len(lens), n)] * 2)
+    v = np.concatenate(rows + [rng.integers(0, n, n - len(lens)) for _ in range(2)])
+    if sym:
+        return O.canon_csr(n, u.astype(np.int32), v.astype(np.int32))
+    key = np.unique(u * n + v)
+    off = np.concatenate([[0], np.cumsum(np.bincount(key // n, minlength=n))]).astype(np.int64)
+    return off, (key % n).astype(np.int32)
+
+
+@pytest.mark.parametrize("mode", [DIRECT, ORIENTED, BY_TASKS])
+@pytest.mark.parametrize("longest", [63, 64, 65, 66, 127, 129, 300, 511, 512, 513, 600, 4095, 4097, 9000])
+@pytest.mark.parametrize("many", [66, 129])
+def test_every_job_has_room(mode, longest, many):
+    """One row of the longest length, many of a bin's least, as the planner meets
+    them: a job for every owner at least."""
+    n = 9000
+    lens = [longest] + [min(many, longest)] * 1200
+    off, adj = _rows(n, lens, longest, mode == ORIENTED)
+    for skip in (0, 1):
+        for kw in ({}, {"policy": T.POLICY_LEARNED}, {"small_max": 1, "mid_max": 1}, {"small_max": 8, "mid_max": 40},
+                   {"job_items": 1, "flush_items": 1}, {"mid_max": 128}):
+            jobs, caps = _plan(mode, off, adj, skip, **kw)
+            assert all(j <= c for j, c in zip(jobs, caps)), (kw, jobs, caps)
+            assert sum(jobs) > 0
+
+
+@pytest.mark.parametrize("n", [16385, 200000, (1 << 20) + 1])
+def test_many_middle_rows_and_one_longer(n):
+    """Directed rows, most of 66 entries: their owners all get jobs of the largest
+    bin where there is no middle one."""
+    lens = [600] + [66] * min(5000, n // 4)
+    off, adj = _rows(n, lens, 7)
+    jobs, caps = _plan(BY_TASKS, off, adj)
+    assert all(j <= c for j, c in zip(jobs, caps)), (jobs, caps)
+    assert max(jobs[1], jobs[2]) > len(lens) // 2
