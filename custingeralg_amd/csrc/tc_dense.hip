@@ -8,7 +8,7 @@
 // any rows (loops, asymmetric ones, the CSR convention), needs no rank order,
 // no task lists and no plan whose sizes the host must read, and runs as two
 // kernels where the oriented count takes more than fifty launches.
-#include "tc_internal.hpp"
+#include "tc_plan.hpp"
 
 #include <algorithm>
 
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(kRowWaves * kWave) void k_dense_rows(DenseArgs A)
     }
 }
 
-// One wave, entries [e0, e1) of row v: the hits of this lane.  Eight lanes
+// One wave, entries [e0, e1) of row v (at least one): the hits of this lane.  Eight lanes
 // share an entry u: each reads 16 bytes of every 128-byte line of u's bit row
 // (whole lines, no reduction per entry) against the same words of v's row,
 // kept in registers for CH of the lines [c0, c1) at a time; U entries per
@@ -170,7 +170,7 @@ __device__ inline uint32_t dense_row(const DenseArgs &A, const DenseGraph &D, in
             S[c] = *reinterpret_cast<const uint4 *>(m + (lv * rb + cb + c * 128));
         int32_t nu[U];  // the next entries, loaded while these rows are
 #pragma unroll
-        for (int q = 0; q < U; ++q) nu[q] = row[min(e0 + grp + q * 8, e1 - 1)];
+        for (int q = 0; q < U; ++q) nu[q] = row[dense_entry(e0 + grp + q * 8, e1)];
 #pragma unroll 1
         for (int32_t eb = e0 + grp; eb - grp < e1; eb += 8 * U) {
             uint32_t u[U];
@@ -179,7 +179,7 @@ __device__ inline uint32_t dense_row(const DenseArgs &A, const DenseGraph &D, in
 #pragma unroll
             for (int q = 0; q < U; ++q) {
                 u[q] = (uint32_t)(nu[q] - D.v0);
-                nu[q] = row[min(eb + (U + q) * 8, e1 - 1)];
+                nu[q] = row[dense_entry(eb + (U + q) * 8, e1)];
             }
 #pragma unroll
             for (int q = 0; q < U; ++q) {
@@ -264,9 +264,8 @@ __global__ __launch_bounds__(256, 8) void k_dense_count(DenseArgs A)
         const int32_t v = (int32_t)r, d = A.len[v];
         if (d > A.long_len) continue;
         const DenseGraph D = graph_of_row(A, v);
-        const uint32_t h = (d >= 2 || A.check_sym) ? dense_part(A, D, v, 0, d, miss) : 0u;
+        const uint32_t h = dense_walked(d, A.check_sym) ? dense_part(A, D, v, 0, d, miss) : 0u;
         if (lane == 0) {
-            // (a row of one entry counts nothing: the reference skips it)
             A.out[v] = d >= 2 ? h : 0u;
             total += d >= 2 ? h : 0u;
         }

@@ -1,7 +1,7 @@
-// tc_plan.hpp -- how an owner's work is cut into jobs: the rule of the
-// planner's kernels, and the host's bounds on what it gives, which the job
-// arrays are sized by.  Both stand here so that one can be checked against the
-// other without a device (tests/cpp/plan_test.hip).
+// tc_plan.hpp -- rules that kernels and host share, and that are checked
+// without a device (tests/cpp/plan_test.hip): how an owner's work is cut into
+// jobs beside the host's bounds on them, which the job arrays are sized by, and
+// the entries that a bit-row count loads.
 #pragma once
 
 #include "tc_internal.hpp"
@@ -155,5 +155,17 @@ inline void plan_caps(const PlanParams &P, int32_t nv, int64_t lists, int64_t lm
         if (b == 2 && any) cap[b] += P.id_tiles > 0 ? owners * P.id_tiles : 2 * (lists / P.lmax[2]);
     }
 }
+
+// Bit rows (tc_dense.hip): whether a row of d entries is walked.  A row of one
+// entry counts nothing (the reference skips it) but is looked at for its
+// reverse; an empty one has no entry to load.
+__host__ __device__ inline bool dense_walked(int32_t d, int32_t check_sym)
+{
+    return d >= 2 || (check_sym && d == 1);
+}
+
+// The place that entry e of the part that ends at e1 is loaded from: past the end
+// the last entry again.
+__host__ __device__ inline int32_t dense_entry(int32_t e, int32_t e1) { return e < e1 ? e : e1 - 1; }
 
 }  // namespace tc

@@ -1,6 +1,5 @@
-// The planner's rule applied to a CSR on the host, owner by owner as the
-// kernels apply it, beside the capacities that its job arrays get.  Loaded by
-// tests/test_plan.py; nothing here touches a device.
+// Rules that kernels and host share, on the host.  Loaded by tests/test_plan.py;
+// nothing here touches a device.
 #include "../../custingeralg_amd/csrc/tc_plan.hpp"
 
 #include <numeric>
@@ -8,6 +7,8 @@
 
 using namespace tc;
 
+// The planner's rule applied to a CSR, owner by owner as the kernels apply it,
+// beside the capacities that the job arrays get.
 // mode: kDirect, kOriented or kByTasks.  Rows sorted, distinct; oriented ones
 // symmetric and loop-free.  jobs[b], caps[b]: jobs of bin b, and room for them.
 extern "C" int plan_probe(int32_t mode, const tc_schedule *sched, int32_t nv, const int64_t *off,
@@ -65,4 +66,23 @@ extern "C" int plan_probe(int32_t mode, const tc_schedule *sched, int32_t nv, co
         jobs[b] += (int64_t)owner_split(L[v], T, work[v], b, plan_wmin(total), P) * owner_tiles(L[v], b, P);
     }
     return TC_OK;
+}
+
+// The least and the largest place that a bit-row count loads of a row of d entries
+// (none: 0, -1), in the order of dense_row: 8 groups, U entries each in flight.
+extern "C" void dense_probe(int32_t d, int32_t check_sym, int32_t U, int32_t *lo, int32_t *hi)
+{
+    *lo = 0;
+    *hi = -1;
+    if (!dense_walked(d, check_sym)) return;
+    auto load = [&](int32_t e) {
+        const int32_t k = dense_entry(e, d);
+        *lo = std::min(*lo, k);
+        *hi = std::max(*hi, k);
+    };
+    for (int32_t grp = 0; grp < 8; ++grp) {
+        for (int32_t q = 0; q < U; ++q) load(grp + q * 8);
+        for (int32_t eb = grp; eb - grp < d; eb += 8 * U)
+            for (int32_t q = 0; q < U; ++q) load(eb + (U + q) * 8);
+    }
 }

@@ -1,5 +1,6 @@
-"""The capacities of the job arrays against the jobs that the planner's rule
-gives, on the host: row lengths around every bin's bounds, in each mode."""
+"""Rules that kernels and host share, on the host: the capacities of the job
+arrays against the jobs that the planner's rule gives, with row lengths around
+every bin's bounds, in each mode; the entries that a bit-row count loads."""
 from __future__ import annotations
 
 import ctypes as C
@@ -66,3 +67,15 @@ def test_many_middle_rows_and_one_longer(n):
     jobs, caps = _plan(BY_TASKS, off, adj)
     assert all(j <= c for j, c in zip(jobs, caps)), (jobs, caps)
     assert max(jobs[1], jobs[2]) > len(lens) // 2
+
+
+@pytest.mark.parametrize("check_sym", [0, 1])
+@pytest.mark.parametrize("unroll", [1, 2, 4])
+def test_bit_rows_load_their_own_entries(check_sym, unroll):
+    """No place outside the row, and every row of two entries or more is loaded."""
+    lib = C.CDLL(_LIB)
+    for d in range(200):
+        lo, hi = C.c_int32(), C.c_int32()
+        lib.dense_probe(C.c_int32(d), C.c_int32(check_sym), C.c_int32(unroll), C.byref(lo), C.byref(hi))
+        assert lo.value == 0 and hi.value < d, d
+        assert d < 2 or hi.value == d - 1
