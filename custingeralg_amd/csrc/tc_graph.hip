@@ -782,16 +782,7 @@ void graph_destroy(Graph *g)
         g->st.pool.p = nullptr;
         g->st.pool.bytes = 0;
     }
-    DevBuf *bufs[] = {&g->st.boff, &g->st.len, &g->st.cap, &g->st.pool, &g->vinfo, &g->padj,
-                      &g->coff, &g->crow, &g->work, &g->jobs, &g->tmp, &g->tmp2, &g->tmp3, &g->tmp4,
-                      &g->accum, &g->bsrc, &g->bdst, &g->bflag, &g->bkeys, &g->bkeys2,
-                      &g->bvals2, &g->boffb, &g->bdel, &g->hrow, &g->flagpool, &g->vmark, &g->order,
-                      &g->rnk, &g->tasks, &g->pcnt, &g->hjobs, &g->outr, &g->dmat, &g->ditems,
-                      &g->dgraphs, &g->dgid, &g->cmat, &g->cgraphs, &g->cblocks};
-    for (DevBuf *b : bufs) b->release(idle);
-    for (DevBuf &b : g->sb) b.release(idle);
-    for (DevBuf &b : g->ov) b.release(idle);
-    for (DevBuf &b : g->lbuf) b.release(idle);
+    g->each_buffer([&](DevBuf &b) { b.release(idle); });
     g->drop_events();
     g->drop_capture();
     if (g->bexec) (void)hipGraphExecDestroy(g->bexec);

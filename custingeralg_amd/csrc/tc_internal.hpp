@@ -205,7 +205,10 @@ struct Graph {
     hipStream_t cap_stream = nullptr;
     hipGraph_t cgraph = nullptr;
     hipGraphExec_t cexec = nullptr;
-    uint64_t cexec_key = 0;
+    // the buffers' addresses at the recording (its launches hold them: a count
+    // with another schedule may have moved a buffer since), and its method
+    uint64_t cexec_key = 0, cexec_layout = 0;
+    int cexec_method = 0;
     // recorded batch sequences (tc_batch_apply with tc_schedule.capture):
     // one per size class and buffer layout, keyed like the counts
     hipGraph_t bgraph = nullptr;
@@ -214,6 +217,30 @@ struct Graph {
     bool bplan_valid = false;
     bool bcap_failed = false;  // a recording failed: batches run plainly
     void drop_capture();
+    // Every buffer of the handle.
+    template <class F> void each_buffer(F f)
+    {
+        DevBuf *one[] = {&st.boff, &st.len, &st.cap, &st.pool, &vinfo, &padj, &coff, &crow, &work, &jobs, &tmp,
+                         &tmp2, &tmp3, &tmp4, &accum, &order, &rnk, &tasks, &hjobs, &outr, &pcnt, &bsrc, &bdst,
+                         &bflag, &bkeys, &bkeys2, &bvals2, &boffb, &bdel, &hrow, &flagpool, &vmark, &dmat, &ditems,
+                         &dgraphs, &dgid, &cmat, &cgraphs, &cblocks};
+        for (DevBuf *b : one) f(*b);
+        for (DevBuf &b : ov) f(b);
+        for (DevBuf &b : sb) f(b);
+        for (DevBuf &b : lbuf) f(b);
+    }
+    // A hash of the buffers' addresses and sizes.
+    uint64_t layout()
+    {
+        uint64_t h = 1469598103934665603ull;
+        each_buffer([&](const DevBuf &b) {
+            for (uint64_t x : {(uint64_t)(uintptr_t)b.p, (uint64_t)b.bytes}) {
+                h = (h ^ x) * 0x9E3779B97F4A7C15ull;
+                h ^= h >> 29;
+            }
+        });
+        return h;
+    }
     void touch()  // the store changed
     {
         ++version;

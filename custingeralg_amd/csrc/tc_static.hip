@@ -3751,8 +3751,9 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     return TC_OK;
 }
 
-// Key of a recorded count: everything its launches bake in (schedule,
-// output, learned table, statistics on or off, the store's version).
+// Key of a recorded count: what its launches bake in (schedule, output, learned
+// table, statistics on or off, the store's version) besides the addresses of
+// the handle's buffers (Graph::layout).
 uint64_t plan_key(const Graph &g, const uint32_t *out, const tc_schedule &sched, bool with_stats,
                   bool skip_lower)
 {
@@ -3787,7 +3788,7 @@ int count_replay(Graph &g, uint64_t *global, tc_stats *stats)
     const unsigned long long *hacc = g.hcounts;
     TC_HIP(hipMemcpyAsync(g.hcounts, g.accum.p, 32 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
     TC_HIP(hipStreamSynchronize(s));
-    if (g.plan.method == TC_METHOD_ORIENTED && hacc[27]) {  // cannot happen for an unchanged store that counted before
+    if (g.cexec_method == TC_METHOD_ORIENTED && hacc[27]) {  // cannot happen for an unchanged store that counted before
         g.symmetric = 0;
         g.touch();
         set_last_error(TC_ERR_INVALID, "oriented layout: the rows are not symmetric");
@@ -3796,11 +3797,11 @@ int count_replay(Graph &g, uint64_t *global, tc_stats *stats)
     if (global) *global = hacc[0];
     if (stats) {
         tc_stats st = {};
-        fill_counters(st, hacc, g.plan.method == TC_METHOD_ORIENTED);
+        fill_counters(st, hacc, g.cexec_method == TC_METHOD_ORIENTED);
         float ms = 0;
         (void)hipEventElapsedTime(&ms, g.ev[0], g.ev[7]);
         st.ms_total = ms;
-        st.method_used = g.plan.method;
+        st.method_used = g.cexec_method;
         st.graph_replay = 1;
         *stats = st;
     }
@@ -3848,6 +3849,8 @@ int count_capture(Graph &g, uint32_t *out, const tc_schedule &sched, tc_stats *s
     g.cgraph = graph;
     g.cexec = exec;
     g.cexec_key = key;
+    g.cexec_layout = g.layout();
+    g.cexec_method = g.plan.method;
     return TC_OK;
 }
 
@@ -3859,7 +3862,10 @@ int static_count(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &s
     if (!sched.capture || g.st.nv == 0 || g.st.nnz == 0)
         return count_pass(g, out, global, sched, stats, skip_lower);
     const uint64_t key = plan_key(g, out, sched, stats != nullptr, skip_lower);
-    if (g.cexec && g.cexec_key == key) return count_replay(g, global, stats);
+    if (g.cexec && g.cexec_key == key) {
+        if (g.cexec_layout == g.layout()) return count_replay(g, global, stats);
+        g.plan.valid = false;  // a plain pass sizes the buffers again
+    }
     if (g.plan.valid && g.plan.key == key) {
         if (count_capture(g, out, sched, stats, skip_lower, key) == TC_OK)
             return count_replay(g, global, stats);
