@@ -40,7 +40,7 @@ MLP_PARAMS = MLP_IN * MLP_HIDDEN + MLP_HIDDEN + MLP_HIDDEN * MLP_HIDDEN + MLP_HI
 # every symbol include/custinger_tc.h declares (checked by the CPU tests)
 EXPORTS = [
     "tc_last_error", "tc_status_string", "tc_version", "tc_device_alloc", "tc_device_free",
-    "tc_memcpy", "tc_memset", "tc_device_synchronize", "tc_device_name",
+    "tc_memcpy", "tc_memset", "tc_device_synchronize", "tc_device_trim", "tc_device_name",
     "tc_graph_create_csr", "tc_graph_destroy", "tc_graph_set_stream", "tc_graph_get_info",
     "tc_graph_to_csr", "tc_graph_degrees", "tc_schedule_default", "tc_static_count",
     "tc_csr_count_device", "tc_batch_apply", "tc_batch_update_only", "tc_batch_prepare",
@@ -191,6 +191,12 @@ def device_name() -> str:
 
 def synchronize() -> None:
     check(lib().tc_device_synchronize())
+
+
+def device_trim() -> None:
+    """Frees the device blocks that closed handles left with the library (up to
+    4 GiB), for another allocator in the process."""
+    check(lib().tc_device_trim())
 
 
 # ------------------------------------------------------------ device arrays

@@ -96,15 +96,7 @@ int tc_version(void) { return 10000; }
 int tc_device_alloc(void **ptr, uint64_t bytes)
 {
     TC_CHECK_ARG(ptr, "tc_device_alloc: null ptr");
-    hipError_t e = hipMalloc(ptr, bytes ? bytes : 16);
-    if (e == hipErrorOutOfMemory) {  // the pool's blocks go first
-        (void)hipGetLastError();
-        tc::pool_flush();
-        e = hipMalloc(ptr, bytes ? bytes : 16);
-    }
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        *ptr = nullptr;
+    if (tc::device_malloc(ptr, bytes ? bytes : 16) != hipSuccess) {
         tc::set_last_error(TC_ERR_OOM, "hipMalloc failed");
         return TC_ERR_OOM;
     }
@@ -115,6 +107,12 @@ int tc_device_free(void *ptr)
 {
     if (!ptr) return TC_OK;
     TC_HIP(hipFree(ptr));
+    return TC_OK;
+}
+
+int tc_device_trim(void)
+{
+    tc::pool_flush();
     return TC_OK;
 }
 

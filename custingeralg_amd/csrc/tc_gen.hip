@@ -246,7 +246,7 @@ int canon_csr_device(int32_t nv, int64_t m, const int32_t *u, const int32_t *v, 
         pos.release();
     };
     int st = TC_OK;
-    if (hipMalloc(&off, (size_t)(nv + 1) * sizeof(int64_t)) != hipSuccess) {
+    if (device_malloc((void **)&off, (size_t)(nv + 1) * sizeof(int64_t)) != hipSuccess) {
         set_last_error(TC_ERR_OOM, "canon: offsets");
         return TC_ERR_OOM;
     }
@@ -271,7 +271,7 @@ int canon_csr_device(int32_t nv, int64_t m, const int32_t *u, const int32_t *v, 
             set_last_error(st, "canon: nnz readback");
             goto fail;
         }
-        if (hipMalloc(&adj, (size_t)(nnz > 0 ? nnz : 1) * sizeof(int32_t)) != hipSuccess) {
+        if (device_malloc((void **)&adj, (size_t)(nnz > 0 ? nnz : 1) * sizeof(int32_t)) != hipSuccess) {
             st = TC_ERR_OOM;
             set_last_error(st, "canon: adjacency");
             goto fail;
@@ -281,7 +281,7 @@ int canon_csr_device(int32_t nv, int64_t m, const int32_t *u, const int32_t *v, 
                                keys.as<uint64_t>(), flag.as<int32_t>(), pos.as<int64_t>(), n, bits_v,
                                nv, adj, off);
     } else {
-        if (hipMalloc(&adj, sizeof(int32_t)) != hipSuccess) {
+        if (device_malloc((void **)&adj, sizeof(int32_t)) != hipSuccess) {
             st = TC_ERR_OOM;
             goto fail;
         }

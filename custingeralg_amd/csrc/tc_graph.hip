@@ -27,7 +27,7 @@ void set_last_error(int code, const std::string &msg)
 // size and device, and handed to the next handle.
 //   Bounded: kHoldBytes in all, no block above kHoldBlock; what exceeds it is
 //   freed, the largest first, and everything held is freed when an allocation
-//   fails.
+//   of this library fails, or by the caller (tc_device_trim).
 //   Safe across streams and threads: a block is given back only when its
 //   device is idle (DevBuf::release synchronises, as hipFree does), so no
 //   kernel of its last owner can still touch it; the lists are under a lock.
@@ -119,6 +119,21 @@ void pool_flush()
     for (void *q : out) (void)hipFree(q);
 }
 
+hipError_t device_malloc(void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        pool_flush();
+        e = hipMalloc(p, bytes);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        *p = nullptr;
+    }
+    return e;
+}
+
 int DevBuf::ensure(size_t need)
 {
     if (need == 0) need = 16;
@@ -134,15 +149,7 @@ int DevBuf::ensure(size_t need)
     size_t got = want;
     p = pool_take(dev, want, got);
     if (!p) {
-        hipError_t e = hipMalloc(&p, want);
-        if (e == hipErrorOutOfMemory) {
-            (void)hipGetLastError();
-            pool_flush();
-            e = hipMalloc(&p, want);
-        }
-        if (e != hipSuccess) {
-            p = nullptr;
-            (void)hipGetLastError();
+        if (device_malloc(&p, want) != hipSuccess) {
             set_last_error(TC_ERR_OOM, "hipMalloc of " + std::to_string(need) + " bytes failed");
             return TC_ERR_OOM;
         }

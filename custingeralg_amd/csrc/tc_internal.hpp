@@ -55,6 +55,8 @@ struct DevBuf {
 
 // Frees every block that the pool holds.
 void pool_flush();
+// hipMalloc; where it finds no memory, the pool's blocks go first.
+hipError_t device_malloc(void **p, size_t bytes);
 
 // ------------------------------------------------------------- helpers --
 __host__ __device__ inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }

@@ -612,8 +612,8 @@ int model_load(const float *params_host)
             return TC_ERR_INVALID;
         }
     if (!g_learn.wb) {
-        TC_HIP(hipMalloc(&g_learn.wb, NP * sizeof(uint16_t)));
-        TC_HIP(hipMalloc(&g_learn.table, kTableDim * kTableDim));
+        TC_HIP(device_malloc((void **)&g_learn.wb, NP * sizeof(uint16_t)));
+        TC_HIP(device_malloc((void **)&g_learn.table, kTableDim * kTableDim));
     }
     std::vector<uint16_t> hb(NP);
     for (int i = 0; i < NP; ++i) hb[i] = f32_to_bf16(params_host[i]);
@@ -647,8 +647,8 @@ int strategy_table_set(const uint8_t *table, int32_t dim)
             return TC_ERR_INVALID;
         }
     if (!g_learn.wb) {
-        TC_HIP(hipMalloc(&g_learn.wb, NP * sizeof(uint16_t)));
-        TC_HIP(hipMalloc(&g_learn.table, kTableDim * kTableDim));
+        TC_HIP(device_malloc((void **)&g_learn.wb, NP * sizeof(uint16_t)));
+        TC_HIP(device_malloc((void **)&g_learn.table, kTableDim * kTableDim));
     }
     TC_HIP(hipMemcpy(g_learn.table, table, kTableDim * kTableDim, hipMemcpyHostToDevice));
     g_learn.ready = true;

@@ -160,7 +160,7 @@ public:
         }
         if (n + 1 > cap_) {
             Release();
-            if (hipMalloc(&pre_, (size_t)(n + 1) * sizeof(int64_t)) != hipSuccess) {
+            if (tc_device_alloc((void **)&pre_, (size_t)(n + 1) * sizeof(int64_t)) != TC_OK) {
                 pre_ = nullptr;
                 return TC_ERR_OOM;
             }
@@ -220,8 +220,8 @@ public:
     int Init(int64_t maxLen)
     {
         Free();
-        if (hipMalloc(&items_, (size_t)(maxLen > 0 ? maxLen : 1) * sizeof(int32_t)) != hipSuccess ||
-            hipMalloc(&end_, sizeof(unsigned long long)) != hipSuccess) {
+        if (tc_device_alloc((void **)&items_, (size_t)(maxLen > 0 ? maxLen : 1) * sizeof(int32_t)) != TC_OK ||
+            tc_device_alloc((void **)&end_, sizeof(unsigned long long)) != TC_OK) {
             Free();
             return TC_ERR_OOM;
         }

@@ -73,8 +73,12 @@ typedef struct tc_graph tc_graph;
  * (0 = exact fit; blocks still round up to a power of two when they grow). */
 int tc_graph_create_csr(int32_t nv, int64_t nnz, const int64_t *off, const int32_t *adj,
                         int location, uint32_t flags, int32_t slack_pct, tc_graph **out);
-/* cuStinger::freecuStinger (tests/cct.cpp:281). */
+/* cuStinger::freecuStinger (tests/cct.cpp:281).  Up to 4 GiB of the device
+ * blocks of closed handles stay with the library for the next handles (none
+ * above 1 GiB).  They are given back when an allocation of the library finds
+ * no memory, or by tc_device_trim, for another allocator in the process. */
 int tc_graph_destroy(tc_graph *g);
+int tc_device_trim(void);
 /* Bind the handle to a HIP stream (NULL = the default stream). */
 int tc_graph_set_stream(tc_graph *g, void *hip_stream);
 

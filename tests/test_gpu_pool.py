@@ -2,6 +2,7 @@
 counts stay exact from several threads at once, with updates in between."""
 from __future__ import annotations
 
+import ctypes as C
 import threading
 
 import numpy as np
@@ -41,3 +42,29 @@ def test_handles_from_several_threads():
     for t in threads:
         t.join()
     assert not faults
+
+
+def test_trim_gives_the_blocks_back():
+    """A closed handle's blocks stay with the library until they are asked for."""
+
+    def free():
+        f, t = C.c_size_t(), C.c_size_t()
+        assert T.lib().hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+
+    T.device_trim()
+    free0 = free()
+    off, adj = O.rmat_graph(17, 24, 3)
+    g = T.cuStinger(off, adj)
+    pv, _, _ = T.static_count(g)
+    held = free0 - free()
+    assert held > 100 << 20
+    g.close()
+    assert free0 - free() > held // 2
+    T.device_trim()
+    # (what the runtime keeps for itself: code objects, small blocks)
+    assert free0 - free() < held // 4
+    g = T.cuStinger(off, adj)
+    again, _, _ = T.static_count(g)
+    g.close()
+    assert np.array_equal(pv, again)
