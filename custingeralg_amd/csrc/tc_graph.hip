@@ -53,7 +53,11 @@ struct BlockPool {
 // Never destroyed: at exit the runtime may be gone before a destructor runs.
 BlockPool &block_pool()
 {
-    static BlockPool *p = new BlockPool;
+    static BlockPool *p = [] {
+        BlockPool *q = new BlockPool;
+        q->kits.reserve(kHoldKits);
+        return q;
+    }();
     return *p;
 }
 
@@ -82,41 +86,51 @@ void *pool_take(int dev, size_t bytes, size_t &got)
     return p;
 }
 
-void pool_give(int dev, void *p, size_t bytes)
+// Takes a block over: it is kept, or freed where host memory is short or the
+// pool would hold too much.  (Nothing here throws: handles are closed from
+// destructors and from C.)
+void pool_give(int dev, void *p, size_t bytes) noexcept
 {
-    std::vector<void *> out;
-    if (bytes > kHoldBlock) {
-        out.push_back(p);
-    } else {
-        BlockPool &P = block_pool();
+    BlockPool &P = block_pool();
+    bool kept = false;
+    if (bytes <= kHoldBlock) {
         std::lock_guard<std::mutex> lock(P.mu);
-        P.blocks.insert({{dev, bytes}, p});
-        P.held += bytes;
-        while (P.held > kHoldBytes) {
+        try {
+            P.blocks.insert({{dev, bytes}, p});
+            P.held += bytes;
+            kept = true;
+        } catch (...) {
+        }
+    }
+    if (!kept) (void)hipFree(p);
+    for (;;) {
+        void *out = nullptr;
+        {
+            std::lock_guard<std::mutex> lock(P.mu);
+            if (P.held <= kHoldBytes) return;
             auto big = P.blocks.begin();
             for (auto it = P.blocks.begin(); it != P.blocks.end(); ++it)
                 if (it->first.second > big->first.second) big = it;
             P.held -= big->first.second;
-            out.push_back(big->second);
+            out = big->second;
             P.blocks.erase(big);
         }
+        (void)hipFree(out);
     }
-    for (void *q : out) (void)hipFree(q);
 }
 
 }  // namespace
 
-void pool_flush()
+void pool_flush() noexcept
 {
-    std::vector<void *> out;
+    BlockPool &P = block_pool();
+    decltype(P.blocks) out;
     {
-        BlockPool &P = block_pool();
         std::lock_guard<std::mutex> lock(P.mu);
-        for (auto &b : P.blocks) out.push_back(b.second);
-        P.blocks.clear();
+        out.swap(P.blocks);
         P.held = 0;
     }
-    for (void *q : out) (void)hipFree(q);
+    for (auto &b : out) (void)hipFree(b.second);
 }
 
 hipError_t device_malloc(void **p, size_t bytes)

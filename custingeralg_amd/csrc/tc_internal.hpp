@@ -54,7 +54,7 @@ struct DevBuf {
 };
 
 // Frees every block that the pool holds.
-void pool_flush();
+void pool_flush() noexcept;
 // hipMalloc; where it finds no memory, the pool's blocks go first.
 hipError_t device_malloc(void **p, size_t bytes);
 
