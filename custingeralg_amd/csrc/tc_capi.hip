@@ -116,6 +116,13 @@ int tc_device_trim(void)
     return TC_OK;
 }
 
+// (not in the header: for the tests)
+int tc_test_block_limit(uint64_t bytes)
+{
+    tc::block_limit = (size_t)bytes;
+    return TC_OK;
+}
+
 int tc_memcpy(void *dst, const void *src, uint64_t bytes, int kind)
 {
     if (!bytes) return TC_OK;

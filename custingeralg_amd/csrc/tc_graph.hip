@@ -133,8 +133,14 @@ void pool_flush() noexcept
     for (auto &b : out) (void)hipFree(b.second);
 }
 
+thread_local size_t block_limit = 0;
+
 hipError_t device_malloc(void **p, size_t bytes)
 {
+    if (block_limit && bytes > block_limit) {
+        *p = nullptr;
+        return hipErrorOutOfMemory;
+    }
     hipError_t e = hipMalloc(p, bytes);
     if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
@@ -161,7 +167,7 @@ int DevBuf::ensure(size_t need)
     (void)hipGetDevice(&dev);
     const size_t want = block_size(need);
     size_t got = want;
-    p = pool_take(dev, want, got);
+    p = block_limit && want > block_limit ? nullptr : pool_take(dev, want, got);
     if (!p) {
         if (device_malloc(&p, want) != hipSuccess) {
             set_last_error(TC_ERR_OOM, "hipMalloc of " + std::to_string(need) + " bytes failed");

@@ -57,6 +57,9 @@ struct DevBuf {
 void pool_flush() noexcept;
 // hipMalloc; where it finds no memory, the pool's blocks go first.
 hipError_t device_malloc(void **p, size_t bytes);
+// For tests of what happens then: blocks of more bytes find no memory in this
+// thread (tc_test_block_limit, 0: no limit).
+extern thread_local size_t block_limit;
 
 // ------------------------------------------------------------- helpers --
 __host__ __device__ inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }

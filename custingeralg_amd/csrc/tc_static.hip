@@ -3445,7 +3445,7 @@ int prepare_direct_tasks(Graph &g, bool skip_lower)
     return TC_OK;
 }
 
-// The per-bin counters of a count (accum words, see count_pass) into stats.
+// The per-bin counters of a count (accum words, see count_once) into stats.
 void fill_counters(tc_stats &st, const unsigned long long *hacc, bool oriented)
 {
     const unsigned long long *jt = hacc + 28;
@@ -3473,8 +3473,10 @@ void fill_counters(tc_stats &st, const unsigned long long *hacc, bool oriented)
 // One count.  While g.capturing (stream capture of a hipGraph), the values
 // the host would read back come from g.plan, and no event is recorded and
 // nothing is read back: the caller reads the results after the replay.
-int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sched,
-               tc_stats *stats, bool skip_lower)
+// lean: without bit matrices, core and direct task lists, whose memory the other
+// routes do without; *spare is set where one of them was taken.
+int count_once(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sched,
+               tc_stats *stats, bool skip_lower, bool lean, bool *spare)
 {
     const int32_t nv = g.st.nv;
     const int64_t nnz = g.st.nnz;
@@ -3506,7 +3508,8 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     TC_TRY(g.accum.ensure(32 * sizeof(unsigned long long)));
     unsigned long long *acc = g.accum.as<unsigned long long>();
     const bool rows = nnz > 0 && rows_eligible(g, sched);
-    const bool dense = rows || (nnz > 0 && dense_eligible(g, sched));
+    const bool dense = rows || (nnz > 0 && !lean && dense_eligible(g, sched));
+    *spare = dense && !rows;
     uint32_t *outp = out;
     if (!outp) {
         TC_TRY(g.tmp4.ensure((size_t)std::max<int32_t>(nv, 1) * sizeof(uint32_t)));
@@ -3570,16 +3573,20 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
     // compact offsets, chunk rows and the (degree-partitioned) vertex views;
     // rows declared symmetric that turn out not to be go the direct way, after
     // a count that finds no jobs
-    if (oriented) TC_TRY(prepare_views(g, true, sched.hub_degree, sched.build, core_size(g, sched)));
+    const int32_t core_k = oriented && !lean ? core_size(g, sched) : 0;
+    *spare = core_k > 0;
+    if (oriented) TC_TRY(prepare_views(g, true, sched.hub_degree, sched.build, core_k));
     if (!oriented) TC_TRY(prepare_views(g, false));
     int mode = oriented ? kOriented : kDirect;
-    if (!oriented && direct_by_tasks(g, sched)) {
+    if (!oriented && !lean && direct_by_tasks(g, sched)) {
+        *spare = true;
         const int dt = prepare_direct_tasks(g, skip_lower);
         if (dt == TC_OK) {
             mode = kByTasks;
         } else if (dt == TC_ERR_OOM) {  // no room for the lists: the row entries themselves
             g.tasks.release();
             g.ov[16].release();
+            g.ov[18].release();
             TC_TRY(build_direct_vinfo(g));
         } else {
             return dt;
@@ -3719,7 +3726,7 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
         if (g.batch_per_graph)
             hipLaunchKernelGGL(k_fill_u64, dim3(grid_for(g.batch_ngraphs, 256, 4096)), dim3(256), 0, s,
                                g.batch_per_graph, (int64_t)g.batch_ngraphs);
-        return count_pass(g, out, global, sched, stats, skip_lower);  // the direct way
+        return count_once(g, out, global, sched, stats, skip_lower, lean, spare);  // the direct way
     }
     for (int b = 0; b < 3; ++b)
         if ((int64_t)hacc[28 + b] > J.cap[b]) {  // (plan_caps bounds them: a fault of the planner)
@@ -3749,6 +3756,20 @@ int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
         *stats = st;
     }
     return TC_OK;
+}
+
+int count_pass(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sched, tc_stats *stats,
+               bool skip_lower)
+{
+    bool spare = false;
+    const int st = count_once(g, out, global, sched, stats, skip_lower, false, &spare);
+    if (st != TC_ERR_OOM || !spare || g.capturing) return st;
+    // what these routes hold goes back, and the count is done without them
+    for (DevBuf *b : {&g.dmat, &g.ditems, &g.cmat, &g.tasks, &g.ov[16], &g.ov[18]}) b->release();
+    if (g.batch_per_graph)
+        hipLaunchKernelGGL(k_fill_u64, dim3(grid_for(g.batch_ngraphs, 256, 4096)), dim3(256), 0, g.stream,
+                           g.batch_per_graph, (int64_t)g.batch_ngraphs);
+    return count_once(g, out, global, sched, stats, skip_lower, true, &spare);
 }
 
 // Key of a recorded count: what its launches bake in (schedule, output, learned
