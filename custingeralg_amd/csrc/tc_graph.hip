@@ -531,7 +531,8 @@ int validate_graph(Graph &g, bool check_symmetry, int64_t *bad_rows)
     g.max_degree = (int32_t)h[4];
     g.degree_stale = false;
     // bit matrices hold a graph's own columns only
-    if (h[5]) {
+    g.batch_cross = h[5] != 0;
+    if (g.batch_cross) {
         g.dense_words = 0;
         g.core_total = 0;
     }

@@ -176,6 +176,7 @@ struct Graph {
     DevBuf cgraphs, cblocks;
     int32_t core_total = 0, core_blocks = 0;
     int64_t dense_words = 0;
+    bool batch_cross = false;  // batched graphs: some entry leaves its graph
     DevBuf lbuf[5];  // delta: items, their prefix, per-edge counts, merge segments, their prefix
     bool degree_stale = false;
     // batched counting: graph boundaries and per-graph output (device)

@@ -132,12 +132,20 @@ inline PlanParams plan_params(const tc_schedule &sched, int mode, bool batched, 
 }
 
 // A bound on the longest owner list of a count (max_degree: the longest row, or a
-// bound on it).  An entry of N+ points to a row no shorter than its own, so that
-// |N+| <= sqrt(nnz).
-inline int64_t longest_list(bool oriented, int32_t nv, int64_t nnz, int64_t max_degree)
+// bound on it).  In the order by degree an entry of N+ points to a row no shorter
+// than its own, so that |N+| <= sqrt(nnz); in that by graph and degree too, unless
+// entries leave their graph.
+inline int64_t longest_list(bool by_degree, int32_t nv, int64_t nnz, int64_t max_degree)
 {
     const int64_t most = std::min<int64_t>(nv, max_degree);
-    return oriented ? std::min<int64_t>(most, (int64_t)std::sqrt((double)nnz) + 1) : most;
+    return by_degree ? std::min<int64_t>(most, (int64_t)std::sqrt((double)nnz) + 1) : most;
+}
+
+inline int64_t longest_list(const Graph &g, bool oriented)
+{
+    const int32_t nv = g.st.nv;
+    return longest_list(oriented && !g.batch_cross, nv, g.st.nnz,
+                        g.validated && !g.degree_stale ? g.max_degree : nv);
 }
 
 // The most jobs that the owners of each bin can have: one per owner and tile, and

@@ -3276,9 +3276,8 @@ int prepare_views(Graph &g, bool oriented, int32_t hub_degree, int fallback, int
     hipLaunchKernelGGL((k_sort_plus_block<16384, 1024>), dim3(cus), dim3(1024), 0, s, vi,
                        lst + hoff[3], lcnt + 3, padj, asym);
     TC_HIP(hipGetLastError());
-    // (a row of N+ has at most as many entries as its square root of nnz: none
-    // can be so long in a smaller graph)
-    if (nnz < int64_t(16384) * 16384) {
+    // (read back only where a row of N+ can be so long)
+    if (longest_list(g, true) <= 16384) {
         g.plan.huge.clear();
     } else if (!g.capturing) {
         int32_t nhuge = 0;
@@ -3615,7 +3614,7 @@ int count_once(Graph &g, uint32_t *out, uint64_t *global, const tc_schedule &sch
                            nullptr, nv, P, work, acc + 26, acc + 27, stats ? acc + 4 : nullptr);
     TC_HIP(hipGetLastError());
     const int64_t lists = oriented ? g.nplus : nnz;
-    const int64_t lmost = longest_list(oriented, nv, nnz, g.validated && !g.degree_stale ? g.max_degree : nv);
+    const int64_t lmost = longest_list(g, oriented);
     JobArrays J = {};
     plan_caps(P, nv, lists, lmost, J.cap);
     const int64_t total_cap = J.cap[0] + J.cap[1] + J.cap[2];
