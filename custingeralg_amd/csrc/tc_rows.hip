@@ -145,12 +145,14 @@ __global__ __launch_bounds__(kWavesPerBlock * kWave, 8) void k_count_rows(RowArg
 }
 
 // per_graph[g] = the sum of its vertices' counts (at most kRowMax^2 each); one
-// block per graph.
+// block per graph.  Vertices outside all boundaries are the first and the last
+// graph's, as everywhere.
 __global__ __launch_bounds__(256) void k_row_graph_sums(const int64_t *__restrict__ voff, int32_t nv,
                                                         const uint32_t *__restrict__ out,
                                                         unsigned long long *__restrict__ per_graph)
 {
-    const int64_t v0 = max(voff[blockIdx.x], (int64_t)0), v1 = min(voff[blockIdx.x + 1], (int64_t)nv);
+    const int64_t v0 = blockIdx.x == 0 ? 0 : max(voff[blockIdx.x], (int64_t)0);
+    const int64_t v1 = blockIdx.x + 1 == gridDim.x ? nv : min(voff[blockIdx.x + 1], (int64_t)nv);
     unsigned long long s = 0;
     for (int64_t v = v0 + threadIdx.x; v < v1; v += blockDim.x) s += out[v];
     const unsigned long long part[1] = {s};
@@ -171,6 +173,8 @@ bool rows_eligible(const Graph &g, const tc_schedule &sched)
     if (sched.policy != TC_POLICY_FIXED || sched.ratio_x16 > 0 || sched.mpath_min > 0 ||
         sched.hub_degree > 0 || sched.build != 0)
         return false;
+    // (a triangle of two graphs is counted whole in its job's graph)
+    if (g.batch_voff && g.batch_cross) return false;
     return g.validated && !g.degree_stale && g.max_degree <= kRowMax &&
            g.st.nnz <= (int64_t)kRowMean * g.st.nv;
 }

@@ -31,3 +31,23 @@ def test_hub_of_another_graph(k):
     assert np.array_equal(pv, ref)
     # (a triangle of two graphs is counted whole in either)
     assert int(pg.sum()) == int(ref.astype(np.uint64).sum())
+
+
+@pytest.mark.parametrize("hub", [0, 300])
+def test_boundaries_short_of_the_vertices(hub):
+    """Vertices before the first boundary and after the last belong to the first
+    and the last graph, whichever route counts (hub: rows above 128 entries)."""
+    rng = np.random.default_rng(hub)
+    n = 4000
+    part = np.array([0, 1500, 2500, n])
+    u = np.concatenate([rng.integers(a, b, 6 * (b - a)) for a, b in zip(part, part[1:])] +
+                       [np.full(hub, 1600)])
+    v = np.concatenate([rng.integers(a, b, 6 * (b - a)) for a, b in zip(part, part[1:])] +
+                       [rng.integers(1500, 2500, hub)])
+    off, adj = O.canon_csr(n, u.astype(np.int32), v.astype(np.int32))
+    ref = O.custinger_count(off, adj)
+    want = np.add.reduceat(ref.astype(np.uint64), part[:-1])
+    for voff in ([0, 1500, 2500, n], [40, 1500, 2500, n - 70], [0, 1500, 2500, n - 1]):
+        pg, pv, _ = T.batched_count(np.array(voff), off, adj, per_vertex=True)
+        assert np.array_equal(pv, ref)
+        assert np.array_equal(pg, want), voff
