@@ -289,25 +289,34 @@ __global__ __launch_bounds__(256) void k_dense_graph_sums(const DenseGraph *__re
 }
 
 // One block: matrix offsets of batched graphs; res[0] = the largest graph's
-// vertices, res[1] = words of all matrices.
+// vertices, res[1] = words of all matrices, res[2] = words of the rows of all
+// entries.
 __global__ __launch_bounds__(256) void k_dense_plan(const int64_t *__restrict__ voff, int32_t G,
+                                                    const int64_t *__restrict__ boff,
+                                                    const int32_t *__restrict__ len, int32_t nv,
                                                     DenseGraph *__restrict__ graphs,
                                                     unsigned long long *__restrict__ res)
 {
-    __shared__ long long part[256], pmax[256];
+    __shared__ long long part[256], pmax[256], pread[256];
     const int t = threadIdx.x;
     const int64_t per = (G + 255) / 256, g0 = min(t * per, (int64_t)G), g1 = min(g0 + per, (int64_t)G);
-    long long words = 0, most = 0;
+    long long words = 0, most = 0, read = 0;
     for (int64_t g = g0; g < g1; ++g) {
-        const int64_t n = voff[g + 1] - voff[g];
+        const int64_t a = voff[g], b = voff[g + 1], n = b - a;
         most = max(most, (long long)n);
-        if (n > 0 && n <= kDenseMax) words += n * dense_chunks((int32_t)n) * kChunkWords;
+        if (n > 0 && n <= kDenseMax) {
+            const int64_t row = (int64_t)dense_chunks((int32_t)n) * kChunkWords;
+            words += n * row;
+            if (a >= 0 && b <= nv) read += (boff[b - 1] + len[b - 1] - boff[a]) * row;
+        }
     }
+    pread[t] = read;
     part[t] = words;
     pmax[t] = most;
     __syncthreads();
-    long long before = 0, all = 0, mx = 0;
+    long long before = 0, all = 0, mx = 0, rd = 0;
     for (int k = 0; k < 256; ++k) {
+        rd += pread[k];
         if (k < t) before += part[k];
         all += part[k];
         mx = max(mx, pmax[k]);
@@ -324,6 +333,7 @@ __global__ __launch_bounds__(256) void k_dense_plan(const int64_t *__restrict__ 
     if (t == 0) {
         res[0] = (unsigned long long)mx;
         res[1] = (unsigned long long)all;
+        res[2] = (unsigned long long)rd;
     }
 }
 
@@ -353,16 +363,18 @@ int dense_plan_batched(Graph &g)
     TC_TRY(g.accum.ensure(32 * sizeof(unsigned long long)));
     DenseGraph *graphs = g.dgraphs.as<DenseGraph>();
     unsigned long long *res = g.accum.as<unsigned long long>();
-    hipLaunchKernelGGL(k_dense_plan, dim3(1), dim3(256), 0, s, g.batch_voff, G, graphs, res);
+    hipLaunchKernelGGL(k_dense_plan, dim3(1), dim3(256), 0, s, g.batch_voff, G, g.st.boff.as<int64_t>(),
+                       g.st.len.as<int32_t>(), g.st.nv, graphs, res);
     TC_HIP(hipGetLastError());
-    unsigned long long h[2];
+    unsigned long long h[3];
     TC_HIP(hipMemcpyAsync(h, res, sizeof(h), hipMemcpyDeviceToHost, s));
     TC_HIP(hipStreamSynchronize(s));
     TC_TRY(g.dgid.ensure((size_t)g.st.nv * sizeof(int32_t)));
     hipLaunchKernelGGL(k_dense_gid, dim3(grid_for(g.st.nv, 256, 4096)), dim3(256), 0, s, graphs, G,
                        g.st.nv, g.dgid.as<int32_t>());
     TC_HIP(hipGetLastError());
-    if (h[0] <= (unsigned long long)kDenseMax && h[1] * 4 <= (unsigned long long)kDenseBytes)
+    if (h[0] <= (unsigned long long)kDenseMax && h[1] * 4 <= (unsigned long long)kDenseBytes &&
+        dense_batch_pays((int64_t)h[1] * 4, (int64_t)h[2] * 4, g.st.nnz))
         g.dense_words = (int64_t)h[1];
     return TC_OK;
 }

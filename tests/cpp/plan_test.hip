@@ -86,3 +86,5 @@ extern "C" void dense_probe(int32_t d, int32_t check_sym, int32_t U, int32_t *lo
             for (int32_t q = 0; q < U; ++q) load(eb + (U + q) * 8);
     }
 }
+
+extern "C" int dense_batch_probe(int64_t mat, int64_t read, int64_t nnz) { return dense_batch_pays(mat, read, nnz); }

@@ -1,0 +1,41 @@
+"""Batches on both sides of the rules that choose their route, against the
+oracle."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import custingeralg_amd as T
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _batch(sizes, mean, hub, seed):
+    """Graphs of random pairs, each with a hub row of hub entries."""
+    rng = np.random.default_rng(seed)
+    voff = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int64)
+    u, v = [], []
+    for a, n in zip(voff, sizes):
+        m = int(n * mean / 2)
+        x, y = rng.integers(0, n, (2, m))
+        h = rng.permutation(n)[:min(hub, n)]
+        u += [x + a, np.full(len(h), n // 2) + a]
+        v += [y + a, h + a]
+    off, adj = O.canon_csr(int(voff[-1]), np.concatenate(u).astype(np.int32), np.concatenate(v).astype(np.int32))
+    return voff, off, adj
+
+
+def _check(voff, off, adj, **sched):
+    ref = O.custinger_count(off, adj)
+    pg, pv, st = T.batched_count(voff, off, adj, T.default_schedule(**sched), per_vertex=True)
+    assert np.array_equal(pv, ref)
+    assert np.array_equal(pg, np.add.reduceat(ref.astype(np.uint64), voff[:-1]))
+    return sum(st["tasks_bin"])
+
+
+@pytest.mark.parametrize("graphs,lists", [(1, False), (2, False), (40, True)])
+def test_wide_bit_rows(graphs, lists):
+    """Graphs of 16384 vertices: their bit rows are 2 KB each."""
+    b = _batch([16384] * graphs, 6, 400, graphs)
+    assert (_check(*b) > 0) == lists

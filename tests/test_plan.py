@@ -79,3 +79,21 @@ def test_bit_rows_load_their_own_entries(check_sym, unroll):
         lib.dense_probe(C.c_int32(d), C.c_int32(check_sym), C.c_int32(unroll), C.byref(lo), C.byref(hi))
         assert lo.value == 0 and hi.value < d, d
         assert d < 2 or hi.value == d - 1
+
+
+@pytest.mark.parametrize("graphs,n,nnz,pays", [
+    # batches that were measured on both routes, the bit rows' time over the lists'
+    (65, 1000, 425986, True),       # 0.3
+    (524, 1000, 18218546, True),    # 0.6
+    (128, 4000, 3588152, True),     # 0.6
+    (2, 16384, 1553072, True),      # 0.4
+    (31, 16384, 3719342, False),    # 2.3
+    (31, 16384, 24092252, False),   # 3.6
+    (128, 8000, 3830094, False),    # 1.9
+    (512, 4000, 48571398, False),   # 1.7
+])
+def test_batches_on_bit_rows(graphs, n, nnz, pays):
+    """Bytes of bit rows written and read, and the entries, decide together."""
+    row = (n + 1023) // 1024 * 128
+    lib = C.CDLL(_LIB)
+    assert bool(lib.dense_batch_probe(C.c_int64(graphs * n * row), C.c_int64(nnz * row), C.c_int64(nnz))) == pays
