@@ -35,6 +35,11 @@ constexpr int kCoreWaves = kCoreThreads / kWave;
 constexpr int kGroupRow = 16;                // rows of S(a) up to this long go four to a wave
 constexpr int kPartRows = 4096;              // batched: rows of a graph per block
 constexpr int64_t kCoreBytes = int64_t(16) << 30;  // all matrices of a batch
+// Entries of a batch per core vertex below which its cores cost more to build (256
+// bytes a vertex) than they save: 4000 R-MAT graphs of 2000 vertices took 4.6, 5.0,
+// 5.5 and 6.0 ms with 1.9, 3.6, 5.2 and 6.8 entries a vertex, without cores 2.9, 3.8,
+// 4.7 and 5.5; 500 of 4000 1.5 with 10.5, 1.6 without.
+constexpr int64_t kCoreEntries = 8;
 
 // The core of one graph: its ranks below the core are [nb, nb + n - k), its
 // core ranks core_lo + [kpre, kpre + k); its bit rows are the matrix's rows
@@ -527,7 +532,7 @@ int32_t core_size(const Graph &g, const tc_schedule &sched)
     if ((sched.policy != TC_POLICY_FIXED && sched.policy != TC_POLICY_LEARNED) || sched.ratio_x16 > 0 ||
         sched.mpath_min > 0 || sched.hub_degree > 0 || sched.build != 0)
         return 0;
-    if (g.batch_voff) return g.core_total;
+    if (g.batch_voff) return g.st.nnz >= kCoreEntries * g.core_total ? g.core_total : 0;
     const int32_t k = (g.st.nnz >= kCoreLargeNnz ? kCoreLarge : kCoreOne) * kCoreCols;
     return g.st.nv > 4 * k ? k : 0;
 }

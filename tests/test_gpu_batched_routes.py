@@ -39,3 +39,12 @@ def test_wide_bit_rows(graphs, lists):
     """Graphs of 16384 vertices: their bit rows are 2 KB each."""
     b = _batch([16384] * graphs, 6, 400, graphs)
     assert (_check(*b) > 0) == lists
+
+
+@pytest.mark.parametrize("mean,core", [(2, False), (12, True)])
+def test_cores_of_sparse_batches(mean, core):
+    """A batch with a graph above the bit rows' size: its cores take the place of
+    task lists only where there are entries enough."""
+    b = _batch([17000] + [1500] * 12, mean, 1200, 3)
+    fewer = _check(*b) < _check(*b, policy=T.POLICY_HASH)  # (a forced strategy has no cores)
+    assert fewer == core
