@@ -374,7 +374,7 @@ int dense_plan_batched(Graph &g)
                        g.st.nv, g.dgid.as<int32_t>());
     TC_HIP(hipGetLastError());
     if (h[0] <= (unsigned long long)kDenseMax && h[1] * 4 <= (unsigned long long)kDenseBytes &&
-        dense_batch_pays((int64_t)h[1] * 4, (int64_t)h[2] * 4, g.st.nnz))
+        dense_batch_pays((int64_t)h[1] * 4, (int64_t)h[2] * 4, g.st.nv, g.st.nnz))
         g.dense_words = (int64_t)h[1];
     return TC_OK;
 }

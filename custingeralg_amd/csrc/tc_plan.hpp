@@ -165,15 +165,16 @@ inline void plan_caps(const PlanParams &P, int32_t nv, int64_t lists, int64_t lm
 }
 
 // Whether a batch of graphs is counted on bit rows: mat bytes of them are written
-// and, a row per entry, read bytes read.  1.2 us per MiB written and 80 per GB read
-// against the task lists' 700 and 40 per million entries: fitted to 817 batches
-// (300 to 16384 vertices a graph, edge factors 2 to 32, 8 MB to 1 GB of bit rows),
-// of which it takes the slower route in none by more than 1.3 times.  By size alone
-// 31 R-MAT graphs of 16384 vertices and edge factor 32 took 8.0 ms on bit rows, 2.2
-// on lists; with edge factor 4 2.0 and 0.86 (two graphs: 0.17 and 0.53).
-inline bool dense_batch_pays(int64_t mat, int64_t read, int64_t nnz)
+// and, a row per entry, read bytes read.  1.4 us per MiB written, 60 per GB read and
+// 300 per million vertices against the task lists' 700 and 40 per million entries:
+// fitted to 845 batches (300 to 16384 vertices a graph, edge factors 1 to 32, up to
+// 1 GB of bit rows and 8M vertices); none of them takes 1.3 times the other route's
+// time.  By size alone 31 R-MAT graphs of 16384 vertices and edge factor 32 took 8.0
+// ms on bit rows, 2.2 on lists; with edge factor 4 2.0 and 0.86 (two graphs: 0.17
+// and 0.53); 8192 graphs of 1000 vertices and edge factor 2 5.5 and 4.0.
+inline bool dense_batch_pays(int64_t mat, int64_t read, int64_t nv, int64_t nnz)
 {
-    return 1.2 * (double)mat / 1048576 + 80e-9 * (double)read <= 700 + 40e-6 * (double)nnz;
+    return 1.4 * (double)mat / 1048576 + 60e-9 * (double)read + 300e-6 * (double)nv <= 700 + 40e-6 * (double)nnz;
 }
 
 // Bit rows (tc_dense.hip): whether a row of d entries is walked.  A row of one

@@ -87,4 +87,7 @@ extern "C" void dense_probe(int32_t d, int32_t check_sym, int32_t U, int32_t *lo
     }
 }
 
-extern "C" int dense_batch_probe(int64_t mat, int64_t read, int64_t nnz) { return dense_batch_pays(mat, read, nnz); }
+extern "C" int dense_batch_probe(int64_t mat, int64_t read, int64_t nv, int64_t nnz)
+{
+    return dense_batch_pays(mat, read, nv, nnz);
+}

@@ -91,9 +91,11 @@ def test_bit_rows_load_their_own_entries(check_sym, unroll):
     (31, 16384, 24092252, False),   # 3.6
     (128, 8000, 3830094, False),    # 1.9
     (512, 4000, 48571398, False),   # 1.7
+    (8192, 1000, 28818864, False),  # 1.4
 ])
 def test_batches_on_bit_rows(graphs, n, nnz, pays):
     """Bytes of bit rows written and read, and the entries, decide together."""
     row = (n + 1023) // 1024 * 128
     lib = C.CDLL(_LIB)
-    assert bool(lib.dense_batch_probe(C.c_int64(graphs * n * row), C.c_int64(nnz * row), C.c_int64(nnz))) == pays
+    assert bool(lib.dense_batch_probe(C.c_int64(graphs * n * row), C.c_int64(nnz * row), C.c_int64(graphs * n),
+                                      C.c_int64(nnz))) == pays
