@@ -164,6 +164,22 @@ inline void plan_caps(const PlanParams &P, int32_t nv, int64_t lists, int64_t lm
     }
 }
 
+// Whether a graph's rows are counted one by one (tc_rows.hip): none longer than
+// kRowMax, and a mean of kRowMean at most, above which the oriented count wins.  Nor
+// where hubs (a longest row of 16 times the mean, as for the core) have many rows to
+// be streamed past: the oriented count streams each pair's shorter list and starts
+// to win near a longest row times the vertices of 2^28.  8M vertices in R-MAT
+// communities of 1000 and edge factor 1 4.2 ms row by row, 2.7 oriented; 2M 1.05 and
+// 1.03, 1M 0.54 and 0.79; of 300 and edge factor 3 at 8M 4.9 and 4.2, at 3M 1.80 and
+// 1.87; 4M of 60 and edge factor 6 (no such hubs) 2.3 and 3.3.
+constexpr int32_t kRowMax = 128, kRowMean = 40;
+inline bool rows_pay(int32_t nv, int64_t nnz, int32_t longest)
+{
+    if (longest > kRowMax || nnz > (int64_t)kRowMean * nv) return false;
+    const double reach = (double)longest * nv;
+    return reach < 16.0 * (double)nnz || reach <= 268435456.0;
+}
+
 // Whether a batch of graphs is counted on bit rows: mat bytes of them are written
 // and, a row per entry, read bytes read.  1.4 us per MiB written, 60 per GB read and
 // 300 per million vertices against the task lists' 700 and 40 per million entries:

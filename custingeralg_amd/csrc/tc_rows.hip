@@ -6,7 +6,7 @@
 // the reference does (src/static_triangle_counting/cct.cu:233-268): the row in
 // a small LDS table, its neighbours' rows streamed past it, out[v] written
 // once.  One kernel, no atomics but the total's, and no sizes to read back.
-#include "tc_internal.hpp"
+#include "tc_plan.hpp"
 
 #include <algorithm>
 
@@ -14,9 +14,7 @@ namespace tc {
 
 namespace {
 
-constexpr int kRowMax = 128;    // longest row
 constexpr int kRowSlots = 512;  // of a wave's table: at most a quarter is used
-constexpr int kRowMean = 40;    // mean row above which the oriented count wins
 constexpr int kWavesPerBlock = 4;
 
 struct RowArgs {
@@ -175,8 +173,7 @@ bool rows_eligible(const Graph &g, const tc_schedule &sched)
         return false;
     // (a triangle of two graphs is counted whole in its job's graph)
     if (g.batch_voff && g.batch_cross) return false;
-    return g.validated && !g.degree_stale && g.max_degree <= kRowMax &&
-           g.st.nnz <= (int64_t)kRowMean * g.st.nv;
+    return g.validated && !g.degree_stale && rows_pay(g.st.nv, g.st.nnz, g.max_degree);
 }
 
 int rows_count(Graph &g, uint32_t *out, unsigned long long *acc, int32_t *bad, bool oriented, bool skip_lower,

@@ -91,3 +91,5 @@ extern "C" int dense_batch_probe(int64_t mat, int64_t read, int64_t nv, int64_t 
 {
     return dense_batch_pays(mat, read, nv, nnz);
 }
+
+extern "C" int rows_probe(int32_t nv, int64_t nnz, int32_t longest) { return rows_pay(nv, nnz, longest); }

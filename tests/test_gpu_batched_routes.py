@@ -48,3 +48,23 @@ def test_cores_of_sparse_batches(mean, core):
     b = _batch([17000] + [1500] * 12, mean, 1200, 3)
     fewer = _check(*b) < _check(*b, policy=T.POLICY_HASH)  # (a forced strategy has no cores)
     assert fewer == core
+
+
+@pytest.mark.parametrize("hub,lists", [(12, False), (110, True)])
+def test_short_rows_of_a_large_graph(hub, lists):
+    """3M vertices in a million triangles, and one longer row: row by row, or with
+    a hub oriented."""
+    n = 3000000
+    rng = np.random.default_rng(hub)
+    a, b, c = rng.integers(0, n, (3, n // 3))
+    h = rng.choice(n, hub, replace=False)
+    u = np.concatenate([a, b, c, np.full(hub, 77)])
+    v = np.concatenate([b, c, a, h])
+    off, adj = O.canon_csr(n, u.astype(np.int32), v.astype(np.int32))
+    assert np.diff(off).max() <= 128
+    ref = O.custinger_count(off, adj)
+    g = T.cuStinger(off, adj)
+    pv, glob, st = T.static_count(g)
+    g.close()
+    assert np.array_equal(pv, ref) and glob == int(ref.astype(np.uint64).sum())
+    assert (sum(st["tasks_bin"]) > 0) == lists

@@ -99,3 +99,20 @@ def test_batches_on_bit_rows(graphs, n, nnz, pays):
     lib = C.CDLL(_LIB)
     assert bool(lib.dense_batch_probe(C.c_int64(graphs * n * row), C.c_int64(nnz * row), C.c_int64(graphs * n),
                                       C.c_int64(nnz))) == pays
+
+
+@pytest.mark.parametrize("nv,nnz,longest,pays", [
+    # graphs that were measured on both routes, row by row over oriented
+    (65536, 1048000, 40, True),       # 0.1
+    (1000000, 1850000, 113, True),    # 0.7
+    (3000000, 11900000, 93, False),   # 0.96
+    (2000000, 7900000, 94, True),     # 0.9
+    (8000000, 14800000, 118, False),  # 1.6
+    (8000000, 31600000, 101, False),  # 1.2
+    (4000000, 26500000, 48, True),    # 0.7
+    (65536, 1048000, 129, False),
+    (65536, 2700000, 60, False),
+])
+def test_rows_one_by_one(nv, nnz, longest, pays):
+    lib = C.CDLL(_LIB)
+    assert bool(lib.rows_probe(C.c_int32(nv), C.c_int64(nnz), C.c_int32(longest))) == pays
