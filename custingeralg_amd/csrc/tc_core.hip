@@ -51,13 +51,6 @@ struct CoreBlock {
     int32_t graph, part, parts, pad;
 };
 
-__device__ inline void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Sum over the 8 lanes of a group (DPP: within quads, then half rows).
 __device__ inline uint32_t group_sum(uint32_t x)
 {
@@ -93,15 +86,15 @@ __global__ __launch_bounds__(256) void k_core_rows(const VInfo *__restrict__ vi,
         const int32_t dp = x.len - x.dm;
         const int32_t *row = padj + x.rb;
         for (int i = lane; i < words; i += kWave) bits[i] = 0u;
-        wave_lds_sync();
+        wave_sync();
         for (int32_t i = lane; i < dp; i += kWave) {
             const uint32_t c = (uint32_t)(row[i] - clo);
             if (c < (uint32_t)D.k) atomicOr(&bits[c >> 5], 1u << (c & 31));
         }
-        wave_lds_sync();
+        wave_sync();
         uint4 *dst = reinterpret_cast<uint4 *>(mat + (int64_t)b * words);
         for (int i = lane; i < words / 4; i += kWave) dst[i] = reinterpret_cast<const uint4 *>(bits)[i];
-        wave_lds_sync();
+        wave_sync();
     }
 }
 
@@ -325,13 +318,13 @@ __device__ inline unsigned long long core_rows(CoreShared<Q> &S, const CoreArgs 
                                 (uint32_t)__shfl((int32_t)lb, src, kWave);
             uint32_t *bits = S.bits[wid][lane / 16];
             for (int w = i16; w < kWords / 4; w += 16) reinterpret_cast<uint4 *>(bits)[w] = make_uint4(0, 0, 0, 0);
-            wave_lds_sync();
+            wave_sync();
             const int32_t *lst = A.padj + (gn > 0 ? glb : 0);
             if (i16 < gn) {
                 const uint32_t c = (uint32_t)(lst[i16] - clo);
                 atomicOr(&bits[c >> 5], 1u << (c & 31));
             }
-            wave_lds_sync();
+            wave_sync();
             int32_t most = gn;  // over the rows
             most = max(most, __shfl_xor(most, 16, kWave));
             most = max(most, __shfl_xor(most, 32, kWave));
@@ -341,7 +334,7 @@ __device__ inline unsigned long long core_rows(CoreShared<Q> &S, const CoreArgs 
                 atomicAdd(&A.outr[sr], h);
                 total += h;
             }
-            wave_lds_sync();
+            wave_sync();
         }
         // longer rows, one at a time
         for (uint64_t m = __ballot(n > kGroupRow); m; m &= m - 1) {
@@ -352,12 +345,12 @@ __device__ inline unsigned long long core_rows(CoreShared<Q> &S, const CoreArgs 
             const int32_t *lst = A.padj + rlb;
             uint32_t *bits = S.bits[wid][0];
             for (int w = lane; w < kWords; w += kWave) bits[w] = 0u;
-            wave_lds_sync();
+            wave_sync();
             for (int32_t e = lane; e < rn; e += kWave) {
                 const uint32_t c = (uint32_t)(lst[e] - clo);
                 atomicOr(&bits[c >> 5], 1u << (c & 31));
             }
-            wave_lds_sync();
+            wave_sync();
             uint32_t h = core_run<Q>(S, mat, clo, lst, rn, grp, kGroups,
                                      (rn + 2 * kGroups - 1) / (2 * kGroups), bits);
             h += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)h, 0x140, 0xF, 0xF, true);  // row_mirror
@@ -369,7 +362,7 @@ __device__ inline unsigned long long core_rows(CoreShared<Q> &S, const CoreArgs 
                 atomicAdd(&A.outr[r], sum);
                 total += sum;
             }
-            wave_lds_sync();
+            wave_sync();
         }
     }
     return total;
@@ -377,8 +370,9 @@ __device__ inline unsigned long long core_rows(CoreShared<Q> &S, const CoreArgs 
 
 // Lane 0 of a group adds h to b's counter in LDS, lane 1 counts the entry (the
 // symmetry check: b must be met |N-(b)| times); both are flushed once per
-// block.  Bound by L2 reads of bit rows (2 MB for 4096 columns: an XCD's L2
-// holds all of it; 18.7 TB/s at R-MAT 24).
+// block.  Bound by L2 reads of bit rows: the 2 MB of 4096 columns fit each XCD's L2
+// (R-MAT 24 with 4096: 18.7 TB/s), the 8 MB of 8192 do not, and a third of the 191
+// GB that R-MAT 24 reads comes from beyond (17.8 TB/s, 10.7 ms).
 template <int Q>
 __global__ __launch_bounds__(kCoreThreads, Q <= 2 ? 7 : Q <= 4 ? 6 : 2) void k_core_count(CoreArgs A)
 {

@@ -67,14 +67,6 @@ __device__ inline DenseGraph graph_of_row(const DenseArgs &A, int32_t v)
     return A.graphs ? A.graphs[A.gid[v]] : A.one;
 }
 
-// LDS written by other lanes of this wave is visible after it.
-__device__ inline void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // The rows of a wave: round-robin over a single graph (a hub's neighbours in id
 // order are often hubs); of batched graphs every XCD (blocks go to them in
 // turn) deals one run of rows, so that its L2 meets few graphs.
@@ -116,7 +108,7 @@ __global__ __launch_bounds__(kRowWaves * kWave) void k_dense_rows(DenseArgs A)
         const int32_t words = D.nch * kChunkWords, d = A.len[v];
         const int32_t *row = A.pool + A.boff[v];
         for (int i = lane; i < words; i += kWave) bits[i] = 0u;
-        wave_lds_sync();
+        wave_sync();
         for (int32_t k0 = lane; k0 < d; k0 += 4 * kWave) {
             int32_t c[4];
 #pragma unroll
@@ -136,11 +128,11 @@ __global__ __launch_bounds__(kRowWaves * kWave) void k_dense_rows(DenseArgs A)
             for (int64_t q = lane; q * A.long_len < d; q += kWave)
                 A.items[part * A.icap + base + q] = make_int2(v, (int32_t)(q * A.long_len));
         }
-        wave_lds_sync();
+        wave_sync();
         uint4 *dst = reinterpret_cast<uint4 *>(A.mat + D.off + (int64_t)(v - D.v0) * words);
         for (int i = lane; i < words / 4; i += kWave)
             dst[i] = reinterpret_cast<const uint4 *>(bits)[i];
-        wave_lds_sync();
+        wave_sync();
     }
 }
 

@@ -307,6 +307,7 @@ void graph_destroy(Graph *g);
 tc_schedule default_schedule();
 
 // ------------------------------------------------------- reductions --
+// LDS written by other lanes of this wave is visible after it.
 __device__ inline void wave_sync()
 {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

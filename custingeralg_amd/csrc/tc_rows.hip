@@ -29,13 +29,6 @@ struct RowArgs {
     int32_t check_sym;
 };
 
-__device__ inline void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 __device__ inline uint32_t row_slot(int32_t w) { return ((uint32_t)w * 0x9E3779B1u) >> 23; }  // of 512
 
 // G lanes stream one neighbour's row, 64 / G rows at a time, two rounds of
@@ -50,7 +43,7 @@ __global__ __launch_bounds__(kWavesPerBlock * kWave, 8) void k_count_rows(RowArg
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     int32_t *T = table[wid];
     for (int q = lane; q < kRowSlots; q += kWave) T[q] = -1;
-    wave_lds_sync();
+    wave_sync();
     unsigned long long total = 0;
     bool miss = false;
     const int64_t nwaves = (int64_t)gridDim.x * kWavesPerBlock;
@@ -71,7 +64,7 @@ __global__ __launch_bounds__(kWavesPerBlock * kWave, 8) void k_count_rows(RowArg
             if (mine[h] >= 0)
                 for (at[h] = row_slot(mine[h]); atomicCAS(&T[at[h]], -1, mine[h]) != -1;)
                     at[h] = (at[h] + 1) & (kRowSlots - 1);
-        wave_lds_sync();
+        wave_sync();
         uint32_t hits = 0;
         for (int h = 0; h * kWave < d; ++h) {
             // this lane's neighbour: its row, empty where there is nothing to do
@@ -126,11 +119,11 @@ __global__ __launch_bounds__(kWavesPerBlock * kWave, 8) void k_count_rows(RowArg
                     }
             }
         }
-        wave_lds_sync();
+        wave_sync();
 #pragma unroll
         for (int h = 0; h < 2; ++h)
             if (mine[h] >= 0) T[at[h]] = -1;
-        wave_lds_sync();
+        wave_sync();
         hits = wave_sum<uint32_t>(hits);
         if (lane == 0) {
             A.out[v] = hits;
