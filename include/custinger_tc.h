@@ -430,7 +430,9 @@ int tc_strategy_table_set(const uint8_t *table_host, int32_t dim);
 
 /* -------------------------------------------------------- autotuning -- */
 /* Sweeps bin thresholds and job grain on g and stores the best schedule as
- * the process default (the reference's exhaustive sweep, tests/cct.cpp:177-209). */
+ * the process default (the reference's exhaustive sweep, tests/cct.cpp:177-209).
+ * A graph that is counted on bit rows or row by row has no jobs to tune: the
+ * built-in schedule is the best then. */
 int tc_autotune(tc_graph *g, tc_schedule *best, double *best_ms);
 /* Makes s the process default schedule (what tc_schedule_default returns and
  * what a NULL schedule means), e.g. one saved from an earlier tc_autotune;

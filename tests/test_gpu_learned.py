@@ -160,3 +160,17 @@ def test_strategy_table_set_drives_the_policy():
     finally:
         Lm.unload()
         g.close()
+
+
+@pytest.mark.parametrize("scale,planned", [(10, False), (14, False), (15, True)])
+def test_autotune_where_nothing_is_planned(scale, planned):
+    """Graphs on bit rows run the same kernels under every schedule of the sweep:
+    the defaults stay; above, the sweep's grains are others than theirs."""
+    off, adj = O.rmat_graph(scale, 16, 3)
+    g = T.cuStinger(off, adj)
+    s, ms = Lm.autotune(g)
+    g.close()
+    Lm.set_default_schedule(None)
+    d = T.default_schedule()
+    same = (s.small_max, s.mid_max, s.job_items, s.flush_items) == (d.small_max, d.mid_max, d.job_items, d.flush_items)
+    assert ms > 0 and same == (not planned)
