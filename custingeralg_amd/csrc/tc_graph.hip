@@ -62,10 +62,11 @@ BlockPool &block_pool()
 }
 
 // Sizes requests share: powers of two up to 1 MB, then eighths of one; blocks
-// that the pool would not keep stay exact.
+// that the pool would not keep stay exact, to whole 256 bytes (kernels read the
+// 16 bytes that a row's last entries lie in).
 size_t block_size(size_t need)
 {
-    if (need > kHoldBlock) return need;
+    if (need > kHoldBlock) return (need + 255) / 256 * 256;
     size_t p2 = 4096;
     while (p2 < need) p2 <<= 1;
     if (p2 <= (size_t(1) << 20)) return p2;
