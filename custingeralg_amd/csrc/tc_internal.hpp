@@ -165,7 +165,7 @@ struct Graph {
     int32_t grow_add = 0;
     // bit-matrix counts (tc_dense.hip): matrix, items of long rows; batched
     // graphs: their matrices' places, the graph of every vertex and the words
-    // of all matrices (0: some graph is too large)
+    // of all matrices (0: the batch is not counted so)
     DevBuf dmat, ditems, dgraphs, dgid;
     // oriented count: the core's bit rows (tc_core.hip) and its size in the
     // current layout (0: none)
